@@ -15,6 +15,8 @@ SIGNATURES = {
     "hk_gemm_tile_choice": (c_int, [c_int] * 5),
     "hk_fp8_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_void_p]),
     "hk_fp8_gemm_variant": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_int, c_void_p]),
+    "hk_fp8_quantize_tensor_workspace_bytes": (c_size_t, []),
+    "hk_fp8_quantize_tensor": (c_int, [c_void_p, c_int, c_size_t, c_void_p, c_void_p, c_void_p, c_size_t, c_void_p]),
     "hk_mxfp4_gemm": (c_int, [c_void_p] * 5 + [c_int] * 3 + [c_void_p]),
     "hk_mxfp4_gemm_variant": (c_int, [c_void_p] * 5 + [c_int] * 4 + [c_void_p]),
     "hk_mxfp4_gemm_workspace_bytes": (c_size_t, [c_int, c_int, c_int]),

@@ -112,6 +112,17 @@ int hk_fp8_gemm_variant(const void* A_e4m3, const void* B_e4m3, void* C_bf16,
                         int M, int N, int K, float scale_a, float scale_b,
                         int variant, void* stream);
 
+/* Per-tensor quantization for hk_fp8_gemm: *host_scale = amax / 448 (1 for an all-zero tensor or one that holds a
+ * NaN), q = e4m3(x / scale), round to nearest even, saturating at +-448. x: n elements of bf16 (x_type 0), fp32
+ * (1) or fp16 (2). host_scale: host memory that the GPU can write (hipHostMalloc). UNLIKE the other entry
+ * points this one waits, for the scale and not for the quantization: on return *host_scale holds it, q is
+ * complete in stream order. workspace: hk_fp8_quantize_tensor_workspace_bytes() bytes of device memory.
+ * HK_ERR_UNSUPPORTED on a stream that is being captured. Stands for the host-side conversion of
+ * kernels/gemm/fp8fp32/profile_utils.cpp:35-45. */
+size_t hk_fp8_quantize_tensor_workspace_bytes(void);
+int hk_fp8_quantize_tensor(const void* x, int x_type, size_t n, void* q_e4m3, float* host_scale,
+                           void* workspace, size_t workspace_bytes, void* stream);
+
 /*
  * MXFP4 GEMM (OCP Microscaling v1.0): C[M,N] = bf16( sum_k a[m,k] * b[n,k] ) with
  *   a[m,k] = e2m1(A[m, k/2] nibble k%2; low nibble = even k) * 2^(A_scales[m, k/32] - 127)
