@@ -78,6 +78,55 @@ __device__ __forceinline__ float glu_act(int act, float g, float u, float alpha,
     return (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + __expf(-alpha * g)));
 }
 
+// MX codes of one row's block of 32 h columns held by the four lanes (r, g = 0..3) of the row: lane (r, g) has columns
+// 16 o + 4 g .. +4 (o = 0, 1) in h[o]. Returns the row's packed bytes (MXFP4: all 16 in lane g = 0; MXFP8: 16 each in
+// lanes g = 0, 1) and the block's exponent; `ok` false (uniform; columns past N): zeros with a scale of one.
+template <bool A8>
+__device__ __forceinline__ v4i mx_block_codes(const float (&h)[2][4], bool ok, int& e) {
+    float amax = 0.f;
+#pragma unroll
+    for (int o = 0; o < 2; ++o)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) amax = fmaxf(amax, fabsf(h[o][j]));
+    // maximum over the four lanes of the row: rows of 16 lanes swapped in registers
+    const uint32_t a = __float_as_uint(amax);
+    const auto s16 = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+    const uint32_t m1 = __float_as_uint(fmaxf(__uint_as_float(s16[0]), __uint_as_float(s16[1])));
+    const auto s32 = __builtin_amdgcn_permlane32_swap(m1, m1, false, false);
+    amax = fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
+    e = A8 ? mx8_block_exponent(amax) : mx_block_exponent(amax);
+    v4i o4;
+    if (A8) {
+        const float hv[8] = {h[0][0], h[0][1], h[0][2], h[0][3], h[1][0], h[1][1], h[1][2], h[1][3]};
+        v2i pk = pack8_e4m3(hv, e);  // .x: columns 4 g .. +4 of the block's first 16, .y: of its second 16
+        if (!ok) { pk = v2i{0, 0}; e = 0; }
+        // rows of 16 lanes swapped between the two registers: lane (r, 0) ends up with the
+        // first 16 columns' codes of all four lanes, lane (r, 1) with the second 16's
+        const auto q16 = __builtin_amdgcn_permlane16_swap((uint32_t)pk.x, (uint32_t)pk.y, false, false);  // [a0 b0 a2 b2], [a1 b1 a3 b3]
+        const auto q02 = __builtin_amdgcn_permlane32_swap(q16[0], q16[0], false, false);  // [a0 b0 ..], [a2 b2 ..]
+        const auto q13 = __builtin_amdgcn_permlane32_swap(q16[1], q16[1], false, false);  // [a1 b1 ..], [a3 b3 ..]
+        o4 = v4i{(int)q02[0], (int)q13[0], (int)q02[1], (int)q13[1]};
+    } else {
+        const float scale = __uint_as_float(e > -127 ? (uint32_t)(e + 127) << 23 : 0x00400000u);
+        uint32_t pk = 0;  // low half: columns 4 g .. +4 of the block's first 16, high half: of its second 16
+        pk = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(pk, h[0][0], h[0][1], scale, 0);
+        pk = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(pk, h[0][2], h[0][3], scale, 1);
+        pk = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(pk, h[1][0], h[1][1], scale, 2);
+        pk = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(pk, h[1][2], h[1][3], scale, 3);
+        if (!ok) { pk = 0; e = 0; }
+        // every lane of a row gets the packed values of all four: p[g'] = pk of lane (r, g')
+        const auto q16 = __builtin_amdgcn_permlane16_swap(pk, pk, false, false);       // [p0 p0 p2 p2], [p1 p1 p3 p3]
+        const auto q02 = __builtin_amdgcn_permlane32_swap(q16[0], q16[0], false, false);  // p0, p2
+        const auto q13 = __builtin_amdgcn_permlane32_swap(q16[1], q16[1], false, false);  // p1, p3
+        // the row's 16 bytes: the first 16 columns' codes (low halves), then the second 16's
+        o4.x = (int)__builtin_amdgcn_perm(q13[0], q02[0], 0x05040100u);
+        o4.y = (int)__builtin_amdgcn_perm(q13[1], q02[1], 0x05040100u);
+        o4.z = (int)__builtin_amdgcn_perm(q13[0], q02[0], 0x07060302u);
+        o4.w = (int)__builtin_amdgcn_perm(q13[1], q02[1], 0x07060302u);
+    }
+    return o4;
+}
+
 // x [rows, cols] bf16 -> packed e2m1 [rows, cols/2] + e8m0 scales [rows, scale_pitch] (columns
 // >= cols/32 are filled with 127). One thread per 8 elements, 4 threads per MX block.
 template <bool A8>
@@ -1173,7 +1222,6 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
             // h = act(gate, up): lane (r, g) holds, for row 16 M + r, the h columns
             // 128 n_tile + 32 w + 16 o + 4 g .. +4 (o = 0, 1): the wave's 32 columns are one MX block
             float h[2][4];
-            float amax = 0.f;
 #pragma unroll
             for (int o = 0; o < 2; ++o) {
                 const v4f gt = acc[M][2 * o], up = acc[M][2 * o + 1];
@@ -1181,47 +1229,10 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
                 for (int j = 0; j < 4; ++j) {
                     if (EXT) h[o][j] = glu_act(p.act, gt[j] + bias_a[o][j], up[j] + bias_b[o][j], p.alpha, p.limit);
                     else h[o][j] = silu_mul(gt[j], up[j]);
-                    amax = fmaxf(amax, fabsf(h[o][j]));
                 }
             }
-            // maximum over the four lanes (r, 0..3) of a row: rows of 16 lanes swapped in registers
-            {
-                const uint32_t a = __float_as_uint(amax);
-                const auto s16 = __builtin_amdgcn_permlane16_swap(a, a, false, false);
-                const uint32_t m1 = __float_as_uint(fmaxf(__uint_as_float(s16[0]), __uint_as_float(s16[1])));
-                const auto s32 = __builtin_amdgcn_permlane32_swap(m1, m1, false, false);
-                amax = fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
-            }
-            int e = A8 ? mx8_block_exponent(amax) : mx_block_exponent(amax);
-            v4i o4;
-            if (A8) {
-                const float hv[8] = {h[0][0], h[0][1], h[0][2], h[0][3], h[1][0], h[1][1], h[1][2], h[1][3]};
-                v2i pk = pack8_e4m3(hv, e);  // .x: columns 4 g .. +4 of the block's first 16, .y: of its second 16
-                if (!st_ok[0]) { pk = v2i{0, 0}; e = 0; }  // columns past N (uniform): zeros with a scale of one
-                // rows of 16 lanes swapped between the two registers: lane (r, 0) ends up with the
-                // first 16 columns' codes of all four lanes, lane (r, 1) with the second 16's
-                const auto q16 = __builtin_amdgcn_permlane16_swap((uint32_t)pk.x, (uint32_t)pk.y, false, false);  // [a0 b0 a2 b2], [a1 b1 a3 b3]
-                const auto q02 = __builtin_amdgcn_permlane32_swap(q16[0], q16[0], false, false);  // [a0 b0 ..], [a2 b2 ..]
-                const auto q13 = __builtin_amdgcn_permlane32_swap(q16[1], q16[1], false, false);  // [a1 b1 ..], [a3 b3 ..]
-                o4 = v4i{(int)q02[0], (int)q13[0], (int)q02[1], (int)q13[1]};
-            } else {
-                const float scale = __uint_as_float(e > -127 ? (uint32_t)(e + 127) << 23 : 0x00400000u);
-                uint32_t pk = 0;  // low half: columns 4 g .. +4 of the block's first 16, high half: of its second 16
-                pk = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(pk, h[0][0], h[0][1], scale, 0);
-                pk = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(pk, h[0][2], h[0][3], scale, 1);
-                pk = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(pk, h[1][0], h[1][1], scale, 2);
-                pk = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(pk, h[1][2], h[1][3], scale, 3);
-                if (!st_ok[0]) { pk = 0; e = 0; }  // columns past N (uniform): zeros with a scale of one
-                // every lane of a row gets the packed values of all four: p[g'] = pk of lane (r, g')
-                const auto q16 = __builtin_amdgcn_permlane16_swap(pk, pk, false, false);       // [p0 p0 p2 p2], [p1 p1 p3 p3]
-                const auto q02 = __builtin_amdgcn_permlane32_swap(q16[0], q16[0], false, false);  // p0, p2
-                const auto q13 = __builtin_amdgcn_permlane32_swap(q16[1], q16[1], false, false);  // p1, p3
-                // the row's 16 bytes: the first 16 columns' codes (low halves), then the second 16's
-                o4.x = (int)__builtin_amdgcn_perm(q13[0], q02[0], 0x05040100u);
-                o4.y = (int)__builtin_amdgcn_perm(q13[1], q02[1], 0x05040100u);
-                o4.z = (int)__builtin_amdgcn_perm(q13[0], q02[0], 0x07060302u);
-                o4.w = (int)__builtin_amdgcn_perm(q13[1], q02[1], 0x07060302u);
-            }
+            int e;
+            const v4i o4 = mx_block_codes<A8>(h, st_ok[0], e);
             asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen\n\ts_nop 1"
                          :: "v"(o4), "v"(st_voff0), "s"(st_srd0) : "memory");
             asm volatile("buffer_store_byte %0, %1, %2, 0 offen"
@@ -1336,6 +1347,10 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
     wait_vmcnt<0>();  // nothing may still be writing LDS when the workgroup retires
 }
 
+}  // namespace hk
+#include "moe_mxfp4_few.h"
+namespace hk {
+
 // ------------------------------------------------------------------------------ un-permute
 // y[t, :] = bf16( add[t, :] + sum_j w[t, j] * o[slot_to_pos[t*k + j], :] ), fp32 accumulation in
 // choice order starting from add (bf16 [T, H], e.g. a shared expert's output) or from 0 when add
@@ -1446,6 +1461,19 @@ static int launch_moe_stream(MoeGemmParams p, int max_items, hipStream_t s, bool
               : launch_moe_stream_nt<MODE, EXT, A8, GATHER, false>(p, max_items, s);
 }
 
+// The few-rows kernel on items of `rows` rows (16, or 32 with MXFP4 activations): four one-wave workgroups per item that the list can hold (the
+// workgroups past its actual length leave at once).
+template <int MODE>
+static int launch_moe_few(const MoeGemmParams& p, int rows, bool a8, bool ext, long long max_items, hipStream_t s) {
+    auto kern = a8 ? (ext ? moe_mxfp4_few_kernel<MODE, true, true, 1> : moe_mxfp4_few_kernel<MODE, false, true, 1>)
+                : rows <= 16 ? (ext ? moe_mxfp4_few_kernel<MODE, true, false, 1> : moe_mxfp4_few_kernel<MODE, false, false, 1>)
+                             : (ext ? moe_mxfp4_few_kernel<MODE, true, false, 2> : moe_mxfp4_few_kernel<MODE, false, false, 2>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)(4 * max_items)), dim3(64), 0, s, p);
+    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
+}
+// Most work items of `rows` rows that S rows in at most E experts give.
+static long long moe_few_max_items(int S, int E, int rows, int n_tiles) { return ((long long)S / rows + min(E, S)) * n_tiles; }
+
 template <int MODE, bool EXT>
 static int launch_moe_gemm(MoeGemmParams p, int max_items, hipStream_t s) {
     auto kern = moe_mxfp4_gemm_kernel<MODE, EXT>;
@@ -1532,6 +1560,15 @@ extern "C" int hk_moe_mxfp4_preshuffle(const void* w, const void* scales, int sc
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
+// Rows per work item of the few-rows kernel (moe_mxfp4_few.h, pre-shuffled weights), or 0 where the streaming kernel
+// is the better one: by the mean number of rows per expert. Routers load their experts unevenly, and an expert with
+// more rows than an item streams its weights again: one fragment of 16 rows up to a mean of 4, two up to 8 (MXFP4
+// activations only: MXFP8 rows are twice the traffic), measured in the header's comment.
+static int moe_few_rows(int T, int k, int E, bool a8) {
+    const long long S = (long long)T * k;
+    return S <= 4ll * E ? 16 : S <= 8ll * E && !a8 ? 32 : 0;
+}
+
 // Workspace layout of hk_moe_mxfp4_forward (all regions 256-byte aligned).
 struct MoeWs {
     size_t ids, w, sorted, offsets, inv, sort_ws, items1, items2, nitems, xq, xs, hq, hs, o, total;
@@ -1544,7 +1581,8 @@ static MoeWs moe_ws_layout(int T, int H, int I, int E, int k, bool a8 = false) {
     const size_t S = (size_t)T * k;
     L.ids = take(S * 4); L.w = take(S * 4); L.sorted = take(S * 4); L.offsets = take((size_t)(E + 1) * 4);
     L.inv = take(S * 4); L.sort_ws = take(hk_moe_sort_workspace_bytes(T, k, E));
-    const int max_tiles = (int)(S / kMoeBM) + E;
+    const int few = moe_few_rows(T, k, E, a8);
+    const int max_tiles = (int)(S / (few ? few : kMoeBM)) + E;
     L.max_items1 = max_tiles * ((I + 127) / 128);
     L.max_items2 = max_tiles * ((H + 255) / 256);
     L.items1 = take((size_t)L.max_items1 * sizeof(MoeItem));
@@ -1589,9 +1627,9 @@ static int moe_mxfp4_check(int T, int H, int I, int E, int k, int w13_scale_pitc
     return HK_OK;
 }
 
-static MoeBuildItems moe_items_args(uint8_t* ws, const MoeWs& L, int I, int H, bool a8, int weight_layout, bool gather) {
+static MoeBuildItems moe_items_args(uint8_t* ws, const MoeWs& L, int I, int H, bool a8, int weight_layout, bool gather, int few) {
     MoeBuildItems b;
-    b.bm = a8 ? (gather ? S4Cfg<true, true>::kBM : S4Cfg<true, false>::kBM) : weight_layout ? kStBM : kMoeBM;
+    b.bm = few ? few : a8 ? (gather ? S4Cfg<true, true>::kBM : S4Cfg<true, false>::kBM) : weight_layout ? kStBM : kMoeBM;
     b.items[0] = (MoeItem*)(ws + L.items1); b.items[1] = (MoeItem*)(ws + L.items2);
     b.n_tiles[0] = (I + 127) / 128; b.n_tiles[1] = (H + 255) / 256;
     return b;
@@ -1667,13 +1705,14 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
     const int S = T * k;
 
     int32_t* nitems = (int32_t*)(ws + L.nitems);
-    const bool gather = moe_gathers(weight_layout, ext, a8, T, H);
+    const int few = weight_layout == 1 ? moe_few_rows(T, k, E, a8) : 0;
+    const bool gather = few || moe_gathers(weight_layout, ext, a8, T, H);
     // non-temporal weight loads while most experts' rows fit one work item (their weights are then read
     // once): mean + one standard deviation of the rows per expert under uniform routing
     const bool nt = moe_rows_fit_one_item(T, k, E, a8 ? (gather ? S4Cfg<true, true>::kBM : S4Cfg<true, false>::kBM) : kStBM);
     if (!x_quantized) {   // (the forward pass of a small layer has done this in its sort launch)
         const int nk1 = (H / 2 + 127) / 128;
-        const MoeBuildItems b = moe_items_args(ws, L, I, H, a8, weight_layout, gather);
+        const MoeBuildItems b = moe_items_args(ws, L, I, H, a8, weight_layout, gather, few);
         const MxQuantizeArgs qa = moe_quantize_args(x_bf16, sorted_slots, slot_to_pos, k, T, H, I, ws, L);
         auto qp = a8 ? (gather ? mx_quantize_permute_kernel<true, false> : mx_quantize_permute_kernel<true, true>)
                      : (gather ? mx_quantize_permute_kernel<false, false> : mx_quantize_permute_kernel<false, true>);
@@ -1696,7 +1735,9 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
     p.out0 = ws + L.hq; p.out_scales = ws + L.hs;
     p.K = H; p.N = I; p.n_tiles_n = (I + 127) / 128;
     p.bias = bias13; p.bias_bytes = (uint32_t)((size_t)E * 2 * I * 4); p.act = activation; p.alpha = alpha; p.limit = limit; p.interleaved = w13_interleaved != 0;
-    if (a8)
+    if (few)
+        st = launch_moe_few<0>(p, few, a8, ext, moe_few_max_items(S, E, few, p.n_tiles_n), s);
+    else if (a8)
         st = ext ? launch_moe_stream<0, true, true>(p, L.max_items1, s, nt)
                  : gather ? launch_moe_stream<0, false, true, true>(p, L.max_items1, s, nt)
                           : launch_moe_stream<0, false, true>(p, L.max_items1, s, nt);
@@ -1720,7 +1761,9 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
     q.out0 = ws + L.o; q.out_scales = nullptr;
     q.K = I; q.N = H; q.n_tiles_n = (H + 255) / 256;
     q.bias = bias2; q.bias_bytes = (uint32_t)((size_t)E * H * 4);
-    if (a8)
+    if (few)
+        st = launch_moe_few<1>(q, few, a8, bias2 != nullptr, moe_few_max_items(S, E, few, q.n_tiles_n), s);
+    else if (a8)
         st = bias2 ? launch_moe_stream<1, true, true>(q, L.max_items2, s, nt) : launch_moe_stream<1, false, true>(q, L.max_items2, s, nt);
     else if (bias2)
         st = weight_layout ? launch_moe_stream<1, true, false>(q, L.max_items2, s, nt) : launch_moe_gemm<1, true>(q, L.max_items2, s);
@@ -1787,12 +1830,13 @@ static int moe_mxfp4_forward_impl(const void* x_bf16, const float* router_logits
     if (st != HK_OK) return st;
     const bool ext = bias13 || bias2 || activation != 0 || w13_interleaved;
     bool fused = false;
-    if (moe_gathers(weight_layout, ext, a8, T, H) && (long long)T * k <= kSortSmallMax && x_bf16 &&
+    const int few = weight_layout == 1 ? moe_few_rows(T, k, E, a8) : 0;
+    if ((few || moe_gathers(weight_layout, ext, a8, T, H)) && (long long)T * k <= kSortSmallMax && x_bf16 &&
         (((uintptr_t)x_bf16 | (uintptr_t)workspace) & 15u) == 0) {
         // sort, item lists and the quantization of x in one launch (moe_sort_quantize_kernel)
         const int S = T * k, nchunks = (S + kSortChunk - 1) / kSortChunk;
         const int nk1 = (H / 2 + 127) / 128;
-        const MoeBuildItems b = moe_items_args(ws, L, I, H, a8, weight_layout, true);
+        const MoeBuildItems b = moe_items_args(ws, L, I, H, a8, weight_layout, true, few);
         const MxQuantizeArgs qa = moe_quantize_args(x_bf16, nullptr, nullptr, k, T, H, I, ws, L);
         const int grid = nchunks + 2 * kFusedItemParts + (T + kQpRows - 1) / kQpRows * ((nk1 + 7) / 8);
         auto kern = a8 ? moe_sort_quantize_kernel<true> : moe_sort_quantize_kernel<false>;
