@@ -909,6 +909,17 @@ __global__ __launch_bounds__(256) void moe_fp8blk_preshuffle_kernel(const uint8_
     *(v4i*)(out + ((size_t)e * per_expert + chunk) * 16) = v;
 }
 
+}  // namespace hk
+#include "moe_fp8blk_few.h"
+namespace hk {
+
+// The few-rows kernel for as many items as the list can hold (the workgroups past its actual length leave at once).
+template <int MODE>
+static int launch_fp8blk_few(const MoeFp8Params& p, long long max_items, hipStream_t s) {
+    hipLaunchKernelGGL(moe_fp8blk_few_kernel<MODE>, dim3((unsigned)(8 * max_items)), dim3(64), 0, s, p);
+    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
+}
+
 template <int MODE, bool GATHER>
 static int launch_fp8blk_gemm(const MoeFp8Params& p, int max_items, hipStream_t s) {
     auto kern = moe_fp8blk_gemm_kernel<MODE, GATHER>;
@@ -950,12 +961,26 @@ static int moe_fp8blk_item_rows(int T, int k, int E) {
     return n_short <= n_long ? kF8BMShort : kF8BM;
 }
 
+// Whether a layer on pre-shuffled weights takes the few-rows kernel (moe_fp8blk_few.h has the measurements): with a
+// mean of at most 2 rows per expert (H = 7168, I = 2048, E = 256, k = 8, us, streaming / few-rows kernel: 1 token
+// 112 / 93, 4 tokens 266 / 254, 16 tokens 754 / 713, 64 tokens 1567 / 1534, 128 tokens 1765 / 1771, 256 tokens
+// 1828 / 1927), or while the gate+up GEMM has less than 3/4 of an item of 16 rows per CU and an expert's weights are
+// not streamed more than twelve times (one expert, H = 7168, I = 2048: 16 rows 99 / 19, 100 rows 106 / 52, 200 rows
+// 89 / 89, 300 rows 104 / 138).
+static bool moe_fp8blk_few(int T, int H, int I, int E, int k) {
+    const long long S = (long long)T * k;
+    if (S * (H > I ? H : I) >= (1ll << 31)) return false;   // its row offsets keep bit 31 free
+    if (S <= 2ll * E) return true;
+    const long long m_tiles = S / kF8FewRows + min((long long)E, S);
+    return S <= 192ll * E && m_tiles * (I / 128) * 4 <= 3ll * moe_num_compute_units();
+}
+
 // n-tiles of 256 weight rows of the two GEMMs: gate+up (mode 0: 128 h columns = 128 gate + 128 up rows
 // per tile) and down (mode 1).
 static inline int fp8blk_n_tiles(int mode, int N) { return mode == 0 ? N / 128 : (int)(((long long)N + 255) / 256); }
 
 struct Fp8Ws {
-    size_t ids, w, sorted, offsets, inv, sort_ws, items1, items2, nitems, xq, xs, hq, hs, o, total;
+    size_t ids, w, sorted, offsets, inv, sort_ws, items1, items2, nitems, xq, xs, hq, hs, hf, o, total;
     int max_items1, max_items2;
 };
 static Fp8Ws fp8_ws_layout(int T, int H, int I, int E, int k) {
@@ -965,7 +990,8 @@ static Fp8Ws fp8_ws_layout(int T, int H, int I, int E, int k) {
     const size_t S = (size_t)T * k;
     L.ids = take(S * 4); L.w = take(S * 4); L.sorted = take(S * 4); L.offsets = take((size_t)(E + 1) * 4);
     L.inv = take(S * 4); L.sort_ws = take(hk_moe_sort_workspace_bytes(T, k, E));
-    const int max_tiles = (int)(S / kF8BMShort) + E;   // whichever item size the layer runs with
+    const bool few = moe_fp8blk_few(T, H, I, E, k);
+    const int max_tiles = (int)(S / (few ? kF8FewRows : kF8BMShort)) + E;   // whichever item size the layer runs with
     L.max_items1 = max_tiles * (I / 128);
     L.max_items2 = max_tiles * ((H + 255) / 256);
     L.items1 = take((size_t)L.max_items1 * sizeof(MoeItem));
@@ -975,6 +1001,7 @@ static Fp8Ws fp8_ws_layout(int T, int H, int I, int E, int k) {
     // gathers activation rows by token index: there is no permuted copy)
     L.xq = take((size_t)T * H); L.xs = take((size_t)T * (H / 128) * 4);
     L.hq = take(S * (size_t)I); L.hs = take(S * (size_t)(I / 128) * 4);
+    L.hf = take(few ? S * (size_t)I * 4 : 0);   // h before its quantization (few-rows kernel)
     L.o = take(S * (size_t)H * 2);
     L.total = off;
     return L;
@@ -1048,6 +1075,76 @@ extern "C" int hk_moe_fp8blk_preshuffle(const void* w, int E, int N, int K, int 
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
+namespace hk {
+// The routing of an expert that every token passes through.
+__global__ __launch_bounds__(256) void moe_identity_routing_kernel(int T, int32_t* __restrict__ sorted_slots,
+                                                                   int32_t* __restrict__ expert_offsets) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < T) sorted_slots[i] = i;
+    if (i < 2) expert_offsets[i] = i * T;
+}
+
+// The two grouped GEMMs of an already validated call. sorted_slots / expert_offsets null: one expert that takes every
+// token in order. out_o: rows of the down GEMM in sorted order.
+static int fp8blk_grouped_gemms(const void* x_e4m3, const float* x_scales, const void* w13, const float* w13_scales,
+                                const void* w2, const float* w2_scales, const int32_t* sorted_slots,
+                                const int32_t* expert_offsets, int T, int H, int I, int E, int k, int weight_layout,
+                                uint8_t* ws, void* out_o, hipStream_t s) {
+    const Fp8Ws L = fp8_ws_layout(T, H, I, E, k);
+    const int S = T * k;
+    const bool few = weight_layout == 1 && moe_fp8blk_few(T, H, I, E, k);
+    const bool identity = !sorted_slots, lists = !few || !identity;
+    int32_t* nitems = (int32_t*)(ws + L.nitems);
+    const int bm = few ? kF8FewRows : weight_layout == 1 ? moe_fp8blk_item_rows(T, k, E) : kF8BM;
+    if (identity && lists) {
+        hipLaunchKernelGGL(moe_identity_routing_kernel, dim3((T + 255) / 256), dim3(256), 0, s, T,
+                           (int32_t*)(ws + L.sorted), (int32_t*)(ws + L.offsets));
+        if (hipGetLastError() != hipSuccess) return HK_ERR_LAUNCH;
+        sorted_slots = (const int32_t*)(ws + L.sorted);
+        expert_offsets = (const int32_t*)(ws + L.offsets);
+    }
+    if (lists)
+        moe_launch_build_items(expert_offsets, E, bm, I / 128, (MoeItem*)(ws + L.items1), (H + 255) / 256,
+                               (MoeItem*)(ws + L.items2), nitems, s);
+    // non-temporal weight loads while most experts' rows fit one work item (their weights are then read once)
+    const bool nt = moe_rows_fit_one_item(T, k, E, bm);
+    // few-rows kernel: most m-tiles that S rows in at most E experts give
+    const long long few_m = lists ? S / kF8FewRows + min(E, S) : (S + kF8FewRows - 1) / kF8FewRows;
+
+    MoeFp8Params p{};
+    p.A = (const uint8_t*)x_e4m3; p.SA = x_scales; p.S = S;   // gathered by token index inside the kernel
+    p.sorted_slots = sorted_slots; p.topk = k; p.T = T;
+    p.B = (const uint8_t*)w13; p.SB = w13_scales;
+    p.b_expert_stride = (long long)2 * I * H; p.sb_expert_stride = (long long)(2 * I / 128) * (H / 128);
+    p.items = lists ? (const MoeItem*)(ws + L.items1) : nullptr; p.num_items = nitems;
+    p.out0 = ws + (few ? L.hf : L.hq); p.out_scales = (float*)(ws + L.hs);
+    p.K = H; p.N = I; p.n_tiles_n = I / 128;
+    int st;
+    if (weight_layout == 1) p.b_expert_stride = (long long)fp8blk_n_tiles(0, I) * (H / 128) * kF8sBTile;
+    if (few) st = launch_fp8blk_few<0>(p, few_m * p.n_tiles_n, s);
+    else if (weight_layout == 1) st = launch_fp8blk_stream<0, true>(p, L.max_items1, s, nt, bm);
+    else st = launch_fp8blk_gemm<0, true>(p, L.max_items1, s);
+    if (st != HK_OK) return st;
+    if (few) {
+        hipLaunchKernelGGL(moe_fp8blk_few_quantize_kernel, dim3((unsigned)(((long long)S * (I / 8) + 255) / 256)), dim3(256),
+                           0, s, (const float*)(ws + L.hf), S, I, ws + L.hq, (float*)(ws + L.hs));
+        if (hipGetLastError() != hipSuccess) return HK_ERR_LAUNCH;
+    }
+
+    MoeFp8Params q{};
+    q.A = ws + L.hq; q.SA = (const float*)(ws + L.hs); q.S = S;
+    q.B = (const uint8_t*)w2; q.SB = w2_scales;
+    q.b_expert_stride = (long long)H * I; q.sb_expert_stride = (long long)(H / 128) * (I / 128);
+    q.items = lists ? (const MoeItem*)(ws + L.items2) : nullptr; q.num_items = nitems + 1;
+    q.out0 = out_o; q.out_scales = nullptr;
+    q.K = I; q.N = H; q.n_tiles_n = (H + 255) / 256;
+    if (weight_layout == 1) q.b_expert_stride = (long long)fp8blk_n_tiles(1, H) * (I / 128) * kF8sBTile;
+    if (few) return launch_fp8blk_few<1>(q, few_m * q.n_tiles_n, s);
+    if (weight_layout == 1) return launch_fp8blk_stream<1, false>(q, L.max_items2, s, nt, bm);
+    return launch_fp8blk_gemm<1, false>(q, L.max_items2, s);
+}
+}  // namespace hk
+
 extern "C" int hk_moe_fp8blk_experts_ex2(const void* x_e4m3, const float* x_scales, const void* w13,
                                          const float* w13_scales, const void* w2, const float* w2_scales,
                                          const float* topk_w, const int32_t* sorted_slots,
@@ -1060,47 +1157,22 @@ extern "C" int hk_moe_fp8blk_experts_ex2(const void* x_e4m3, const float* x_scal
                              y_add_bf16_or_null, workspace, workspace_bytes);
     if (st != HK_OK) return st;
     const Fp8Ws L = fp8_ws_layout(T, H, I, E, k);
-    hipStream_t s = (hipStream_t)stream;
     uint8_t* ws = (uint8_t*)workspace;
-    const int S = T * k;
-    int32_t* nitems = (int32_t*)(ws + L.nitems);
-    const int bm = weight_layout == 1 ? moe_fp8blk_item_rows(T, k, E) : kF8BM;
-    moe_launch_build_items(expert_offsets, E, bm, I / 128, (MoeItem*)(ws + L.items1), (H + 255) / 256,
-                           (MoeItem*)(ws + L.items2), nitems, s);
-    // non-temporal weight loads while most experts' rows fit one work item (their weights are then read once)
-    const bool nt = moe_rows_fit_one_item(T, k, E, bm);
-
-    MoeFp8Params p{};
-    p.A = (const uint8_t*)x_e4m3; p.SA = x_scales; p.S = S;   // gathered by token index inside the kernel
-    p.sorted_slots = sorted_slots; p.topk = k; p.T = T;
-    p.B = (const uint8_t*)w13; p.SB = w13_scales;
-    p.b_expert_stride = (long long)2 * I * H; p.sb_expert_stride = (long long)(2 * I / 128) * (H / 128);
-    p.items = (const MoeItem*)(ws + L.items1); p.num_items = nitems;
-    p.out0 = ws + L.hq; p.out_scales = (float*)(ws + L.hs);
-    p.K = H; p.N = I; p.n_tiles_n = I / 128;
-    if (weight_layout == 1) {
-        p.b_expert_stride = (long long)fp8blk_n_tiles(0, I) * (H / 128) * kF8sBTile;
-        st = launch_fp8blk_stream<0, true>(p, L.max_items1, s, nt, bm);
-    } else {
-        st = launch_fp8blk_gemm<0, true>(p, L.max_items1, s);
-    }
-    if (st != HK_OK) return st;
-
-    MoeFp8Params q{};
-    q.A = ws + L.hq; q.SA = (const float*)(ws + L.hs); q.S = S;
-    q.B = (const uint8_t*)w2; q.SB = w2_scales;
-    q.b_expert_stride = (long long)H * I; q.sb_expert_stride = (long long)(H / 128) * (I / 128);
-    q.items = (const MoeItem*)(ws + L.items2); q.num_items = nitems + 1;
-    q.out0 = ws + L.o; q.out_scales = nullptr;
-    q.K = I; q.N = H; q.n_tiles_n = (H + 255) / 256;
-    if (weight_layout == 1) {
-        q.b_expert_stride = (long long)fp8blk_n_tiles(1, H) * (I / 128) * kF8sBTile;
-        st = launch_fp8blk_stream<1, false>(q, L.max_items2, s, nt, bm);
-    } else {
-        st = launch_fp8blk_gemm<1, false>(q, L.max_items2, s);
-    }
+    st = fp8blk_grouped_gemms(x_e4m3, x_scales, w13, w13_scales, w2, w2_scales, sorted_slots, expert_offsets, T, H, I, E,
+                              k, weight_layout, ws, ws + L.o, (hipStream_t)stream);
     if (st != HK_OK) return st;
     return hk_moe_unpermute_add(ws + L.o, topk_w, slot_to_pos, T, k, H, y_add_bf16_or_null, y_bf16, stream);
+}
+
+extern "C" int hk_moe_fp8blk_shared_expert(const void* x_e4m3, const float* x_scales, const void* w13,
+                                           const float* w13_scales, const void* w2, const float* w2_scales,
+                                           void* y_bf16, int T, int H, int I, int weight_layout, void* workspace,
+                                           size_t workspace_bytes, void* stream) {
+    const int st = fp8blk_validate(x_e4m3, x_scales, w13, w13_scales, w2, w2_scales, y_bf16, T, H, I, 1, 1,
+                                   weight_layout, nullptr, workspace, workspace_bytes);
+    if (st != HK_OK) return st;
+    return fp8blk_grouped_gemms(x_e4m3, x_scales, w13, w13_scales, w2, w2_scales, nullptr, nullptr, T, H, I, 1, 1,
+                                weight_layout, (uint8_t*)workspace, y_bf16, (hipStream_t)stream);
 }
 
 extern "C" int hk_moe_fp8blk_experts_ex(const void* x_e4m3, const float* x_scales, const void* w13,

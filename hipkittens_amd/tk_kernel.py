@@ -597,15 +597,18 @@ def dispatch_moe_fp8blk_experts(x, x_scales, w13, w13_scales, w2, w2_scales, wei
 
 def dispatch_moe_fp8blk_shared_expert(x, x_scales, w13, w13_scales, w2, w2_scales, y, workspace) -> None:
     """The dense MLP every token passes through (DeepSeek-V3 shared expert): w13 [1, 2I, H],
-    w2 [1, H, I] in the routed experts' format, run as a one-expert layer with identity routing.
+    w2 [1, H, I] in the routed experts' format, run as a one-expert layer (include/hk355.h:
+    hk_moe_fp8blk_shared_expert).
     workspace: moe_fp8blk_workspace_bytes(T, H, I, 1, 1) bytes. Its output is what the routed layer
     takes as y_add."""
-    T = x.shape[0]
-    ones = torch.ones((T, 1), dtype=torch.float32, device=x.device)
-    ident = torch.arange(T, dtype=torch.int32, device=x.device)
-    offsets = torch.tensor([0, T], dtype=torch.int32, device=x.device)
-    dispatch_moe_fp8blk_experts(x, x_scales, w13, w13_scales, w2, w2_scales, ones, ident, offsets, ident, y,
-                                workspace)
+    T, H, I, E, layout, w13, w13_scales, w2, w2_scales = _check_fp8blk(x, x_scales, w13, w13_scales, w2, w2_scales, y)
+    if E != 1:
+        raise RuntimeError("a shared expert's weights are one expert's")
+    _check_tensor(workspace, "workspace", (torch.uint8,), 1)
+    st = _lib.load_library().hk_moe_fp8blk_shared_expert(
+        x.data_ptr(), x_scales.data_ptr(), w13.data_ptr(), w13_scales.data_ptr(), w2.data_ptr(),
+        w2_scales.data_ptr(), y.data_ptr(), T, H, I, layout, workspace.data_ptr(), workspace.numel(), _stream(x))
+    _lib.check(st, "dispatch_moe_fp8blk_shared_expert")
 
 
 def dispatch_moe_fp8blk(x, x_scales, router_logits, router_bias, w13, w13_scales, w2, w2_scales, y, topk: int,

@@ -415,6 +415,11 @@ int hk_moe_fp8blk_experts_ex2(const void* x_e4m3, const float* x_scales, const v
                               int T, int H, int I, int E, int k, int weight_layout,
                               const void* y_add_bf16_or_null, void* workspace, size_t workspace_bytes,
                               void* stream);
+/* The expert that every token passes through (w13 [1, 2I, H], w2 [1, H, I], weight_layout as above): y = its MLP of
+ * every row of x, with nothing to route. workspace: hk_moe_fp8blk_workspace_bytes(T, H, I, 1, 1). */
+int hk_moe_fp8blk_shared_expert(const void* x_e4m3, const float* x_scales, const void* w13, const float* w13_scales,
+                                const void* w2, const float* w2_scales, void* y_bf16, int T, int H, int I,
+                                int weight_layout, void* workspace, size_t workspace_bytes, void* stream);
 int hk_moe_fp8blk_forward_ex2(const void* x_e4m3, const float* x_scales, const float* router_logits,
                               const float* router_bias_or_null, int n_group, int topk_group,
                               float routed_scale, const void* w13, const float* w13_scales,
