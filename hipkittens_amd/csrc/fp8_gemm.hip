@@ -70,8 +70,10 @@ __global__ __launch_bounds__(kPcThreads) void fp8_gemm_prodcons_kernel(
     gemm_prodcons_body<Fp8Mma, EDGE>(smem, A, B, C, M, N, K, alpha, tiles_m, tiles_n);
 }
 
+// (two waves per SIMD as the register budget: with all 512 registers the compiler moves the accumulators between the
+// two register files on every other K-step)
 template <int TILE, int STAGES, bool EDGE, bool SPLIT>
-__global__ __launch_bounds__(256) void fp8_gemm_small_tile_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void fp8_gemm_small_tile_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, uint16_t* __restrict__ C,
     int M, int N, int K, float alpha, int tiles_m, int tiles_n, int kps, float* __restrict__ partial) {
     extern __shared__ __attribute__((aligned(2048))) uint8_t smem[];

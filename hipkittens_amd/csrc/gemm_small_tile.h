@@ -8,15 +8,13 @@
 namespace hk {
 
 // 128x128-tile kernel body for problems with too few 256x256 tiles to occupy the chip (a 1024^3
-// GEMM has 16 of them for 256 CUs): 4 waves, each a 64x64 patch (16 MFMA tiles), three LDS
-// stages of 2 x 16 KiB with two K-steps of loads in flight, plain loop (such problems are
-// bound by launch, prologue and epilogue latency, not by the K loop's schedule). Same tile
-// format, B-row permutation and epilogue as the large-tile kernels.
+// GEMM has 16 of them for 256 CUs): 4 waves, each a 64x64 patch (16 MFMA tiles), four LDS
+// stages of 2 x 16 KiB (MXFP4: three). Same tile format, B-row permutation and epilogue as the
+// large-tile kernels.
 constexpr int kSmallTile = 128;
 constexpr int kSmallTileBytes = kSmallTile * BK;          // 16 KiB per operand
 constexpr int kSmallStageBytes = 2 * kSmallTileBytes;
-constexpr int kSmallStages = 3;
-constexpr int kSmallLdsBytes = kSmallStages * kSmallStageBytes;  // 96 KiB
+constexpr int kSmallStages = 4, kSmallStagesScaled = 3;
 // the same kernel with 64x64 tiles and four 16 KiB stages (two workgroups per CU): for problems
 // with so few 128x128 tiles that a quarter of the tile is needed to give every CU work
 constexpr int kTinyTile = 64;
@@ -58,7 +56,7 @@ __device__ __forceinline__ void gemm_small_tile_body(
     constexpr int LPT = 2 * NDMA + (kScaled ? 1 : 0);  // loads per wave per K-step
     // scales: four slots, each the 16 bytes (two K-steps) of the TILE rows of A, then of B
     constexpr int kScaleSlot = 2 * TILE * 16, kScaleBase = STAGES * kSB;
-    static_assert(STAGES >= 3 && STAGES <= 8 && (STAGES - 2) * LPT < 64, "vmcnt range");
+    static_assert(STAGES >= 3 && STAGES <= 8 && (STAGES - 1) * LPT < 64, "vmcnt range");
     static_assert(!kScaled || STAGES <= 5, "four scale slots cover the K-step pairs of at most five stages");
     const int lane = lane_id(), w = wave_id();
     const int wm = w >> 1, wn = w & 1;
@@ -153,49 +151,117 @@ __device__ __forceinline__ void gemm_small_tile_body(
 #pragma unroll
         for (int n = 0; n < NT; ++n) acc[m][n] = v4f{0.f, 0.f, 0.f, 0.f};
 
-    // K-steps kt .. kt + STAGES - 2 are in flight or in LDS while step kt is multiplied
+    if constexpr (kScaled) {
+        // K-steps kt .. kt + STAGES - 2 are in flight or in LDS while step kt is multiplied
 #pragma unroll
-    for (int p = 0; p < STAGES - 1; ++p)
-        if (p < nkt) issue_tile(p, p);
-    int st = 0;
-    for (int kt = 0; kt < nkt; ++kt) {
-        // this wave's part of K-step kt has landed (the loads of the steps behind it may still fly)
-        wait_tiles(min(nkt - 1 - kt, STAGES - 2));
-        block_barrier();  // ... everyone's; and everyone is done with the stage of K-step kt - 1
-        if (kt + STAGES - 1 < nkt) issue_tile(st == 0 ? STAGES - 1 : st - 1, kt + STAGES - 1);
-        const uint32_t so = (uint32_t)st * kSB;
-        v8i bf[NT];
+        for (int p = 0; p < STAGES - 1; ++p)
+            if (p < nkt) issue_tile(p, p);
+        int st = 0;
+        for (int kt = 0; kt < nkt; ++kt) {
+            // this wave's part of K-step kt has landed (the loads of the steps behind it may still fly)
+            wait_tiles(min(nkt - 1 - kt, STAGES - 2));
+            block_barrier();  // ... everyone's; and everyone is done with the stage of K-step kt - 1
+            if (kt + STAGES - 1 < nkt) issue_tile(st == 0 ? STAGES - 1 : st - 1, kt + STAGES - 1);
+            const uint32_t so = (uint32_t)st * kSB;
+            v8i bf[NT];
 #pragma unroll
-        for (int n = 0; n < NT; ++n) bf[n] = lds_frag(b_lo0 + so, b_hi0 + so, n * 16 * BK);
-        if constexpr (kScaled) {
-            // the lane's scale bytes: row 16 f + r of the wave's patch, byte g of each half's dword
-            const int ktg = kt0 + kt;
-            const uint32_t sbase = lds0 + kScaleBase + (uint32_t)((ktg >> 1) & 3) * kScaleSlot + (uint32_t)(ktg & 1) * 8u + r * 16u +
-                                   ((ktg >> 1) == sc.tail_pair ? (uint32_t)sc.tail_shift : 0u);
-            const uint32_t sh = 8u * g;
-            v2i bs[NT];
+            for (int n = 0; n < NT; ++n) bf[n] = lds_frag(b_lo0 + so, b_hi0 + so, n * 16 * BK);
+            {
+                // the lane's scale bytes: row 16 f + r of the wave's patch, byte g of each half's dword
+                const int ktg = kt0 + kt;
+                const uint32_t sbase = lds0 + kScaleBase + (uint32_t)((ktg >> 1) & 3) * kScaleSlot + (uint32_t)(ktg & 1) * 8u + r * 16u +
+                                       ((ktg >> 1) == sc.tail_pair ? (uint32_t)sc.tail_shift : 0u);
+                const uint32_t sh = 8u * g;
+                v2i bs[NT];
 #pragma unroll
-            for (int n = 0; n < NT; ++n) {
-                bs[n] = *(lds_v2i_t*)(uintptr_t)(sbase + TILE * 16 + (wn * TN + 16 * n) * 16);
-                bs[n].x = (int)((uint32_t)bs[n].x >> sh); bs[n].y = (int)((uint32_t)bs[n].y >> sh);
+                for (int n = 0; n < NT; ++n) {
+                    bs[n] = *(lds_v2i_t*)(uintptr_t)(sbase + TILE * 16 + (wn * TN + 16 * n) * 16);
+                    bs[n].x = (int)((uint32_t)bs[n].x >> sh); bs[n].y = (int)((uint32_t)bs[n].y >> sh);
+                }
+#pragma unroll
+                for (int m = 0; m < MT; ++m) {
+                    const v8i af = lds_frag(a_lo0 + so, a_hi0 + so, m * 16 * BK);
+                    v2i as = *(lds_v2i_t*)(uintptr_t)(sbase + (wm * TM + 16 * m) * 16);
+                    as.x = (int)((uint32_t)as.x >> sh); as.y = (int)((uint32_t)as.y >> sh);
+#pragma unroll
+                    for (int n = 0; n < NT; ++n) MMA::mma(acc[m][n], bf[n], af, bs[n], as);
+                }
             }
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                const v8i af = lds_frag(a_lo0 + so, a_hi0 + so, m * 16 * BK);
-                v2i as = *(lds_v2i_t*)(uintptr_t)(sbase + (wm * TM + 16 * m) * 16);
-                as.x = (int)((uint32_t)as.x >> sh); as.y = (int)((uint32_t)as.y >> sh);
-#pragma unroll
-                for (int n = 0; n < NT; ++n) MMA::mma(acc[m][n], bf[n], af, bs[n], as);
-            }
-        } else {
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                const v8i af = lds_frag(a_lo0 + so, a_hi0 + so, m * 16 * BK);
-#pragma unroll
-                for (int n = 0; n < NT; ++n) MMA::mma(acc[m][n], bf[n], af);
-            }
+            st = st == STAGES - 1 ? 0 : st + 1;
         }
-        st = st == STAGES - 1 ? 0 : st + 1;
+    } else {
+        // The reads of the next K-step's fragments and the loads of K-step kt + STAGES are spread over the MFMAs of
+        // K-step kt. One wave per SIMD runs a 128x128 tile, and LDS reads in front of the MFMAs leave the matrix cores
+        // idle while the LDS delivers 64 KiB and takes in 32 KiB per K-step (768 clocks against the MFMAs' 512).
+        // us, reads first / spread (and four stages instead of three with 128x128 tiles): FP8 1024^3 5.1 / 4.6, 2048^3
+        // 13.5 / 11.6, M = 400, N = K = 4096 22.3 / 17.9 (128x128 tiles), M = 128, N = 1024, K = 8192 20.7 / 16.4;
+        // BF16 1024^3 7.5 / 6.3, 1000 x 4096 x 4096 42.2 / 38.7. The scaled FP4 MFMAs are half as long and need two
+        // shifts per scale and fragment beside them: the same order is 5 to 12 % slower there, so that form keeps its
+        // reads in front.
+        struct Frags { v8i a[MT], b[NT]; };
+        Frags fr[2];
+        // fragment x of the K-step in stage `stage`: B's NT, then A's MT
+        auto read_frag = [&](Frags& f, int stage, int x) __attribute__((always_inline)) {
+            const uint32_t so = (uint32_t)stage * kSB;
+            if (x < NT) f.b[x < NT ? x : 0] = lds_frag(b_lo0 + so, b_hi0 + so, x * 16 * BK);
+            else f.a[x >= NT ? x - NT : 0] = lds_frag(a_lo0 + so, a_hi0 + so, (x - NT) * 16 * BK);
+        };
+        // load j (A's pieces, then B's) of K-step kt_local. Past the last one the descriptors are empty (zeros arrive):
+        // every K-step is followed by the same number of loads, which keeps the counted waits constant and the K loop
+        // free of branches.
+        auto issue_load = [&](int stage, int kt_local, int j) __attribute__((always_inline)) {
+            const int kt = kt0 + min(kt_local, nkt - 1);
+            v4i da = srd_a, db = srd_b;
+            if (kt_local >= nkt) { da.z = 0; db.z = 0; }
+            const uint32_t k0 = (uint32_t)kt * BK, vor = kt == nk - 1 ? tail_or : 0u;
+            const uint32_t dst = lds_wave + (uint32_t)stage * kSB;
+            if (j < NDMA) dma16(da, dst + j * NW * 1024, voff_a[j < NDMA ? j : 0] | vor, k0);
+            else dma16(db, dst + kTB + (j - NDMA) * NW * 1024, voff_b[j >= NDMA ? j - NDMA : 0] | vor, k0);
+        };
+        // all stages are filled ahead; stage kt is free for K-step kt + STAGES once everyone's fragments of K-step kt
+        // are in registers
+#pragma unroll
+        for (int p = 0; p < STAGES; ++p)
+#pragma unroll
+            for (int j = 0; j < LPT; ++j) issue_load(p, p, j);
+        wait_vmcnt<(STAGES - 1) * LPT>();
+        block_barrier();
+#pragma unroll
+        for (int x = 0; x < MT + NT; ++x) read_frag(fr[0], 0, x);
+        int st = 0, kt = 0;   // stage of K-step kt
+        auto step = [&]<int P, bool LAST>() __attribute__((always_inline)) {
+            Frags &cur = fr[P], &nxt = fr[P ^ 1];
+            constexpr int kMma = MT * NT, kFirst = NT / 2;   // MFMAs in all, in front of the barrier
+            constexpr int kItems = MT + NT + LPT;
+            static_assert(MT + NT == LPT, "reads and loads alternate");
+            const int st_next = st == STAGES - 1 ? 0 : st + 1;
+#pragma unroll
+            for (int q = 0; q < (LAST ? kMma : kFirst); ++q) MMA::mma(acc[q / NT][q % NT], cur.b[q % NT], cur.a[q / NT]);
+            if constexpr (LAST) return;
+            // this wave's part of the next K-step has landed and its fragments of this one are in registers ...
+            wait_vmcnt<(STAGES - 2) * LPT>();
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            block_barrier();   // ... and so are everyone's
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int q = kFirst; q < kMma; ++q) {
+                MMA::mma(acc[q / NT][q % NT], cur.b[q % NT], cur.a[q / NT]);
+#pragma unroll
+                for (int i = (q - kFirst) * kItems / (kMma - kFirst); i < (q - kFirst + 1) * kItems / (kMma - kFirst); ++i) {
+                    if ((i & 1) == 0) read_frag(nxt, st_next, i >> 1);
+                    else issue_load(st, kt + STAGES, i >> 1);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            st = st_next;
+            ++kt;
+        };
+        while (kt + 1 < nkt) {
+            step.template operator()<0, false>();
+            step.template operator()<1, false>();
+        }
+        if (kt < nkt) step.template operator()<0, true>();
+        wait_vmcnt<0>();   // nothing may still be writing LDS when the workgroup retires
     }
     if (!SPLIT) {
         store_c_tile<MT, NT, EDGE>(acc, C, M, N, row0 + wm * TM, col0 + wn * TN, alpha);

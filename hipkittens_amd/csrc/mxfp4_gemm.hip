@@ -588,8 +588,8 @@ static int mxfp4_gemm_impl(const void* A, const void* A_scales, int sa_pitch, co
     if (!size_ok || !sr.ok) return HK_ERR_BAD_SHAPE;
     if (variant == 2) {
         const bool e = (M % kSmallTile) != 0 || (N % kSmallTile) != 0;
-        return e ? launch_mxfp4_small_tile<kSmallTile, kSmallStages, true>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s)
-                 : launch_mxfp4_small_tile<kSmallTile, kSmallStages, false>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s);
+        return e ? launch_mxfp4_small_tile<kSmallTile, kSmallStagesScaled, true>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s)
+                 : launch_mxfp4_small_tile<kSmallTile, kSmallStagesScaled, false>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s);
     }
     if (variant == 3) {
         const bool e = (M % kTinyTile) != 0 || (N % kTinyTile) != 0;
