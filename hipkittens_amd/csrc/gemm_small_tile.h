@@ -323,9 +323,10 @@ static __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* 
 //     tile count cannot: 72 tiles of 256 are one round where their 288 tiles of 128 are two (the large tile
 //     wins by 4-12 % from a K of about 4096 elements on), 64 tiles of 256 are one round of four times the work
 //     of the single round of 256 small tiles (the small tile wins by 60 %). Measured against the best of the
-//     three kernels on 360 shapes per format, every launch on another copy of B (a model's weights come from HBM, not
-//     from the memory-side cache), the rule alone is more than 5 % behind on 9 / 22 / 20 shapes (FP8 / BF16 /
-//     MXFP4), mostly by 5 to 10 % where a long B is read by several rows of small tiles;
+//     three kernels, every launch on another copy of B (a model's weights come from HBM, not from the memory-side
+//     cache), the rule alone is more than 5 % behind on 7 / 5 of 414 shapes (FP8 / BF16; 42 / 40 with the constants
+//     that fitted these kernels before their loads and LDS reads were spread over the MFMAs) and on 20 of 360 (MXFP4),
+//     mostly by 5 to 10 % where a long B is read by several rows of small tiles;
 //  2. a generated table of the shapes on which a sweep found the rule's choice more than a few percent behind
 //     another tile (tile_table.inc, written by `python -m hipkittens_amd.tile_sweep FORMAT --emit`; the
 //     counterpart of the reference's per-shape analysis/baselines/gemm/utils/tuned.yaml). An entry is keyed by
@@ -368,8 +369,8 @@ static inline int pick_tile(int fmt, int M, int N, int nk, TileRule r, bool cons
     return pick_tile_rule(M, N, nk, r, cus);
 }
 // the formats' constants (K-steps: 128 bytes of an operand row)
-constexpr TileRule kTileRuleFp8{{7.43f, 3.28f, 2.02f}, {1.078f, 0.585f, 0.372f}};
-constexpr TileRule kTileRuleBf16{{7.75f, 3.15f, 2.17f}, {1.051f, 0.562f, 0.336f}};
+constexpr TileRule kTileRuleFp8{{7.10f, 3.28f, 2.02f}, {1.060f, 0.533f, 0.385f}};
+constexpr TileRule kTileRuleBf16{{8.57f, 2.79f, 2.20f}, {0.983f, 0.495f, 0.336f}};
 constexpr TileRule kTileRuleMxfp4{{7.71f, 3.13f, 1.94f}, {1.316f, 0.767f, 0.549f}};
 
 // Number of K ranges the split-K path would use: as many as fill the CUs, each at least 4
