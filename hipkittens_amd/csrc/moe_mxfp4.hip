@@ -1389,6 +1389,8 @@ namespace hk {
 // lane (gridDim.y): with a workgroup per token most CUs have nothing to do, and its 256 threads go over the
 // columns two (H = 2880) to four times (7168) in turn. Layer times, a workgroup per token / shared: 4 tokens,
 // H = 2880, k = 4 50.9 / 50.4 us (the kernel itself 3.9 us now); 16 tokens, H = 7168, k = 8 673.3 / 670.8 (4.6 us).
+// The kernel back to back: 4 tokens, H = 2880 2.4 / 2.1 us; H = 7168, k = 8: 16 tokens 4.7 / 2.5, 128 6.0 / 3.4,
+// 255 7.0 / 5.1; from 256 on there is a workgroup for every CU either way (not measured split).
 // o has T * k rows; a position outside [0, T * k) (a caller's broken slot_to_pos) is not read and adds
 // nothing, like an expert id out of range in the sort.
 constexpr int kUnpermuteSplitTokens = 256;   // a workgroup for every CU
