@@ -967,12 +967,13 @@ static int moe_fp8blk_item_rows(int T, int k, int E) {
 // 1828 / 1927), or while the gate+up GEMM has less than 3/4 of an item of 16 rows per CU and an expert's weights are
 // not streamed more than twelve times (one expert, H = 7168, I = 2048: 16 rows 99 / 19, 100 rows 106 / 52, 200 rows
 // 89 / 89, 300 rows 104 / 138).
+constexpr int kF8FewMaxMean = 192;
 static bool moe_fp8blk_few(int T, int H, int I, int E, int k) {
     const long long S = (long long)T * k;
     if (S * (H > I ? H : I) >= (1ll << 31)) return false;   // its row offsets keep bit 31 free
     if (S <= 2ll * E) return true;
     const long long m_tiles = S / kF8FewRows + min((long long)E, S);
-    return S <= 192ll * E && m_tiles * (I / 128) * 4 <= 3ll * moe_num_compute_units();
+    return S <= (long long)kF8FewMaxMean * E && m_tiles * (I / 128) * 4 <= 3ll * moe_num_compute_units();
 }
 
 // n-tiles of 256 weight rows of the two GEMMs: gate+up (mode 0: 128 h columns = 128 gate + 128 up rows
@@ -980,9 +981,12 @@ static bool moe_fp8blk_few(int T, int H, int I, int E, int k) {
 static inline int fp8blk_n_tiles(int mode, int N) { return mode == 0 ? N / 128 : (int)(((long long)N + 255) / 256); }
 
 struct Fp8Ws {
-    size_t ids, w, sorted, offsets, inv, sort_ws, items1, items2, nitems, xq, xs, hq, hs, hf, o, total;
+    size_t ids, w, sorted, offsets, inv, sort_ws, items1, items2, nitems, xq, xs, hq, hs, o, total;
     int max_items1, max_items2;
 };
+// No region shrinks when T grows (a workspace allocated for the largest batch serves every smaller one), and none
+// depends on the device: the item lists and h in fp32 have room for the few-rows kernel wherever any device's rule
+// could choose it.
 static Fp8Ws fp8_ws_layout(int T, int H, int I, int E, int k) {
     Fp8Ws L;
     size_t off = 0;
@@ -990,8 +994,8 @@ static Fp8Ws fp8_ws_layout(int T, int H, int I, int E, int k) {
     const size_t S = (size_t)T * k;
     L.ids = take(S * 4); L.w = take(S * 4); L.sorted = take(S * 4); L.offsets = take((size_t)(E + 1) * 4);
     L.inv = take(S * 4); L.sort_ws = take(hk_moe_sort_workspace_bytes(T, k, E));
-    const bool few = moe_fp8blk_few(T, H, I, E, k);
-    const int max_tiles = (int)(S / (few ? kF8FewRows : kF8BMShort)) + E;   // whichever item size the layer runs with
+    const size_t few_rows = std::min(S, (size_t)kF8FewMaxMean * E);   // slots of the largest batch that few-rows items cover
+    const int max_tiles = (int)std::max(few_rows / kF8FewRows, S / kF8BMShort) + E;
     L.max_items1 = max_tiles * (I / 128);
     L.max_items2 = max_tiles * ((H + 255) / 256);
     L.items1 = take((size_t)L.max_items1 * sizeof(MoeItem));
@@ -1001,8 +1005,8 @@ static Fp8Ws fp8_ws_layout(int T, int H, int I, int E, int k) {
     // gathers activation rows by token index: there is no permuted copy)
     L.xq = take((size_t)T * H); L.xs = take((size_t)T * (H / 128) * 4);
     L.hq = take(S * (size_t)I); L.hs = take(S * (size_t)(I / 128) * 4);
-    L.hf = take(few ? S * (size_t)I * 4 : 0);   // h before its quantization (few-rows kernel)
-    L.o = take(S * (size_t)H * 2);
+    // o, and before it h in fp32 (few-rows kernel: quantized to hq before the down GEMM writes o)
+    L.o = take(std::max(S * (size_t)H * 2, few_rows * (size_t)I * 4));
     L.total = off;
     return L;
 }
@@ -1117,7 +1121,7 @@ static int fp8blk_grouped_gemms(const void* x_e4m3, const float* x_scales, const
     p.B = (const uint8_t*)w13; p.SB = w13_scales;
     p.b_expert_stride = (long long)2 * I * H; p.sb_expert_stride = (long long)(2 * I / 128) * (H / 128);
     p.items = lists ? (const MoeItem*)(ws + L.items1) : nullptr; p.num_items = nitems;
-    p.out0 = ws + (few ? L.hf : L.hq); p.out_scales = (float*)(ws + L.hs);
+    p.out0 = ws + (few ? L.o : L.hq); p.out_scales = (float*)(ws + L.hs);
     p.K = H; p.N = I; p.n_tiles_n = I / 128;
     int st;
     if (weight_layout == 1) p.b_expert_stride = (long long)fp8blk_n_tiles(0, I) * (H / 128) * kF8sBTile;
@@ -1127,7 +1131,7 @@ static int fp8blk_grouped_gemms(const void* x_e4m3, const float* x_scales, const
     if (st != HK_OK) return st;
     if (few) {
         hipLaunchKernelGGL(moe_fp8blk_few_quantize_kernel, dim3((unsigned)(((long long)S * (I / 8) + 255) / 256)), dim3(256),
-                           0, s, (const float*)(ws + L.hf), S, I, ws + L.hq, (float*)(ws + L.hs));
+                           0, s, (const float*)(ws + L.o), S, I, ws + L.hq, (float*)(ws + L.hs));
         if (hipGetLastError() != hipSuccess) return HK_ERR_LAUNCH;
     }
 

@@ -1599,12 +1599,14 @@ extern "C" int hk_moe_mxfp4_preshuffle(const void* w, const void* scales, int sc
 // is the better one: by the mean number of rows per expert. Routers load their experts unevenly, and an expert with
 // more rows than an item streams its weights again: one fragment of 16 rows up to a mean of 4, two up to 8 (MXFP4
 // activations only: MXFP8 rows are twice the traffic), measured in the header's comment.
+constexpr int kFewMaxMean16 = 4, kFewMaxMean32 = 8;
 static int moe_few_rows(int T, int k, int E, bool a8) {
     const long long S = (long long)T * k;
-    return S <= 4ll * E ? 16 : S <= 8ll * E && !a8 ? 32 : 0;
+    return S <= (long long)kFewMaxMean16 * E ? 16 : S <= (long long)kFewMaxMean32 * E && !a8 ? 32 : 0;
 }
 
-// Workspace layout of hk_moe_mxfp4_forward (all regions 256-byte aligned).
+// Workspace layout of hk_moe_mxfp4_forward (all regions 256-byte aligned). No region shrinks when T grows: a workspace
+// allocated for the largest batch serves every smaller one.
 struct MoeWs {
     size_t ids, w, sorted, offsets, inv, sort_ws, items1, items2, nitems, xq, xs, hq, hs, o, total;
     int max_items1, max_items2;
@@ -1616,8 +1618,9 @@ static MoeWs moe_ws_layout(int T, int H, int I, int E, int k, bool a8 = false) {
     const size_t S = (size_t)T * k;
     L.ids = take(S * 4); L.w = take(S * 4); L.sorted = take(S * 4); L.offsets = take((size_t)(E + 1) * 4);
     L.inv = take(S * 4); L.sort_ws = take(hk_moe_sort_workspace_bytes(T, k, E));
-    const int few = moe_few_rows(T, k, E, a8);
-    const int max_tiles = (int)(S / (few ? few : kMoeBM)) + E;
+    // items of 16, 32 or kMoeBM rows (moe_few_rows), each up to the largest S that they are used for
+    const size_t few_tiles = std::max(std::min(S, (size_t)kFewMaxMean16 * E) / 16, a8 ? 0 : std::min(S, (size_t)kFewMaxMean32 * E) / 32);
+    const int max_tiles = (int)std::max(few_tiles, S / kMoeBM) + E;
     L.max_items1 = max_tiles * ((I + 127) / 128);
     L.max_items2 = max_tiles * ((H + 255) / 256);
     L.items1 = take((size_t)L.max_items1 * sizeof(MoeItem));
