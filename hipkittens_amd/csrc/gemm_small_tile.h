@@ -130,11 +130,12 @@ __device__ __forceinline__ void gemm_small_tile_body(
         switch (tiles) {
             case 0: wait_vmcnt<0>(); break;
             case 1: wait_vmcnt<LPT>(); break;
-            case 2: wait_vmcnt<(STAGES > 3 ? 2 : 1) * LPT>(); break;
-            case 3: wait_vmcnt<(STAGES > 4 ? 3 : 1) * LPT>(); break;
-            case 4: wait_vmcnt<(STAGES > 5 ? 4 : 1) * LPT>(); break;
-            case 5: wait_vmcnt<(STAGES > 6 ? 5 : 1) * LPT>(); break;
-            default: wait_vmcnt<(STAGES > 7 ? 6 : 1) * LPT>(); break;
+            case 2: wait_vmcnt<(STAGES > 2 ? 2 : 1) * LPT>(); break;
+            case 3: wait_vmcnt<(STAGES > 3 ? 3 : 1) * LPT>(); break;
+            case 4: wait_vmcnt<(STAGES > 4 ? 4 : 1) * LPT>(); break;
+            case 5: wait_vmcnt<(STAGES > 5 ? 5 : 1) * LPT>(); break;
+            case 6: wait_vmcnt<(STAGES > 6 ? 6 : 1) * LPT>(); break;
+            default: wait_vmcnt<(STAGES > 7 ? 7 : 1) * LPT>(); break;
         }
     };
 
@@ -193,11 +194,13 @@ __device__ __forceinline__ void gemm_small_tile_body(
         // The reads of the next K-step's fragments and the loads of K-step kt + STAGES are spread over the MFMAs of
         // K-step kt. One wave per SIMD runs a 128x128 tile, and LDS reads in front of the MFMAs leave the matrix cores
         // idle while the LDS delivers 64 KiB and takes in 32 KiB per K-step (768 clocks against the MFMAs' 512).
-        // us, reads first / spread (and four stages instead of three with 128x128 tiles): FP8 1024^3 5.1 / 4.6, 2048^3
-        // 13.5 / 11.6, M = 400, N = K = 4096 22.3 / 17.9 (128x128 tiles), M = 128, N = 1024, K = 8192 20.7 / 16.4;
-        // BF16 1024^3 7.5 / 6.3, 1000 x 4096 x 4096 42.2 / 38.7. The scaled FP4 MFMAs are half as long and need two
-        // shifts per scale and fragment beside them: the same order is 5 to 12 % slower there, so that form keeps its
-        // reads in front.
+        // us, reads first / spread (and four stages instead of three with 128x128 tiles): FP8 1024^3 5.0 / 4.2, 2048^3
+        // 13.2 / 10.3, 400 x 6000 x 4096 22.6 / 18.7; BF16 1024^3 7.4 / 5.6, 2048^3 22.3 / 19.0. The scaled FP4 MFMAs are
+        // half as long and need two shifts per scale and fragment beside them: the same order is 5 to 12 % slower there,
+        // so that form keeps its reads in front.
+        // No loads go out past the last K-step: as loads of zeros that keep the waits constant they made few K-steps
+        // slower than with the reads first (FP8, reads first / spread with them / spread without: 512 x 4096 x 256 3.7 / 4.2
+        // / 3.5, 17 x 32512 x 1024 8.5 / 9.1 / 8.5), and many K-steps 1 to 8 % slower than without.
         struct Frags { v8i a[MT], b[NT]; };
         Frags fr[2];
         // fragment x of the K-step in stage `stage`: B's NT, then A's MT
@@ -206,40 +209,42 @@ __device__ __forceinline__ void gemm_small_tile_body(
             if (x < NT) f.b[x < NT ? x : 0] = lds_frag(b_lo0 + so, b_hi0 + so, x * 16 * BK);
             else f.a[x >= NT ? x - NT : 0] = lds_frag(a_lo0 + so, a_hi0 + so, (x - NT) * 16 * BK);
         };
-        // load j (A's pieces, then B's) of K-step kt_local. Past the last one the descriptors are empty (zeros arrive):
-        // every K-step is followed by the same number of loads, which keeps the counted waits constant and the K loop
-        // free of branches.
+        // load j (A's pieces, then B's) of K-step kt_local < nkt
         auto issue_load = [&](int stage, int kt_local, int j) __attribute__((always_inline)) {
-            const int kt = kt0 + min(kt_local, nkt - 1);
-            v4i da = srd_a, db = srd_b;
-            if (kt_local >= nkt) { da.z = 0; db.z = 0; }
+            const int kt = kt0 + kt_local;
             const uint32_t k0 = (uint32_t)kt * BK, vor = kt == nk - 1 ? tail_or : 0u;
             const uint32_t dst = lds_wave + (uint32_t)stage * kSB;
-            if (j < NDMA) dma16(da, dst + j * NW * 1024, voff_a[j < NDMA ? j : 0] | vor, k0);
-            else dma16(db, dst + kTB + (j - NDMA) * NW * 1024, voff_b[j >= NDMA ? j - NDMA : 0] | vor, k0);
+            if (j < NDMA) dma16(srd_a, dst + j * NW * 1024, voff_a[j < NDMA ? j : 0] | vor, k0);
+            else dma16(srd_b, dst + kTB + (j - NDMA) * NW * 1024, voff_b[j >= NDMA ? j - NDMA : 0] | vor, k0);
         };
         // all stages are filled ahead; stage kt is free for K-step kt + STAGES once everyone's fragments of K-step kt
         // are in registers
 #pragma unroll
         for (int p = 0; p < STAGES; ++p)
+            if (p < nkt) {
 #pragma unroll
-            for (int j = 0; j < LPT; ++j) issue_load(p, p, j);
-        wait_vmcnt<(STAGES - 1) * LPT>();
+                for (int j = 0; j < LPT; ++j) issue_load(p, p, j);
+            }
+        wait_tiles(min(nkt, STAGES) - 1);
         block_barrier();
 #pragma unroll
         for (int x = 0; x < MT + NT; ++x) read_frag(fr[0], 0, x);
         int st = 0, kt = 0;   // stage of K-step kt
-        auto step = [&]<int P, bool LAST>() __attribute__((always_inline)) {
+        // K-step kt with its fragments in fr[P]. kMain: constant wait, the loads of K-step kt + STAGES among the MFMAs;
+        // kTail: counted wait, no loads; kLast: the MFMAs alone.
+        enum { kMain, kTail, kLast };
+        auto step = [&]<int P, int KIND>() __attribute__((always_inline)) {
             Frags &cur = fr[P], &nxt = fr[P ^ 1];
             constexpr int kMma = MT * NT, kFirst = NT / 2;   // MFMAs in all, in front of the barrier
             constexpr int kItems = MT + NT + LPT;
             static_assert(MT + NT == LPT, "reads and loads alternate");
             const int st_next = st == STAGES - 1 ? 0 : st + 1;
 #pragma unroll
-            for (int q = 0; q < (LAST ? kMma : kFirst); ++q) MMA::mma(acc[q / NT][q % NT], cur.b[q % NT], cur.a[q / NT]);
-            if constexpr (LAST) return;
+            for (int q = 0; q < (KIND == kLast ? kMma : kFirst); ++q) MMA::mma(acc[q / NT][q % NT], cur.b[q % NT], cur.a[q / NT]);
+            if constexpr (KIND == kLast) return;
             // this wave's part of the next K-step has landed and its fragments of this one are in registers ...
-            wait_vmcnt<(STAGES - 2) * LPT>();
+            if constexpr (KIND == kMain) wait_vmcnt<(STAGES - 2) * LPT>();
+            else wait_tiles(min(nkt - kt, STAGES) - 2);
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             block_barrier();   // ... and so are everyone's
             __builtin_amdgcn_sched_barrier(0);
@@ -249,19 +254,42 @@ __device__ __forceinline__ void gemm_small_tile_body(
 #pragma unroll
                 for (int i = (q - kFirst) * kItems / (kMma - kFirst); i < (q - kFirst + 1) * kItems / (kMma - kFirst); ++i) {
                     if ((i & 1) == 0) read_frag(nxt, st_next, i >> 1);
-                    else issue_load(st, kt + STAGES, i >> 1);
+                    else if (KIND == kMain) issue_load(st, kt + STAGES, i >> 1);
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
             st = st_next;
             ++kt;
         };
-        while (kt + 1 < nkt) {
-            step.template operator()<0, false>();
-            step.template operator()<1, false>();
+        // an even count's first K-step by itself, its reads behind its MFMAs: an odd one is left, so that the last K-step's
+        // fragments are in fr[0] (a last K-step in either buffer costs the 128x128 tile its registers)
+        if ((nkt & 1) == 0) {
+#pragma unroll
+            for (int q = 0; q < MT * NT; ++q) MMA::mma(acc[q / NT][q % NT], fr[0].b[q % NT], fr[0].a[q / NT]);
+            wait_tiles(min(nkt, STAGES) - 2);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            block_barrier();
+            if (STAGES < nkt) {
+#pragma unroll
+                for (int j = 0; j < LPT; ++j) issue_load(0, STAGES, j);
+            }
+            st = kt = 1;
+#pragma unroll
+            for (int x = 0; x < MT + NT; ++x) read_frag(fr[0], 1, x);
         }
-        if (kt < nkt) step.template operator()<0, true>();
-        wait_vmcnt<0>();   // nothing may still be writing LDS when the workgroup retires
+        while (kt + 1 + STAGES < nkt) {
+            step.template operator()<0, kMain>();
+            step.template operator()<1, kMain>();
+        }
+        if (kt + STAGES < nkt) {
+            step.template operator()<0, kMain>();
+            step.template operator()<1, kTail>();
+        }
+        while (kt + 1 < nkt) {
+            step.template operator()<0, kTail>();
+            step.template operator()<1, kTail>();
+        }
+        step.template operator()<0, kLast>();
     }
     if (!SPLIT) {
         store_c_tile<MT, NT, EDGE>(acc, C, M, N, row0 + wm * TM, col0 + wn * TN, alpha);
