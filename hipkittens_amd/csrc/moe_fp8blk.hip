@@ -916,7 +916,10 @@ namespace hk {
 // The few-rows kernel for as many items as the list can hold (the workgroups past its actual length leave at once).
 template <int MODE>
 static int launch_fp8blk_few(const MoeFp8Params& p, long long max_items, hipStream_t s) {
-    hipLaunchKernelGGL(moe_fp8blk_few_kernel<MODE>, dim3((unsigned)(8 * max_items)), dim3(64), 0, s, p);
+    // (a ring of seven K-steps for a K of four at most fetches past its end: the two calls above 410 -> 405, 97 -> 94 us; a
+    // longer K wants the seven in flight: one expert of H = 7168, I = 2048, 16 rows 36 us against 39 with four)
+    auto kern = p.K <= 512 ? moe_fp8blk_few_kernel<MODE, 4> : moe_fp8blk_few_kernel<MODE, 7>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)(8 * max_items)), dim3(64), 0, s, p);
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
@@ -961,12 +964,12 @@ static int moe_fp8blk_item_rows(int T, int k, int E) {
     return n_short <= n_long ? kF8BMShort : kF8BM;
 }
 
-// Whether a layer on pre-shuffled weights takes the few-rows kernel (moe_fp8blk_few.h has the measurements): with a
-// mean of at most 2 rows per expert (H = 7168, I = 2048, E = 256, k = 8, us, streaming / few-rows kernel: 1 token
-// 112 / 93, 4 tokens 266 / 254, 16 tokens 754 / 713, 64 tokens 1567 / 1534, 128 tokens 1765 / 1771, 256 tokens
-// 1828 / 1927), or while the gate+up GEMM has less than 3/4 of an item of 16 rows per CU and an expert's weights are
-// not streamed more than twelve times (one expert, H = 7168, I = 2048: 16 rows 99 / 19, 100 rows 106 / 52, 200 rows
-// 89 / 89, 300 rows 104 / 138).
+// Whether a layer on pre-shuffled weights takes the few-rows kernel: with a mean of at most 2 rows per expert
+// (H = 7168, I = 2048, E = 256, k = 8, us, streaming / few-rows kernel: 1 token 117 / 90, 4 tokens 262 / 244, 16 tokens
+// 746 / 704, 64 tokens 1549 / 1516, 128 tokens 1738 / 1748, 256 tokens 1794 / 1885), or while the gate+up GEMM has less
+// than 3/4 of an item of 16 rows per CU and an expert's weights are not streamed more than twelve times (one expert,
+// H = 7168, I = 2048: 16 rows 83 / 19, 100 rows 90 / 49, 200 rows 89 / 83, 300 rows 88 / 131). On 150 layers drawn inside
+// the rule (H 1024 to 8192, I 256 to 3072, 1 to 256 experts) it was 1.03 to 3.9 times as fast as the streaming kernel.
 constexpr int kF8FewMaxMean = 192;
 static bool moe_fp8blk_few(int T, int H, int I, int E, int k) {
     const long long S = (long long)T * k;

@@ -14,8 +14,8 @@
 //   - An item's 16 activation rows are fetched by every wave from L2: 2 KiB per 4 KiB of weights. (Items of 32 or 64
 //     rows were slower from 1 to 500 rows per expert.)
 //   - Same MFMAs, scaling FMAs and order per output element as the streaming kernel: identical bits.
-// Shared expert of that layer, its whole call, us, streaming / this kernel: 1 token 98 / 17, 16 tokens 99 / 19 (2.4
-// TB/s of weights), 64 tokens 101 / 33. moe_fp8blk_few has the rule and the routed layer's figures.
+// Shared expert of that layer, its whole call, us, streaming / this kernel: 1 token 97 / 16, 16 tokens 83 / 19 (2.4
+// TB/s of weights), 64 tokens 85 / 32. moe_fp8blk_few has the rule and the routed layer's figures.
 #pragma once
 
 namespace hk {
@@ -28,9 +28,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t f8few_rsrc(const void* p, uint
 
 // p.items null: one expert that holds all S rows in order, item i = rows kF8FewRows (i / n_tiles).., tile i % n_tiles.
 // p.sorted_slots null: row `pos` of the order is token pos.
-template <int MODE>
+// D: K-steps of the ring, D - 1 of them in flight.
+template <int MODE, int D>
 __global__ __launch_bounds__(64, 2) void moe_fp8blk_few_kernel(const MoeFp8Params p) {
-    constexpr int D = 7;
     constexpr int kNt = 2;   // cache policy of the weight loads: non-temporal
     const int it = blockIdx.x >> 3, w = blockIdx.x & 7;
     MoeItem item;
@@ -96,7 +96,8 @@ __global__ __launch_bounds__(64, 2) void moe_fp8blk_few_kernel(const MoeFp8Param
         fetch(ring[d], d);
         __builtin_amdgcn_sched_barrier(0);   // (a K-step's loads are older than the next one's: the waits count on it)
     }
-    for (int kt = 0; kt < nk; kt += D) {
+    int kt = 0;
+    for (; kt + D < nk; kt += D) {
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             fetch(ring[(d + D - 1) % D], kt + d + D - 1);
@@ -105,6 +106,13 @@ __global__ __launch_bounds__(64, 2) void moe_fp8blk_few_kernel(const MoeFp8Param
             __builtin_amdgcn_sched_barrier(0);
         }
     }
+    // The last D K-steps at most: nothing is fetched or multiplied past nk (as loads and MFMAs of zeros, up to D - 1 of them
+    // per wave, they made a narrow expert slower than the streaming kernel: H = 7168, I = 512, mean 2 rows of 256 experts,
+    // streaming 440, with them 461, without 410 us; 16 experts, mean 32 rows 98 / 107 / 97).
+    fetch(ring[D - 1], kt + D - 1);
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (kt + d < nk) compute(ring[d]);
 
     // lane (r, g) holds, for row r of the item, 8 columns of o (down) or gate and up of 4 columns of h
     if (r >= item.rows) return;
