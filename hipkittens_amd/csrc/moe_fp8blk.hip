@@ -1062,6 +1062,11 @@ extern "C" size_t hk_moe_fp8blk_workspace_bytes(int T, int H, int I, int E, int 
     return fp8_ws_layout(T, H, I, E, k).total;
 }
 
+extern "C" int hk_moe_fp8blk_few_rows(int T, int H, int I, int E, int k) {
+    if (fp8blk_check(T, H, I, E, k) != HK_OK) return HK_ERR_BAD_SHAPE;
+    return moe_fp8blk_few(T, H, I, E, k) ? kF8FewRows : 0;
+}
+
 extern "C" int hk_moe_fp8blk_preshuffle_bytes(int E, int N, int K, int mode, size_t* w_bytes) {
     if (!w_bytes) return HK_ERR_NULL_POINTER;
     if (E <= 0 || N <= 0 || K <= 0 || (K % 128) != 0 || (N % 128) != 0 || mode < 0 || mode > 1) return HK_ERR_BAD_SHAPE;

@@ -1598,11 +1598,28 @@ extern "C" int hk_moe_mxfp4_preshuffle(const void* w, const void* scales, int sc
 // Rows per work item of the few-rows kernel (moe_mxfp4_few.h, pre-shuffled weights), or 0 where the streaming kernel
 // is the better one: by the mean number of rows per expert. Routers load their experts unevenly, and an expert with
 // more rows than an item streams its weights again: one fragment of 16 rows up to a mean of 4, two up to 8 (MXFP4
-// activations only: MXFP8 rows are twice the traffic), measured in the header's comment.
+// activations only: MXFP8 rows are twice the traffic).
+// The exception is a layer that the streaming kernel runs at full rate: many items per CU (its last round is a small
+// part), and little of what it walks besides weights (an item takes K-steps in groups of four, and about one more for
+// its epilogue). Weights that are streamed again cost more than is gained there beyond a mean of 1. us, streaming / few-rows, plain
+// epilogues: 3072 x 3072, 128 experts, top-4 (walked / held 1.08, 18 items per CU): mean 1 188 / 190, 4 282 / 295, 8 299
+// / 321; H = I = 2048, 256 experts, top-8 (1.13, 24): mean 2 239 / 239, 4 262 / 270, 8 276 / 298. On the line's other side:
+// H = 2944, I = 2304 (1.26, 15): mean 4 228 / 219; the same 3072 with 64 experts (9 items per CU) mean 8 1.01 to 1.03
+// times as fast. With biases / clamped SwiGLU or MXFP8 rows the streaming kernel has more to do beside the weights: only
+// from 18 items per CU on, and up to a mean of 3 / 2 (4096 x 4096, 128 experts, biases: 1.02 times as fast at 3, 0.98 at
+// 4, 0.95 at 8; H = 5120, I = 2880, MXFP8: 1.0 at 2, 0.98 at 3); with both it is never ahead. Items of 32 rows lose
+// already at a walked / held of up to 1.35 from 18 items per CU on (H = 1664, I = 4096, 256 experts: 1.30, 39 items
+// per CU, mean 5 439 / 446, 8 456 / 490). (`ext`: biases, clamped SwiGLU or interleaved rows.)
 constexpr int kFewMaxMean16 = 4, kFewMaxMean32 = 8;
-static int moe_few_rows(int T, int k, int E, bool a8) {
+static int moe_few_rows(int T, int H, int I, int E, int k, bool a8, bool ext) {
     const long long S = (long long)T * k;
-    return S <= (long long)kFewMaxMean16 * E ? 16 : S <= (long long)kFewMaxMean32 * E && !a8 ? 32 : 0;
+    auto up = [](long long x, int m) { return (x + m - 1) / m; };
+    const long long n1 = up(I, 128), n2 = up(H, 256), items = E * (n1 + n2), cus = moe_num_compute_units();
+    // K-steps walked against those that hold weights, H I / (128 * 256) + H I / 256^2
+    const double ratio = (double)(n1 * (4 * up(H, 1024) + 1) + n2 * (4 * up(I, 1024) + 1)) / (3.0 * H * I / 65536);
+    if (ratio < 1.25 && items >= (a8 || ext ? 18 : 13) * cus && !(a8 && ext)) return S <= (a8 ? 2ll : ext ? 3ll : 1ll) * E ? 16 : 0;
+    if (S <= (long long)kFewMaxMean16 * E) return 16;
+    return S <= (long long)kFewMaxMean32 * E && !a8 && !(ratio < 1.35 && items >= 18 * cus) ? 32 : 0;
 }
 
 // Workspace layout of hk_moe_mxfp4_forward (all regions 256-byte aligned). No region shrinks when T grows: a workspace
@@ -1656,6 +1673,10 @@ static bool moe_mxfp4_shape_ok(int T, int H, int I, int E, int k) {
     return (long long)T * k < (1ll << 24) && (long long)T * k * (((I / 2 + 127) / 128) * 128) < (1ll << 31) &&
            (long long)T * k * (((H / 2 + 127) / 128) * 128) < (1ll << 31) && (long long)2 * I * (H / 2) < (1ll << 31) &&
            (long long)H * (I / 2) < (1ll << 31);
+}
+extern "C" int hk_moe_mxfp4_few_rows(int T, int H, int I, int E, int k, int mxfp8, int ext) {
+    if (!moe_mxfp4_shape_ok(T, H, I, E, k)) return HK_ERR_BAD_SHAPE;
+    return moe_few_rows(T, H, I, E, k, mxfp8 != 0, ext != 0);
 }
 static int moe_mxfp4_check(int T, int H, int I, int E, int k, int w13_scale_pitch, int w2_scale_pitch) {
     if (!moe_mxfp4_shape_ok(T, H, I, E, k)) return HK_ERR_BAD_SHAPE;
@@ -1743,7 +1764,7 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
     const int S = T * k;
 
     int32_t* nitems = (int32_t*)(ws + L.nitems);
-    const int few = weight_layout == 1 ? moe_few_rows(T, k, E, a8) : 0;
+    const int few = weight_layout == 1 ? moe_few_rows(T, H, I, E, k, a8, ext) : 0;
     const bool gather = few || moe_gathers(weight_layout, ext, a8, T, H);
     // non-temporal weight loads while most experts' rows fit one work item (their weights are then read
     // once): mean + one standard deviation of the rows per expert under uniform routing
@@ -1868,7 +1889,7 @@ static int moe_mxfp4_forward_impl(const void* x_bf16, const float* router_logits
     if (st != HK_OK) return st;
     const bool ext = bias13 || bias2 || activation != 0 || w13_interleaved;
     bool fused = false;
-    const int few = weight_layout == 1 ? moe_few_rows(T, k, E, a8) : 0;
+    const int few = weight_layout == 1 ? moe_few_rows(T, H, I, E, k, a8, ext) : 0;
     if ((few || moe_gathers(weight_layout, ext, a8, T, H)) && (long long)T * k <= kSortSmallMax && x_bf16 &&
         (((uintptr_t)x_bf16 | (uintptr_t)workspace) & 15u) == 0) {
         // sort, item lists and the quantization of x in one launch (moe_sort_quantize_kernel)
