@@ -1601,15 +1601,16 @@ extern "C" int hk_moe_mxfp4_preshuffle(const void* w, const void* scales, int sc
 // activations only: MXFP8 rows are twice the traffic).
 // The exception is a layer that the streaming kernel runs at full rate: many items per CU (its last round is a small
 // part), and little of what it walks besides weights (an item takes K-steps in groups of four, and about one more for
-// its epilogue). Weights that are streamed again cost more than is gained there beyond a mean of 1. us, streaming / few-rows, plain
-// epilogues: 3072 x 3072, 128 experts, top-4 (walked / held 1.08, 18 items per CU): mean 1 188 / 190, 4 282 / 295, 8 299
-// / 321; H = I = 2048, 256 experts, top-8 (1.13, 24): mean 2 239 / 239, 4 262 / 270, 8 276 / 298. On the line's other side:
-// H = 2944, I = 2304 (1.26, 15): mean 4 228 / 219; the same 3072 with 64 experts (9 items per CU) mean 8 1.01 to 1.03
-// times as fast. With biases / clamped SwiGLU or MXFP8 rows the streaming kernel has more to do beside the weights: only
-// from 18 items per CU on, and up to a mean of 3 / 2 (4096 x 4096, 128 experts, biases: 1.02 times as fast at 3, 0.98 at
-// 4, 0.95 at 8; H = 5120, I = 2880, MXFP8: 1.0 at 2, 0.98 at 3); with both it is never ahead. Items of 32 rows lose
-// already at a walked / held of up to 1.35 from 18 items per CU on (H = 1664, I = 4096, 256 experts: 1.30, 39 items
-// per CU, mean 5 439 / 446, 8 456 / 490). (`ext`: biases, clamped SwiGLU or interleaved rows.)
+// its epilogue). Weights that are streamed again cost more than is gained there beyond a mean of 1. us, streaming /
+// few-rows, plain epilogues: 3072 x 3072, 128 experts, top-4 (walked / held 1.08, 18 items per CU): mean 1 188 / 190, 4
+// 282 / 295, 8 299 / 321; H = I = 2048, 256 experts, top-8 (1.13, 24): mean 2 223 / 222, 4 261 / 269, 8 276 / 298. On the
+// line's other side: H = 2944, I = 2304, 128 experts (1.26, 15): mean 4 228 / 219; 4096 x 4096, 64 experts (1.06, 12
+// items per CU): mean 4 278 / 265, 8 289 / 284. With biases / clamped SwiGLU or MXFP8 rows the streaming kernel has more to do
+// beside the weights: only from 18 items per CU on, and up to a mean of 3 / 2 (4096 x 4096, 128 experts, biases: 1.02
+// times as fast at 3, 0.98 at 4, 0.95 at 8; 3072 x 3072, MXFP8: 2 241 / 239, 3 270 / 274, 4 286 / 295); with both it is
+// never ahead. Items of 32 rows lose already at a walked / held of up to 1.35 from 18 items per CU on (H = 1664,
+// I = 4096, 256 experts: 1.30, 39 items per CU, mean 5 439 / 446, 8 456 / 490). (`ext`: biases, clamped SwiGLU or
+// interleaved rows.)
 constexpr int kFewMaxMean16 = 4, kFewMaxMean32 = 8;
 static int moe_few_rows(int T, int H, int I, int E, int k, bool a8, bool ext) {
     const long long S = (long long)T * k;
