@@ -9,6 +9,7 @@ values are clamped to +-448 first.
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 
@@ -40,10 +41,18 @@ def _quantize_fp8_per_tensor_gpu(x: torch.Tensor):
     return q, scale.item()
 
 
+def _is_plain(x: torch.Tensor) -> bool:
+    """Whether x is no more than its memory: a kernel launched on its address does not see what torch keeps beside
+    it (a subclass's dispatch, a tangent, a function transform's wrapper, a pending negation, a trace)."""
+    return type(x) in (torch.Tensor, torch.nn.Parameter) and not torch.compiler.is_compiling() \
+        and not torch._C._functorch.is_functorch_wrapped_tensor(x) and not x.requires_grad and not x.is_neg() \
+        and forward_ad.unpack_dual(x).tangent is None
+
+
 def quantize_fp8_per_tensor(x: torch.Tensor):
     """(e4m3 tensor, fp32 scale) with scale = amax/448 so that x ~= q.float() * scale."""
-    if x.device.type == "cuda" and x.dtype in _X_TYPES and x.numel() > 0 and x.is_contiguous() \
-            and x.data_ptr() % 16 == 0 and not x.requires_grad:
+    if x.device.type == "cuda" and x.dtype in _X_TYPES and _is_plain(x) and x.numel() > 0 and x.is_contiguous() \
+            and x.data_ptr() % 16 == 0:
         return _quantize_fp8_per_tensor_gpu(x)
     xf = x.float()
     amax = xf.abs().max()

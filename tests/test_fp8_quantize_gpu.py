@@ -92,3 +92,69 @@ def test_bad_arguments():
     assert lib.hk_fp8_quantize_tensor(a, 0, 0, a, a, a, 4096, None) == -2
     assert lib.hk_fp8_quantize_tensor(a + 2, 0, 16, a, a, a, 4096, None) == -3
     assert lib.hk_fp8_quantize_tensor(a, 0, 16, a, a, a, 4095, None) == -4
+
+
+class _Tagged(torch.Tensor):
+    pass
+
+
+def _carriers(x):
+    """Functions that quantize x as something more than its memory."""
+    from torch.autograd import forward_ad
+
+    import hipkittens_amd as hk
+
+    f = hk.quant.quantize_fp8_per_tensor
+    dx = torch.linspace(-1, 1, x.numel(), device=x.device).reshape(x.shape).to(x.dtype)
+
+    def dual():
+        with forward_ad.dual_level():
+            q, s = f(forward_ad.make_dual(x, dx))
+            primal, tangent = forward_ad.unpack_dual(q)
+            return primal.float() * s, tangent.float()
+
+    def jvp():
+        return torch.func.jvp(lambda v: f(v)[0].float(), (x,), (dx,))
+
+    def subclass():
+        q, s = f(x.as_subclass(_Tagged))
+        assert type(q) is _Tagged
+        return (q.as_subclass(torch.Tensor).float() * s,)
+
+    def negated():
+        q, s = f(torch._neg_view(x))
+        return (q.float() * s,)
+
+    def compiled():
+        q, s = torch.compile(f, backend="eager")(x)
+        return (q.float() * s,)
+
+    return [dual, jvp, subclass, negated, compiled]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("i", range(5))
+def test_tensors_that_are_more_than_their_memory(hk, i):
+    x = torch.randn(48, 64, generator=torch.Generator().manual_seed(3)).cuda()
+    got, want = _carriers(x)[i](), _carriers(x.cpu())[i]()
+    for a, b in zip(got, want):
+        assert torch.equal(a.cpu(), b)
+
+
+def test_what_counts_as_plain():
+    from torch.autograd import forward_ad
+
+    from hipkittens_amd.quant import _is_plain
+
+    x = torch.randn(4, 4)
+    assert _is_plain(x) and _is_plain(x[1:]) and _is_plain(torch.nn.Parameter(x, requires_grad=False))
+    assert not _is_plain(x.clone().requires_grad_()) and not _is_plain(x.as_subclass(_Tagged))
+    assert not _is_plain(torch._neg_view(x))
+    seen = []
+    torch.func.jvp(lambda v: (seen.append(_is_plain(v)), v)[1], (x,), (x,))
+    torch.func.grad(lambda v: (seen.append(_is_plain(v)), v.sum())[1])(x)
+    torch.vmap(lambda v: (seen.append(_is_plain(v)), v)[1])(x)
+    with forward_ad.dual_level():
+        seen.append(_is_plain(forward_ad.make_dual(x, x)))
+        assert _is_plain(x)
+    assert seen == [False] * 4
