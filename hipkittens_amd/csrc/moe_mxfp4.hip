@@ -1385,15 +1385,13 @@ namespace hk {
 // chunk are issued together; KU == 0: any k, one row at a time. Same operations in the same order.
 // The rows of o are read exactly once: non-temporal loads (213 -> 187 us at T = 8192, k = 8,
 // H = 7168, i.e. 5.7 TB/s; the GPT-OSS-like layer 10 us less).
-// Below kUnpermuteSplitTokens tokens a token's columns are shared among one-wave workgroups of one column chunk per
-// lane (gridDim.y): with a workgroup per token most CUs have nothing to do, and its 256 threads go over the
-// columns two (H = 2880) to four times (7168) in turn. Layer times, a workgroup per token / shared: 4 tokens,
-// H = 2880, k = 4 50.9 / 50.4 us (the kernel itself 3.9 us now); 16 tokens, H = 7168, k = 8 673.3 / 670.8 (4.6 us).
-// The kernel back to back: 4 tokens, H = 2880 2.4 / 2.1 us; H = 7168, k = 8: 16 tokens 4.7 / 2.5, 128 6.0 / 3.4,
-// 255 7.0 / 5.1; from 256 on there is a workgroup for every CU either way (not measured split).
+// While there are fewer tokens than CUs, a token's columns are shared among one-wave workgroups of one column chunk per
+// lane (gridDim.y): with a workgroup per token CUs have nothing to do, and its 256 threads go over the columns
+// two (H = 2880) to four times (7168) in turn. The kernel back to back, us, a workgroup per token / shared: 4 tokens,
+// H = 2880, k = 4 2.4 / 2.1; H = 7168, k = 8: 16 tokens 4.7 / 2.5, 128 6.0 / 3.4, 255 7.0 / 5.1 (whole layers gain
+// less than their timings differ by). From 256 on there is a workgroup for every CU either way (not measured split).
 // o has T * k rows; a position outside [0, T * k) (a caller's broken slot_to_pos) is not read and adds
 // nothing, like an expert id out of range in the sort.
-constexpr int kUnpermuteSplitTokens = 256;   // a workgroup for every CU
 template <int KU>
 __global__ __launch_bounds__(256) void moe_unpermute_kernel(const uint16_t* __restrict__ o,
                                                             const float* __restrict__ w,
@@ -1554,7 +1552,7 @@ extern "C" int hk_moe_unpermute_add(const void* o_bf16, const float* w, const in
     if (T <= 0 || k <= 0 || H <= 0 || (H % 8) != 0) return HK_ERR_BAD_SHAPE;
     if (((uintptr_t)o_bf16 | (uintptr_t)y_bf16 | (uintptr_t)add_bf16_or_null) & 15u) return HK_ERR_BAD_ALIGNMENT;
     auto kern = k <= 4 ? moe_unpermute_kernel<4> : k <= 8 ? moe_unpermute_kernel<8> : moe_unpermute_kernel<0>;
-    const bool split = T < kUnpermuteSplitTokens;
+    const bool split = T < moe_num_compute_units();
     const dim3 grid(T, split ? min((H / 8 + 63) / 64, 65535) : 1);
     hipLaunchKernelGGL(kern, grid, dim3(split ? 64 : 256), 0, (hipStream_t)stream, (const uint16_t*)o_bf16,
                        w, slot_to_pos, T, k, H, (const uint16_t*)add_bf16_or_null, (uint16_t*)y_bf16);
