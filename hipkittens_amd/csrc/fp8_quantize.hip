@@ -169,8 +169,10 @@ static int launch_fp8_tensor_quantize(const void* x, long long n, void* q, uint3
 }
 
 // Returns once *word differs from `unset`. The watched store is the first thing a kernel that was just launched
-// does, so this polls (a store to host memory is seen 2-3 us earlier than the end of the kernel through
-// hipStreamSynchronize) and hands over to hipStreamSynchronize when the stream has more than that to do first.
+// does, so this polls (on an idle stream a store to host memory is seen 2-3 us earlier than the end of the kernel through
+// hipStreamSynchronize) and hands over to hipStreamSynchronize when the stream has 20 ms and more to do first. The poll
+// keeps its core busy, and so does the runtime's own wait: behind 10 ms of queued GEMMs this, hipStreamSynchronize and
+// torch's copy of a scalar to the host each take 10.3 ms of CPU time.
 static int await_host_word(const volatile uint32_t* word, uint32_t unset, hipStream_t s) {
     const auto until = std::chrono::steady_clock::now() + std::chrono::milliseconds(20);
     for (;;) {
