@@ -1598,27 +1598,31 @@ extern "C" int hk_moe_mxfp4_preshuffle(const void* w, const void* scales, int sc
 // more rows than an item streams its weights again: one fragment of 16 rows up to a mean of 4, two up to 8 (MXFP4
 // activations only: MXFP8 rows are twice the traffic).
 // The exception is a layer that the streaming kernel runs at full rate: many items per CU (its last round is a small
-// part), and little of what it walks besides weights (an item takes K-steps in groups of four, and about one more for
-// its epilogue). Weights that are streamed again cost more than is gained there beyond a mean of 1. us, streaming /
-// few-rows, plain epilogues: 3072 x 3072, 128 experts, top-4 (walked / held 1.08, 18 items per CU): mean 1 188 / 190, 4
-// 282 / 295, 8 299 / 321; H = I = 2048, 256 experts, top-8 (1.13, 24): mean 2 223 / 222, 4 261 / 269, 8 276 / 298. On the
-// line's other side: H = 2944, I = 2304, 128 experts (1.26, 15): mean 4 228 / 219; 4096 x 4096, 64 experts (1.06, 12
-// items per CU): mean 4 278 / 265, 8 289 / 284. With biases / clamped SwiGLU or MXFP8 rows the streaming kernel has more to do
-// beside the weights: only from 18 items per CU on, and up to a mean of 3 / 2 (4096 x 4096, 128 experts, biases: 1.02
-// times as fast at 3, 0.98 at 4, 0.95 at 8; 3072 x 3072, MXFP8: 2 241 / 239, 3 270 / 274, 4 286 / 295); with both it is
-// never ahead. Items of 32 rows lose already at a walked / held of up to 1.35 from 18 items per CU on (H = 1664,
-// I = 4096, 256 experts: 1.30, 39 items per CU, mean 5 439 / 446, 8 456 / 490). (`ext`: biases, clamped SwiGLU or
-// interleaved rows.)
+// part), and little that it walks beside weights (`spare`: an item takes K-steps in groups of four, and about one more
+// for its epilogue). Weights that are streamed again then cost more than the few-rows kernel gains. The lines lie between
+// layers timed on both, us, streaming / few-rows, with spare and items per CU:
+//   - tight, plain epilogues (a mean of 1 at most): 3072 x 3072, 128 experts (0.08, 18) mean 1 188 / 190, 4 282 / 295;
+//     2048 x 2048, 256 experts (0.13, 24) mean 2 223 / 222, 4 261 / 269; H = 2880, I = 3392, 256 experts (0.24, 39) mean 2
+//     495 / 502, 4 578 / 602. Not: 2880 x 2880, 128 experts (0.20, 17.5) mean 1.2 196 / 187, 2.5 242 / 237, 4 258 / 257;
+//   - tight with biases / clamped SwiGLU or MXFP8 rows, for which the streaming kernel has more to do (2): H = 4928,
+//     I = 3840, biases (0.12, 25) mean 3 526 / 540, 8 594 / 622; 3072 x 3072, MXFP8 mean 2 241 / 239, 3 270 / 274, 4 286 /
+//     295. Not: H = 4096, I = 2752, biases (0.13, 19) mean 4 378 / 361. With both the streaming kernel is never ahead;
+//   - items of 32 rows, plain epilogues: 2880 x 2880 mean 5 275 / 277, 8 287 / 298; H = 2688, I = 1664, 256 experts (0.31,
+//     24) mean 8 315 / 331. Not: 4096 x 4096, 64 experts (0.06, 12) mean 8 289 / 284; H = 2496, I = 2688 (0.31, 15.5) mean
+//     5 229 / 221.
+// (`ext`: biases, clamped SwiGLU or interleaved rows.)
 constexpr int kFewMaxMean16 = 4, kFewMaxMean32 = 8;
 static int moe_few_rows(int T, int H, int I, int E, int k, bool a8, bool ext) {
     const long long S = (long long)T * k;
     auto up = [](long long x, int m) { return (x + m - 1) / m; };
-    const long long n1 = up(I, 128), n2 = up(H, 256), items = E * (n1 + n2), cus = moe_num_compute_units();
-    // K-steps walked against those that hold weights, H I / (128 * 256) + H I / 256^2
-    const double ratio = (double)(n1 * (4 * up(H, 1024) + 1) + n2 * (4 * up(I, 1024) + 1)) / (3.0 * H * I / 65536);
-    if (ratio < 1.25 && items >= (a8 || ext ? 18 : 13) * cus && !(a8 && ext)) return S <= (a8 ? 2ll : ext ? 3ll : 1ll) * E ? 16 : 0;
-    if (S <= (long long)kFewMaxMean16 * E) return 16;
-    return S <= (long long)kFewMaxMean32 * E && !a8 && !(ratio < 1.35 && items >= 18 * cus) ? 32 : 0;
+    const long long n1 = up(I, 128), n2 = up(H, 256);
+    const double per_cu = (double)E * (n1 + n2) / moe_num_compute_units();
+    // K-steps walked over those that hold weights (H I / (128 * 256) + H I / 256^2)
+    const double spare = (n1 * (4 * up(H, 1024) + 1) + n2 * (4 * up(I, 1024) + 1)) / (3.0 * H * I / 65536) - 1.0;
+    const bool tight = spare < 0.015 * (per_cu - 12) && !(a8 && ext);
+    if (S <= (long long)(!tight ? kFewMaxMean16 : a8 || ext ? 2 : 1) * E) return 16;
+    const bool no32 = a8 || tight || (!ext && spare < 0.025 * (per_cu - 9.5));
+    return S <= (long long)kFewMaxMean32 * E && !no32 ? 32 : 0;
 }
 
 // Workspace layout of hk_moe_mxfp4_forward (all regions 256-byte aligned). No region shrinks when T grows: a workspace

@@ -13,13 +13,17 @@ lib = hipkittens_amd.load_library()
     (2880, 2880, 32, 4, 65, 0, 0, 0), (2880, 2880, 32, 4, 32, 1, 0, 16), (2880, 2880, 32, 4, 33, 1, 0, 0),
     # layers that the streaming kernel runs at full rate (3 to 7 % slower on the few-rows kernel from a mean of 4 on)
     (3072, 3072, 128, 4, 32, 0, 0, 16), (3072, 3072, 128, 4, 33, 0, 0, 0), (3072, 3072, 128, 4, 256, 0, 0, 0),
-    (3072, 3072, 128, 4, 96, 0, 1, 16), (3072, 3072, 128, 4, 97, 0, 1, 0), (3072, 3072, 128, 4, 64, 1, 0, 16), (3072, 3072, 128, 4, 65, 1, 0, 0),
-    (3072, 3072, 128, 4, 128, 1, 1, 16), (4096, 4096, 128, 8, 128, 0, 0, 0), (2048, 2048, 256, 8, 256, 0, 0, 0),
-    (2624, 2048, 256, 8, 256, 0, 0, 0), (2880, 2880, 128, 4, 256, 0, 0, 0), (7168, 2048, 128, 8, 64, 0, 0, 0),
-    (1664, 4096, 256, 8, 128, 0, 0, 16), (1664, 4096, 256, 8, 129, 0, 0, 0), (1664, 4096, 256, 8, 256, 0, 1, 0),
+    (3072, 3072, 128, 4, 64, 0, 1, 16), (3072, 3072, 128, 4, 65, 0, 1, 0), (3072, 3072, 128, 4, 64, 1, 0, 16),
+    (3072, 3072, 128, 4, 65, 1, 0, 0), (3072, 3072, 128, 4, 128, 1, 1, 16), (4096, 4096, 128, 8, 128, 0, 0, 0),
+    (2048, 2048, 256, 8, 256, 0, 0, 0), (7168, 2048, 128, 8, 64, 0, 0, 0), (2880, 3392, 256, 8, 128, 0, 0, 0),
+    (4928, 3840, 128, 8, 128, 0, 1, 0),
+    # those that it runs a little below that: no items of 32 rows
+    (2880, 2880, 128, 4, 128, 0, 0, 16), (2880, 2880, 128, 4, 129, 0, 0, 0), (2624, 2048, 256, 8, 256, 0, 0, 0),
+    (1664, 4096, 256, 8, 256, 0, 0, 0), (1664, 4096, 256, 8, 256, 0, 1, 0),
     # fewer items per CU, the longer epilogues, or many K-steps walked without weights
-    (3072, 3072, 64, 4, 128, 0, 0, 32), (2880, 2880, 128, 4, 256, 0, 1, 32), (4096, 2048, 128, 8, 64, 0, 1, 16),
-    (2944, 2304, 128, 8, 64, 0, 0, 16), (2112, 3776, 128, 8, 128, 0, 0, 32), (1984, 1216, 256, 8, 256, 0, 1, 32)])
+    (4096, 4096, 64, 4, 128, 0, 0, 32), (4096, 2752, 128, 8, 64, 0, 1, 16), (2880, 2880, 128, 4, 256, 0, 1, 32), (4096, 2048, 128, 8, 64, 0, 1, 16),
+    (2944, 2304, 128, 8, 64, 0, 0, 16), (3456, 2880, 128, 8, 67, 0, 1, 32), (2688, 1664, 256, 8, 160, 0, 1, 32),
+    (2688, 1664, 256, 8, 160, 0, 0, 0), (2112, 3776, 128, 8, 128, 0, 0, 32), (1984, 1216, 256, 8, 256, 0, 1, 32)])
 def test_mxfp4(H, I, E, k, T, mxfp8, ext, rows):
     assert lib.hk_moe_mxfp4_few_rows(T, H, I, E, k, mxfp8, ext) == rows
 
