@@ -50,6 +50,9 @@ MXFP4 = [
 @pytest.mark.parametrize("T,E,k,H,I,hot", MXFP4)
 def test_moe_mxfp4_few_rows(hk, T, E, k, H, I, hot, act, ext):
     print(f"moe_mxfp4 few rows T={T} E={E} k={k} H={H} I={I} hot={hot} {act} ext={ext}", flush=True)
+    # MXFP8 layers with a mean above 4 rows take the streaming kernel
+    rows = 16 if T * k <= 4 * E else 0 if act == "mxfp8" else 32
+    assert hk.load_library().hk_moe_mxfp4_few_rows(T, H, I, E, k, act == "mxfp8", ext) == rows
     rng = np.random.default_rng(T + E + H + I)
     x = _bf16(rng.standard_normal((T, H)))
     logits = _logits(rng, T, E, hot)

@@ -23,15 +23,21 @@ def _layer(hk, T, E, H, I, seed):
 
 
 # K-steps of gate+up = H / 128, of down = I / 128: fewer than, as many as and more than the ring's seven; an odd
-# number of 128-column blocks of H; experts with 15 to 17 rows and more; the rule's edges (2 rows per expert and one
-# slot more; 3/4 of an item per CU and one m-tile more on 256 CUs)
+# number of 128-column blocks of H; experts with 15 to 17 rows and more; the rule's edges on 256 CUs, each followed by a
+# layer beyond it that takes the streaming kernel (2 rows per expert; 3/4 of an item per CU; 192 rows per expert)
+STREAMING = {(129, 64, 1, 256, 2048), (320, 2, 1, 256, 1152), (385, 2, 1, 256, 896)}
+
+
 @pytest.mark.parametrize("T,E,k,H,I", [(1, 8, 8, 128, 128), (3, 16, 4, 768, 896), (16, 64, 8, 896, 1024),
                                        (33, 16, 1, 1024, 128), (15, 2, 1, 1152, 256), (32, 2, 1, 256, 384),
                                        (34, 2, 2, 384, 640), (380, 2, 1, 256, 896), (384, 2, 1, 256, 896),
-                                       (128, 64, 1, 256, 2048), (129, 64, 1, 256, 2048)])
+                                       (385, 2, 1, 256, 896), (319, 2, 1, 256, 1152), (320, 2, 1, 256, 1152),
+                                       (128, 64, 1, 256, 2048), (129, 64, 1, 256, 2048),
+                                       (20, 16, 4, 640, 512), (20, 16, 4, 512, 640)])   # rings of four and seven K-steps
 def test_routed_layer_has_the_bits_of_the_plain_layout(hk, T, E, k, H, I):
     print(f"fp8blk few T={T} E={E} k={k} H={H} I={I}", flush=True)
     tk = hk.tk_kernel
+    assert hk.load_library().hk_moe_fp8blk_few_rows(T, H, I, E, k) == (0 if (T, E, k, H, I) in STREAMING else 16)
     xq, xs, logits, plain = _layer(hk, T, E, H, I, T + E + H)
     ws = torch.empty(tk.moe_fp8blk_workspace_bytes(T, H, I, E, k), dtype=torch.uint8, device=DEV)
     out = []
@@ -50,6 +56,8 @@ def test_routed_layer_has_the_bits_of_the_plain_layout(hk, T, E, k, H, I):
 def test_shared_expert_has_the_bits_of_the_plain_layout_and_of_the_routed_call(hk, T, H, I):
     print(f"fp8blk shared T={T} H={H} I={I}", flush=True)
     tk = hk.tk_kernel
+    # few rows up to 3/4 of an item per CU (I = 1920: 191 tokens) and 192 rows
+    assert hk.load_library().hk_moe_fp8blk_few_rows(T, H, I, 1, 1) == (16 if T < 192 else 0)
     xq, xs, _, plain = _layer(hk, T, 1, H, I, T + H)
     ws = torch.empty(tk.moe_fp8blk_workspace_bytes(T, H, I, 1, 1), dtype=torch.uint8, device=DEV)
     shuffled = (tk.MoeFp8BlkShuffledWeights.from_plain(*plain), None, None, None)
