@@ -93,7 +93,7 @@ int hk_fp8_gemm_static_ws(const void* A_e4m3, const void* B_e4m3, void* C_bf16, 
  * hand-interleaved schedule over a five-slot LDS ring with the loads spread over the whole K-step
  * (what hk_fp8_gemm picks for large problems: the tile with the smallest estimated time, see
  * hk_gemm_tile_choice), 5 = 128x128x128 tile, 4
- * waves, plain loop over three LDS stages (picked for smaller problems), 6 = the same loop with
+ * waves, four LDS stages, loads and LDS reads between the MFMAs (picked for smaller problems), 6 = the same loop with
  * 64x64 tiles and four stages, two workgroups per CU (picked for the smallest), 7 = 192x256x128
  * tile, sixteen waves: four producers that only issue the
  * global->LDS loads and twelve consumers that only multiply (the wave-specialised structure of the
@@ -190,7 +190,7 @@ int hk_bf16_gemm_ws(const void* A_bf16, const void* B_bf16, void* C_bf16, int M,
 
 /* Same contract on a chosen kernel: 0 = portable kernel (any shape), 1 = 256x256x64 tile kernel
  * (the FP8 ring schedule; the last K-step of a K that is not a multiple of 64 is zero-filled),
- * 2 = 128x128 tiles / three LDS stages, 3 = 64x64 tiles / four stages (the FP8 GEMM's small-tile
+ * 2 = 128x128 tiles / four LDS stages, 3 = 64x64 tiles / four stages (the FP8 GEMM's small-tile
  * kernels with the bf16 MFMA; hk_bf16_gemm picks them by tile count as hk_fp8_gemm does), 4 = 256x256x64
  * tile kernel with the reference's 8-wave ping-pong schedule
  * (kernels/gemm/bf16fp32/mi325x/256_256_64_16.cpp:73-155), 5 = 192x256x64 tile producer / consumer kernel
@@ -388,8 +388,8 @@ int hk_moe_fp8blk_forward(const void* x_e4m3, const float* x_scales, const float
 
 /* The two entry points above with a residual y_add [T, H] bf16 (or NULL) that is added, in fp32,
  * to the weighted sum of the routed experts before the single bf16 rounding: the DeepSeek-V3
- * shared expert. Its output is computed with hk_moe_fp8blk_experts on trivial routing (E = 1,
- * k = 1, weight 1, identity order), then passed here. y_add may alias y_bf16. */
+ * shared expert. Its output is computed with hk_moe_fp8blk_shared_expert, then passed here.
+ * y_add may alias y_bf16. */
 int hk_moe_fp8blk_experts_ex(const void* x_e4m3, const float* x_scales, const void* w13,
                              const float* w13_scales, const void* w2, const float* w2_scales,
                              const float* topk_w, const int32_t* sorted_slots,
