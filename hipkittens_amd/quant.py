@@ -12,6 +12,7 @@ import torch
 from torch.autograd import forward_ad
 
 from . import _lib
+from .tk_kernel import _stream
 
 E4M3_MAX = 448.0
 
@@ -36,7 +37,7 @@ def _quantize_fp8_per_tensor_gpu(x: torch.Tensor):
     ws = torch.empty(_WS_BYTES, dtype=torch.uint8, device=dev)
     scale = torch.empty(1, dtype=torch.float32, pin_memory=True)
     st = lib.hk_fp8_quantize_tensor(x.data_ptr(), _X_TYPES[x.dtype], x.numel(), q.data_ptr(), scale.data_ptr(),
-                                    ws.data_ptr(), _WS_BYTES, torch.cuda.current_stream(dev).cuda_stream)
+                                    ws.data_ptr(), _WS_BYTES, _stream(x))
     _lib.check(st, "quantize_fp8_per_tensor")
     return q, scale.item()
 
@@ -46,7 +47,7 @@ def _is_plain(x: torch.Tensor) -> bool:
     it (a subclass's dispatch, a tangent, a function transform's wrapper, a pending negation, a trace)."""
     return type(x) in (torch.Tensor, torch.nn.Parameter) and not torch.compiler.is_compiling() \
         and not torch._C._functorch.is_functorch_wrapped_tensor(x) and not x.requires_grad and not x.is_neg() \
-        and forward_ad.unpack_dual(x).tangent is None
+        and (forward_ad._current_level < 0 or forward_ad.unpack_dual(x).tangent is None)   # (no level, no duals)
 
 
 def quantize_fp8_per_tensor(x: torch.Tensor):
