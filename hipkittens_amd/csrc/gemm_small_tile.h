@@ -352,7 +352,7 @@ static __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* 
 //     wins by 4-12 % from a K of about 4096 elements on), 64 tiles of 256 are one round of four times the work
 //     of the single round of 256 small tiles (the small tile wins by 60 %). Measured against the best of the
 //     three kernels, every launch on another copy of B (a model's weights come from HBM, not from the memory-side
-//     cache), the rule alone is more than 5 % behind on 7 / 5 of 414 shapes (FP8 / BF16; 42 / 40 with the constants
+//     cache), the rule alone is more than 5 % behind on 7 / 6 of 414 shapes (FP8 / BF16; 42 / 40 with the constants
 //     that fitted these kernels before their loads and LDS reads were spread over the MFMAs) and on 20 of 360 (MXFP4),
 //     mostly by 5 to 10 % where a long B is read by several rows of small tiles;
 //  2. a generated table of the shapes on which a sweep found the rule's choice more than a few percent behind
