@@ -13,6 +13,7 @@ SIGNATURES = {
     "hk_status_string": (ctypes.c_char_p, [c_int]),
     "hk_version": (c_int, []),
     "hk_gemm_tile_choice": (c_int, [c_int] * 5),
+    "hk_gemm_shorter_tile": (c_int, [c_int] * 4),
     "hk_moe_mxfp4_few_rows": (c_int, [c_int] * 7),
     "hk_moe_fp8blk_few_rows": (c_int, [c_int] * 5),
     "hk_fp8_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_void_p]),

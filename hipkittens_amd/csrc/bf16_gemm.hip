@@ -28,6 +28,7 @@ __device__ __forceinline__ void mfma_bf16_16x16x32_acc(v4f& acc, const v4i& x, c
 struct Bf16RingMma {
     struct Frag { v4i lo, hi; };  // K elements 8 g .. +8 and 32 + 8 g .. +8 of the lane's row
     static constexpr int kPasses = 2;
+    static constexpr bool kScaled = false;
     static __device__ __forceinline__ Frag load(uint32_t lo, uint32_t hi, int imm) {
         Frag f;
         f.lo = *(lds_v4i_t*)(uintptr_t)(lo + imm);
@@ -44,12 +45,12 @@ struct Bf16RingMma {
 // STREAM_C: C is stored with the non-temporal hint; the host asks for it for large outputs of whole tiles while the
 // operands fit the memory-side cache (launch_bf16_ring has the rule and the measurements; 8192^3: 1577 -> 1593
 // TFLOP/s on one box, 1541 -> 1558 on another). (FP8 and MXFP4 at 8192^3: -1.0 / -1.5 %.)
-template <bool EDGE, bool STREAM_C = false>
+template <bool EDGE, bool STREAM_C = false, int TILE_M = BM, int TILE_N = BN>
 __global__ __launch_bounds__(256) void bf16_gemm_4wave_ring_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, uint16_t* __restrict__ C,
     int M, int N, int K, float alpha, int tiles_m, int tiles_n, int band_n) {
     extern __shared__ __attribute__((aligned(2048))) uint8_t smem[];
-    gemm_ring_body<Bf16RingMma, EDGE, STREAM_C>(smem, A, B, C, M, N, 2 * K, alpha, tiles_m, tiles_n, band_n);
+    gemm_ring_body<Bf16RingMma, EDGE, STREAM_C, TILE_M, TILE_N>(smem, A, B, C, M, N, 2 * K, alpha, tiles_m, tiles_n, band_n);
 }
 
 
@@ -206,39 +207,39 @@ static int launch_bf16_splitk(const void* A, const void* B, void* C, int M, int 
                                     B, C, M, N, 2 * K, 1.0f, splits, partial, stream);
 }
 
-template <bool EDGE, bool STREAM_C>
-static int launch_bf16_ring_kernel(const void* A, const void* B, void* C, int M, int N, int K, int band_n,
-                                  hipStream_t stream) {
-    auto kern = bf16_gemm_4wave_ring_kernel<EDGE, STREAM_C>;
-    constexpr int lds_bytes = 5 * kTileBytes;
-    static DeviceOnce configured;
-    if (!set_lds_limit_once((const void*)kern, lds_bytes, configured)) return HK_ERR_LAUNCH;
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+template <bool STREAM_C, int TILE_M = BM, int TILE_N = BN>
+static int launch_bf16_ring_kernel(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream) {
+    const bool edge = (M % TILE_M) != 0 || (N % TILE_N) != 0;
+    auto kern = edge ? bf16_gemm_4wave_ring_kernel<true, false, TILE_M, TILE_N>
+                     : bf16_gemm_4wave_ring_kernel<false, STREAM_C, TILE_M, TILE_N>;
+    constexpr int lds_bytes = ring_lds_bytes(TILE_M, TILE_N, false);
+    static DeviceOnce configured[2];
+    if (!set_lds_limit_once((const void*)kern, lds_bytes, configured[edge])) return HK_ERR_LAUNCH;
+    const int tiles_m = (M + TILE_M - 1) / TILE_M, tiles_n = (N + TILE_N - 1) / TILE_N;
     hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(256), lds_bytes, stream, (const uint8_t*)A,
-                       (const uint8_t*)B, (uint16_t*)C, M, N, K, 1.0f, tiles_m, tiles_n, band_n);
+                       (const uint8_t*)B, (uint16_t*)C, M, N, K, 1.0f, tiles_m, tiles_n,
+                       raster_band(((long long)M + N) * K * 2, tiles_n));
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
-template <bool EDGE>
 static int launch_bf16_ring(const void* A, const void* B, void* C, int M, int N, int K, hipStream_t stream) {
     const int tiles_n = (N + BN - 1) / BN;
-    const int band_n = raster_band(((long long)M + N) * K * 2, tiles_n);
     // whole tiles, operands that fit the memory-side cache (no bands) and a C of 96 MB or more: C goes out with the
     // non-temporal hint (8192^3: +0.7 to 1.2 %; 4096^3, a C of 32 MB: -1.2 %; 16384^3, banded: -0.75 %)
-    if constexpr (!EDGE)
-        if (band_n >= tiles_n && (long long)M * N * 2 >= (96ll << 20))
-            return launch_bf16_ring_kernel<false, true>(A, B, C, M, N, K, band_n, stream);
-    return launch_bf16_ring_kernel<EDGE, false>(A, B, C, M, N, K, band_n, stream);
+    if ((M % BM) == 0 && (N % BN) == 0 && raster_band(((long long)M + N) * K * 2, tiles_n) >= tiles_n &&
+        (long long)M * N * 2 >= (96ll << 20))
+        return launch_bf16_ring_kernel<true>(A, B, C, M, N, K, stream);
+    return launch_bf16_ring_kernel<false>(A, B, C, M, N, K, stream);
 }
 
 }  // namespace hk
 
-extern "C" int hk_bf16_gemm_variant(const void* A, const void* B, void* C, int M, int N, int K, int variant,
-                                    void* stream) {
+// variant: as hk_bf16_gemm_variant, or one of the ring kernel's shorter tiles (kVariant192x256, kVariant256x192).
+static int bf16_gemm_impl(const void* A, const void* B, void* C, int M, int N, int K, int variant, void* stream) {
     using namespace hk;
     if (!A || !B || !C) return HK_ERR_NULL_POINTER;
     if (M <= 0 || N <= 0 || K <= 0 || (K % 8) != 0 || gemm_dims_too_large(M, N, K)) return HK_ERR_BAD_SHAPE;
     if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15u) return HK_ERR_BAD_ALIGNMENT;
-    if (variant < 0 || variant > 6) return HK_ERR_UNSUPPORTED;
+    if (variant < 0) return HK_ERR_UNSUPPORTED;
     if (variant == 6 && M > kSkinnyMaxM) return HK_ERR_UNSUPPORTED;
     hipStream_t s = (hipStream_t)stream;
     if (variant == 0) {
@@ -264,10 +265,17 @@ extern "C" int hk_bf16_gemm_variant(const void* A, const void* B, void* C, int M
         const bool e = (M % kPcBM) != 0 || (N % BN) != 0;
         return e ? launch_bf16_prodcons<true>(A, B, C, M, N, K, s) : launch_bf16_prodcons<false>(A, B, C, M, N, K, s);
     }
-    const bool edge = (M % BM) != 0 || (N % BN) != 0;
     if (variant == 4)
-        return edge ? launch_bf16_pingpong<true>(A, B, C, M, N, K, s) : launch_bf16_pingpong<false>(A, B, C, M, N, K, s);
-    return edge ? launch_bf16_ring<true>(A, B, C, M, N, K, s) : launch_bf16_ring<false>(A, B, C, M, N, K, s);
+        return (M % BM) != 0 || (N % BN) != 0 ? launch_bf16_pingpong<true>(A, B, C, M, N, K, s)
+                                              : launch_bf16_pingpong<false>(A, B, C, M, N, K, s);
+    if (variant == kVariant192x256) return launch_bf16_ring_kernel<false, 192, 256>(A, B, C, M, N, K, s);
+    if (variant == kVariant256x192) return launch_bf16_ring_kernel<false, 256, 192>(A, B, C, M, N, K, s);
+    return launch_bf16_ring(A, B, C, M, N, K, s);
+}
+
+extern "C" int hk_bf16_gemm_variant(const void* A, const void* B, void* C, int M, int N, int K, int variant,
+                                    void* stream) {
+    return bf16_gemm_impl(A, B, C, M, N, K, variant > 6 ? -1 : variant, stream);
 }
 
 extern "C" int hk_bf16_gemm(const void* A, const void* B, void* C, int M, int N, int K, void* stream) {
@@ -277,8 +285,9 @@ extern "C" int hk_bf16_gemm(const void* A, const void* B, void* C, int M, int N,
     // the same choice of tile as hk_fp8_gemm (pick_tile), with this format's measured corrections
     const int tile = pick_tile(kFmtBf16, M, N, (int)((2ll * K + BK - 1) / BK), kTileRuleBf16);
     const bool skinny = tile_ok && use_skinny(M, N, (int)((2ll * K + BK - 1) / BK), false, moe_num_compute_units());
-    const int variant = !tile_ok ? 0 : skinny ? 6 : tile == kTinyTile ? 3 : tile == kSmallTile ? 2 : 1;
-    return hk_bf16_gemm_variant(A, B, C, M, N, K, variant, stream);
+    const int shorter = pick_shorter_tile(M, N, (int)((2ll * K + BK - 1) / BK), tile, kTileRuleBf16, kShorterTileBf16);
+    const int variant = !tile_ok ? 0 : skinny ? 6 : shorter ? shorter : tile == kTinyTile ? 3 : tile == kSmallTile ? 2 : 1;
+    return bf16_gemm_impl(A, B, C, M, N, K, variant, stream);
 }
 
 extern "C" size_t hk_bf16_gemm_workspace_bytes(int M, int N, int K) {

@@ -27,6 +27,7 @@ namespace hk {
 struct Fp8RingMma {
     using Frag = v8i;
     static constexpr int kPasses = 1;
+    static constexpr bool kScaled = false;
     static __device__ __forceinline__ Frag load(uint32_t lo, uint32_t hi, int imm) { return lds_frag(lo, hi, imm); }
     template <int PASS>
     static __device__ __forceinline__ void mma(v4f& acc, const Frag& b, const Frag& a) {
@@ -34,12 +35,12 @@ struct Fp8RingMma {
     }
     static __device__ __forceinline__ int raster_group(int, int) { return 4; }
 };
-template <bool EDGE>
+template <bool EDGE, int TILE_M = BM, int TILE_N = BN>
 __global__ __launch_bounds__(256) void fp8_gemm_4wave_ring_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, uint16_t* __restrict__ C,
     int M, int N, int K, float alpha, int tiles_m, int tiles_n, int band_n) {
     extern __shared__ __attribute__((aligned(2048))) uint8_t smem[];
-    gemm_ring_body<Fp8RingMma, EDGE>(smem, A, B, C, M, N, K, alpha, tiles_m, tiles_n, band_n);
+    gemm_ring_body<Fp8RingMma, EDGE, false, TILE_M, TILE_N>(smem, A, B, C, M, N, K, alpha, tiles_m, tiles_n, band_n);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -193,14 +194,15 @@ static int launch_tile128_splitk(const void* A, const void* B, void* C, int M, i
                                     B, C, M, N, K, alpha, splits, partial, stream);
 }
 
-template <bool EDGE>
+template <int TILE_M = BM, int TILE_N = BN>
 static int launch_4wave(const void* A, const void* B, void* C, int M, int N, int K, float alpha,
                         hipStream_t stream) {
-    auto kern = fp8_gemm_4wave_ring_kernel<EDGE>;
-    constexpr int lds_bytes = 5 * kTileBytes;
-    static DeviceOnce configured;
-    if (!set_lds_limit_once((const void*)kern, lds_bytes, configured)) return HK_ERR_LAUNCH;
-    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const bool edge = (M % TILE_M) != 0 || (N % TILE_N) != 0;
+    auto kern = edge ? fp8_gemm_4wave_ring_kernel<true, TILE_M, TILE_N> : fp8_gemm_4wave_ring_kernel<false, TILE_M, TILE_N>;
+    constexpr int lds_bytes = ring_lds_bytes(TILE_M, TILE_N, false);
+    static DeviceOnce configured[2];
+    if (!set_lds_limit_once((const void*)kern, lds_bytes, configured[edge])) return HK_ERR_LAUNCH;
+    const int tiles_m = (M + TILE_M - 1) / TILE_M, tiles_n = (N + TILE_N - 1) / TILE_N;
     hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(256), lds_bytes, stream,
                        (const uint8_t*)A, (const uint8_t*)B, (uint16_t*)C, M, N, K, alpha, tiles_m,
                        tiles_n, raster_band(((long long)M + N) * K, tiles_n));
@@ -209,13 +211,14 @@ static int launch_4wave(const void* A, const void* B, void* C, int M, int N, int
 
 }  // namespace hk
 
-extern "C" int hk_fp8_gemm_variant(const void* A, const void* B, void* C, int M, int N, int K,
-                                   float scale_a, float scale_b, int variant, void* stream) {
+// variant: as hk_fp8_gemm_variant, or one of the ring kernel's shorter tiles (kVariant192x256, kVariant256x192).
+static int fp8_gemm_impl(const void* A, const void* B, void* C, int M, int N, int K, float scale_a, float scale_b,
+                         int variant, void* stream) {
     using namespace hk;
     if (!A || !B || !C) return HK_ERR_NULL_POINTER;
     if (M <= 0 || N <= 0 || K <= 0 || (K % 16) != 0 || gemm_dims_too_large(M, N, K)) return HK_ERR_BAD_SHAPE;
     if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15u) return HK_ERR_BAD_ALIGNMENT;
-    if (variant < 0 || variant > 8 || variant == 2 || variant == 3) return HK_ERR_UNSUPPORTED;
+    if (variant < 0 || variant == 2 || variant == 3) return HK_ERR_UNSUPPORTED;
     if (variant == 8 && M > kSkinnyMaxM) return HK_ERR_UNSUPPORTED;
     // K tails: the tile kernels zero-fill the last K-step of any K % 16 == 0
     if (variant != 0 && (long long)K * BM >= (1ll << 31)) return HK_ERR_BAD_SHAPE;
@@ -243,10 +246,17 @@ extern "C" int hk_fp8_gemm_variant(const void* A, const void* B, void* C, int M,
         const bool e = (M % kPcBM) != 0 || (N % BN) != 0;
         return e ? launch_prodcons<true>(A, B, C, M, N, K, alpha, s) : launch_prodcons<false>(A, B, C, M, N, K, alpha, s);
     }
-    const bool edge = (M % BM) != 0 || (N % BN) != 0;
     if (variant == 1)
-        return edge ? launch_pingpong<true>(A, B, C, M, N, K, alpha, s) : launch_pingpong<false>(A, B, C, M, N, K, alpha, s);
-    return edge ? launch_4wave<true>(A, B, C, M, N, K, alpha, s) : launch_4wave<false>(A, B, C, M, N, K, alpha, s);
+        return (M % BM) != 0 || (N % BN) != 0 ? launch_pingpong<true>(A, B, C, M, N, K, alpha, s)
+                                              : launch_pingpong<false>(A, B, C, M, N, K, alpha, s);
+    if (variant == kVariant192x256) return launch_4wave<192, 256>(A, B, C, M, N, K, alpha, s);
+    if (variant == kVariant256x192) return launch_4wave<256, 192>(A, B, C, M, N, K, alpha, s);
+    return launch_4wave(A, B, C, M, N, K, alpha, s);
+}
+
+extern "C" int hk_fp8_gemm_variant(const void* A, const void* B, void* C, int M, int N, int K,
+                                   float scale_a, float scale_b, int variant, void* stream) {
+    return fp8_gemm_impl(A, B, C, M, N, K, scale_a, scale_b, variant > 8 ? -1 : variant, stream);
 }
 
 extern "C" size_t hk_fp8_gemm_workspace_bytes(int M, int N, int K) {
@@ -334,6 +344,17 @@ extern "C" int hk_gemm_tile_choice(int format, int M, int N, int K, int consult_
     return pick_tile(format, M, N, nk, rule, consult_table != 0);
 }
 
+extern "C" int hk_gemm_shorter_tile(int format, int M, int N, int K) {
+    using namespace hk;
+    if (format < 0 || format > 2 || M <= 0 || N <= 0 || K <= 0 || gemm_dims_too_large(M, N, K)) return HK_ERR_BAD_SHAPE;
+    const long long row_bytes = format == kFmtFp8 ? K : format == kFmtBf16 ? 2ll * K : K / 2;
+    const int nk = (int)((row_bytes + BK - 1) / BK);
+    const TileRule rule = format == kFmtFp8 ? kTileRuleFp8 : format == kFmtBf16 ? kTileRuleBf16 : kTileRuleMxfp4;
+    const ShorterTileRule sr = format == kFmtFp8 ? kShorterTileFp8 : format == kFmtBf16 ? kShorterTileBf16 : kShorterTileMxfp4;
+    const int v = pick_shorter_tile(M, N, nk, pick_tile(format, M, N, nk, rule), rule, sr);
+    return v == kVariant192x256 ? 1 : v == kVariant256x192 ? 2 : 0;
+}
+
 extern "C" int hk_fp8_gemm(const void* A, const void* B, void* C, int M, int N, int K,
                            float scale_a, float scale_b, void* stream) {
     using namespace hk;
@@ -343,6 +364,7 @@ extern "C" int hk_fp8_gemm(const void* A, const void* B, void* C, int M, int N, 
     const int tile = pick_tile(kFmtFp8, M, N, (K + BK - 1) / BK, kTileRuleFp8);
     // few rows: one pass over B by the skinny kernel where that is faster (use_skinny)
     const bool skinny = tile_ok && use_skinny(M, N, (K + BK - 1) / BK, false, moe_num_compute_units());
-    const int variant = !tile_ok ? 0 : skinny ? 8 : tile == kTinyTile ? 6 : tile == kSmallTile ? 5 : 4;
-    return hk_fp8_gemm_variant(A, B, C, M, N, K, scale_a, scale_b, variant, stream);
+    const int shorter = pick_shorter_tile(M, N, (K + BK - 1) / BK, tile, kTileRuleFp8, kShorterTileFp8);
+    const int variant = !tile_ok ? 0 : skinny ? 8 : shorter ? shorter : tile == kTinyTile ? 6 : tile == kSmallTile ? 5 : 4;
+    return fp8_gemm_impl(A, B, C, M, N, K, scale_a, scale_b, variant, stream);
 }

@@ -401,6 +401,33 @@ constexpr TileRule kTileRuleFp8{{7.10f, 3.28f, 2.02f}, {1.060f, 0.533f, 0.385f}}
 constexpr TileRule kTileRuleBf16{{8.57f, 2.79f, 2.20f}, {0.983f, 0.495f, 0.336f}};
 constexpr TileRule kTileRuleMxfp4{{7.71f, 3.13f, 1.94f}, {1.316f, 0.767f, 0.549f}};
 
+// The ring kernel's shorter tiles (gemm_ring.h): 192x256 or 256x192 in the place of the tile that pick_tile names, where
+// the same cost model, one workgroup per CU, gives them less time. The constants, and the factor on the estimate for a
+// 128- or 64-tile (which is high where it is compared with these), are fitted to 91 shapes per format on an MI355X
+// (M 500 ... 8192, (N, K) 4096 x 4096 ... 14336 x 4096, 2880 x 2880, 10000 x 1024, copies of B in rotation): no shape
+// is more than 3 % behind what it had, and the geometric mean falls by 5.5 (FP8), 6.3 (BF16) and 6.3 % (MXFP4), of 6.5,
+// 6.9 and 7.0 that the best kernel for every shape would give. Examples, us before / after: BF16 3001 x 4096 x 4096
+// 90.1 / 74.9 (192 tiles of 256x256 against 256 of 192x256), 4096 x 2880 x 2880 69.2 / 54.1; FP8 8192 x 2880 x 2880
+// 71.8 / 58.6; MXFP4 4096 x 2880 x 2880 35.2 / 27.8; and not taken: BF16 4096 x 4096 x 4096 96.3 / 130.9 (256 tiles of
+// 256x256, one round; 352 of 192x256, two).
+constexpr int kVariant192x256 = 100, kVariant256x192 = 101;   // the GEMM entry points' internal numbers for them
+struct ShorterTileRule { float fixed, per_step, small; };
+constexpr ShorterTileRule kShorterTileFp8{5.7f, 0.87f, 0.82f}, kShorterTileBf16{5.6f, 0.925f, 0.94f}, kShorterTileMxfp4{7.3f, 1.29f, 1.0f};
+static inline int pick_shorter_tile(int M, int N, int nk, int tile, TileRule rule, ShorterTileRule shorter) {
+    const long long cus = moe_num_compute_units();
+    auto rounds = [&](int tm, int tn, long long capacity) {
+        const long long tiles = (((long long)M + tm - 1) / tm) * (((long long)N + tn - 1) / tn);
+        return (double)((tiles + capacity - 1) / capacity);
+    };
+    const int i = tile == kTinyTile ? 2 : tile == kSmallTile ? 1 : 0;
+    const double now = rounds(tile, tile, i == 2 ? 2 * cus : cus) * ((double)rule.fixed[i] + (double)rule.per_step[i] * nk) *
+                       (i == 0 ? 1.0 : (double)shorter.small);
+    const double one = (double)shorter.fixed + (double)shorter.per_step * nk;
+    const double t0 = rounds(192, 256, cus) * one, t1 = rounds(256, 192, cus) * one;
+    if ((t0 < t1 ? t0 : t1) > now) return 0;
+    return t0 < t1 ? kVariant192x256 : kVariant256x192;
+}
+
 // Number of K ranges the split-K path would use: as many as fill the CUs, each at least 4
 // K-steps long, at most 16; 1 = the problem has enough tiles or too short a K.
 // K: the operands' row length in bytes; min_nk: the shortest K (in K-steps) that is split.

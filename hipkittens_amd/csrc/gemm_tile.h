@@ -46,9 +46,13 @@ __device__ __forceinline__ Frag4 lds_frag4(uint32_t addr_lo, uint32_t addr_hi, i
 // STREAM: the full-tile stores carry the non-temporal hint (C is written once and not read by the kernel;
 // keeping it out of the L2 leaves that cache to the operand panels). Only the BF16 ring kernel has an
 // instantiation with it (bf16_gemm.hip has the measurements).
+// EDGE: a patch that lies inside C all the same (most of a ragged problem's) takes the plain stores.
 template <int MT, int NT, bool EDGE, bool STREAM = false>
 __device__ __forceinline__ void store_c_tile(const v4f (&acc)[MT][NT], uint16_t* __restrict__ C,
                                              int M, int N, int row_base, int col_base, float alpha) {
+    if constexpr (EDGE)
+        if (row_base + 16 * MT <= M && col_base + 16 * NT <= N && (N & 7) == 0)
+            return store_c_tile<MT, NT, false, STREAM>(acc, C, M, N, row_base, col_base, alpha);
     const int r = lane_id() & 15, g = lane_id() >> 4;
 #pragma unroll
     for (int m = 0; m < MT; ++m) {

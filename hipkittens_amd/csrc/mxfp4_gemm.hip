@@ -26,6 +26,7 @@
 // it are out of the descriptor's range for the last row (nothing is fetched, zeros land in LDS) and
 // belong to K blocks past K otherwise; the readers add the same shift to their LDS address.
 #include "gemm_tile.h"
+#include "gemm_ring.h"
 #include "gemm_small_tile.h"
 #include "gemm_pingpong.h"
 #include "gemm_prodcons.h"
@@ -49,6 +50,7 @@ __device__ __forceinline__ void mfma_fp4_acc(v4f& acc, const v4i& x, const v4i& 
         : "v"(x), "v"(y), "v"(sx), "v"(sy));
 }
 
+// (Rows past M or N: outside the descriptors, as in gemm_ring.h; EDGE is the epilogue's.)
 template <bool EDGE>
 __global__ __launch_bounds__(256) void mxfp4_gemm_4wave_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ SA, const uint8_t* __restrict__ B,
@@ -78,32 +80,17 @@ __global__ __launch_bounds__(256) void mxfp4_gemm_4wave_kernel(
     const v4i srd_sb = make_srd(SB + (size_t)col0 * sb_pitch, scale_rows_bytes(b_rows, sb_pitch, scale_row_bytes));
 
     // operand tiles: as in the FP8 kernel
-    uint32_t voff_a[EDGE ? NDMA : 1], voff_b[EDGE ? NDMA : 1];
-#pragma unroll
-    for (int i = 0; i < (EDGE ? NDMA : 1); ++i) {
-        const int R = 8 * (i * NW + w) + (lane >> 3);
-        const uint32_t c = swz_chunk(R, lane & 7);
-        int ra = R, rb = b_row_to_col(R);
-        if (EDGE) {
-            ra = min(ra, a_rows - 1);
-            rb = min(rb, b_rows - 1);
-        }
-        voff_a[i] = (uint32_t)ra * (uint32_t)Kb + c * 16u;
-        voff_b[i] = (uint32_t)rb * (uint32_t)Kb + c * 16u;
+    uint32_t voff_a, voff_b;
+    {
+        const int R = 8 * w + (lane >> 3);
+        const uint32_t c = swz_chunk(R, lane & 7) * 16u;
+        voff_a = (uint32_t)R * (uint32_t)Kb + c;
+        voff_b = (uint32_t)b_row_to_col(R) * (uint32_t)Kb + c;
     }
     // scale tiles: this wave loads LDS rows 64w..64w+63 of each operand, lane l -> row 64w + l,
     // 16 bytes = the row's scales of K-steps 2p and 2p+1
-    uint32_t voff_sa, voff_sb;
-    {
-        const int R = 64 * w + lane;
-        int ra = R, rb = b_row_to_col(R);
-        if (EDGE) {
-            ra = min(ra, a_rows - 1);
-            rb = min(rb, b_rows - 1);
-        }
-        voff_sa = (uint32_t)ra * (uint32_t)sa_pitch;
-        voff_sb = (uint32_t)rb * (uint32_t)sb_pitch;
-    }
+    const uint32_t voff_sa = (uint32_t)(64 * w + lane) * (uint32_t)sa_pitch;
+    const uint32_t voff_sb = (uint32_t)b_row_to_col(64 * w + lane) * (uint32_t)sb_pitch;
     const uint32_t dma_row_stride = to_sgpr((uint32_t)(8 * NW) * (uint32_t)Kb);
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
     const uint32_t lds_wave = to_sgpr(lds0 + (uint32_t)w * 1024u);
@@ -113,10 +100,7 @@ __global__ __launch_bounds__(256) void mxfp4_gemm_4wave_kernel(
     // 16 bytes lie past the end of the row: out of the buffer's range, so zeros land in LDS
     auto dma_one = [&](int op, int i, int stage, uint32_t k0, v4i srd, uint32_t vor) {
         const uint32_t dst = lds_wave + (uint32_t)stage * kStageBytes + op * kTileBytes + i * NW * 1024;
-        if (EDGE)
-            dma16(srd, dst, (op ? voff_b[i] : voff_a[i]) | vor, k0);
-        else
-            dma16(srd, dst, (op ? voff_b[0] : voff_a[0]) | vor, k0 + i * dma_row_stride);
+        dma16(srd, dst, (op ? voff_b : voff_a) | vor, k0 + i * dma_row_stride);
     };
     // this wave's scale load of operand `op` for the pair of K-steps `pair` (stage pair % 2)
     auto dma_scale = [&](int op, uint32_t pair, v4i srd) {
@@ -287,6 +271,29 @@ __global__ __launch_bounds__(256) void mxfp4_gemm_4wave_kernel(
     mfma_drain_agpr(acc);
 
     store_c_tile<MT, NT, EDGE>(acc, C, M, N, row0 + wm * TM, col0 + wn * TN, 1.0f);
+}
+
+// The five-slot ring schedule (gemm_ring.h) with the scaled FP4 MFMA, for its two shorter tiles: they leave LDS for the
+// scales, and the loads are spread over the whole K-step instead of standing behind its barrier.
+struct Mxfp4RingMma {
+    using Frag = Frag4;   // MX blocks g and 4 + g of the K-step
+    static constexpr int kPasses = 2;
+    static constexpr bool kScaled = true;
+    static __device__ __forceinline__ Frag load(uint32_t lo, uint32_t hi, int imm) { return lds_frag4(lo, hi, imm); }
+    template <int PASS>
+    static __device__ __forceinline__ void mma(v4f& acc, const Frag& b, const Frag& a, int sb, int sa) {
+        if constexpr (PASS == 0) mfma_fp4_acc(acc, b.lo, a.lo, sb, sa);
+        else mfma_fp4_acc(acc, b.hi, a.hi, sb, sa);
+    }
+    static __device__ __forceinline__ int raster_group(int band_n, int tiles_n) { return band_n < tiles_n ? 4 : 8; }
+};
+// K: the operands' row length in bytes.
+template <bool EDGE, int TILE_M, int TILE_N>
+__global__ __launch_bounds__(256) void mxfp4_gemm_4wave_ring_kernel(
+    const uint8_t* __restrict__ A, const uint8_t* __restrict__ B, uint16_t* __restrict__ C, int M, int N, int K,
+    int tiles_m, int tiles_n, int band_n, RingScales sc) {
+    extern __shared__ __attribute__((aligned(2048))) uint8_t smem[];
+    gemm_ring_body<Mxfp4RingMma, EDGE, false, TILE_M, TILE_N>(smem, A, B, C, M, N, K, 1.0f, tiles_m, tiles_n, band_n, sc);
 }
 
 // Portable kernel for any M, N and K % 32 == 0: operands and scales straight from global
@@ -532,12 +539,12 @@ static int launch_mxfp4_pingpong(const void* A, const void* SA, const void* B, c
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
-template <bool EDGE>
 static int launch_mxfp4_4wave(const void* A, const void* SA, const void* B, const void* SB, void* C,
                               int M, int N, int K, int sa_pitch, int sb_pitch, Mxfp4ScaleRows sr, hipStream_t stream) {
-    auto kern = mxfp4_gemm_4wave_kernel<EDGE>;
-    static DeviceOnce configured;
-    if (!set_lds_limit_once((const void*)kern, kLdsBytesFp4, configured)) return HK_ERR_LAUNCH;
+    const bool edge = (M % BM) != 0 || (N % BN) != 0;
+    auto kern = edge ? mxfp4_gemm_4wave_kernel<true> : mxfp4_gemm_4wave_kernel<false>;
+    static DeviceOnce configured[2];
+    if (!set_lds_limit_once((const void*)kern, kLdsBytesFp4, configured[edge])) return HK_ERR_LAUNCH;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(256), kLdsBytesFp4, stream,
                        (const uint8_t*)A, (const uint8_t*)SA, (const uint8_t*)B, (const uint8_t*)SB,
@@ -546,11 +553,26 @@ static int launch_mxfp4_4wave(const void* A, const void* SA, const void* B, cons
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
+template <int TILE_M, int TILE_N>
+static int launch_mxfp4_ring(const void* A, const void* SA, const void* B, const void* SB, void* C, int M, int N, int K,
+                             int sa_pitch, int sb_pitch, Mxfp4ScaleRows sr, hipStream_t stream) {
+    const bool edge = (M % TILE_M) != 0 || (N % TILE_N) != 0;
+    auto kern = edge ? mxfp4_gemm_4wave_ring_kernel<true, TILE_M, TILE_N> : mxfp4_gemm_4wave_ring_kernel<false, TILE_M, TILE_N>;
+    constexpr int lds_bytes = ring_lds_bytes(TILE_M, TILE_N, true);
+    static DeviceOnce configured[2];
+    if (!set_lds_limit_once((const void*)kern, lds_bytes, configured[edge])) return HK_ERR_LAUNCH;
+    const int tiles_m = (M + TILE_M - 1) / TILE_M, tiles_n = (N + TILE_N - 1) / TILE_N;
+    hipLaunchKernelGGL(kern, dim3(tiles_m * tiles_n), dim3(256), lds_bytes, stream, (const uint8_t*)A, (const uint8_t*)B,
+                       (uint16_t*)C, M, N, K / 2, tiles_m, tiles_n, raster_band(((long long)M + N) * (K / 2), tiles_n),
+                       RingScales{(const uint8_t*)SA, (const uint8_t*)SB, sa_pitch, sb_pitch, sr.tail_pair, sr.tail_shift, sr.row_bytes});
+    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
+}
+
 }  // namespace hk
 
 // variant: -1 = choose, 0 = portable kernel, 1 = 256x256 tile kernel (4 waves), 2 / 3 = 128x128 / 64x64 tiles,
 // 4 = 256x256 tile kernel with the 8-wave ping-pong schedule, 5 = 192x256 tile producer / consumer kernel,
-// 6 = the skinny kernel (at most 64 rows of A).
+// 6 = the skinny kernel (at most 64 rows of A); kVariant192x256 / kVariant256x192 = the ring kernel's tiles.
 // Scale rows are sa_pitch / sb_pitch bytes apart (>= K / 32).
 static int mxfp4_gemm_impl(const void* A, const void* A_scales, int sa_pitch, const void* B, const void* B_scales,
                            int sb_pitch, void* C, int M, int N, int K, int variant, void* stream) {
@@ -560,7 +582,7 @@ static int mxfp4_gemm_impl(const void* A, const void* A_scales, int sa_pitch, co
         gemm_dims_too_large(M, N, K))
         return HK_ERR_BAD_SHAPE;
     if (((uintptr_t)A | (uintptr_t)B | (uintptr_t)C) & 15u) return HK_ERR_BAD_ALIGNMENT;
-    if (variant < -1 || variant > 6) return HK_ERR_UNSUPPORTED;
+    if (variant < -1) return HK_ERR_UNSUPPORTED;
     if (variant == 6 && M > kSkinnyMaxMScaled) return HK_ERR_UNSUPPORTED;
     // what the tile kernels need of the scale rows (any pitch and alignment; see mxfp4_scale_rows)
     const Mxfp4ScaleRows sr = mxfp4_scale_rows(K, sa_pitch, sb_pitch);
@@ -568,7 +590,8 @@ static int mxfp4_gemm_impl(const void* A, const void* A_scales, int sa_pitch, co
     if (variant < 0) {
         // the choice of tile of hk_fp8_gemm (pick_tile); a K-step is 256 elements here
         const int tile = pick_tile(kFmtMxfp4, M, N, (K / 2 + BK - 1) / BK, kTileRuleMxfp4);
-        variant = !(sr.ok && size_ok) ? 0 : tile == kTinyTile ? 3 : tile == kSmallTile ? 2 : 1;
+        const int shorter = pick_shorter_tile(M, N, (K / 2 + BK - 1) / BK, tile, kTileRuleMxfp4, kShorterTileMxfp4);
+        variant = !(sr.ok && size_ok) ? 0 : shorter ? shorter : tile == kTinyTile ? 3 : tile == kSmallTile ? 2 : 1;
         // few rows: one pass over B by the skinny kernel where that is faster (use_skinny); it takes any scale rows
         if (size_ok && use_skinny(M, N, (K / 2 + BK - 1) / BK, false, moe_num_compute_units(), kSkinnyMaxMScaled, 2)) variant = 6;
     }
@@ -596,8 +619,10 @@ static int mxfp4_gemm_impl(const void* A, const void* A_scales, int sa_pitch, co
         return e ? launch_mxfp4_small_tile<kTinyTile, kTinyStages, true>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s)
                  : launch_mxfp4_small_tile<kTinyTile, kTinyStages, false>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s);
     }
-    const bool edge = (M % BM) != 0 || (N % BN) != 0;
+    if (variant == kVariant192x256) return launch_mxfp4_ring<192, 256>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s);
+    if (variant == kVariant256x192) return launch_mxfp4_ring<256, 192>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s);
     if (variant == 4 || variant == 5) {
+        const bool edge = (M % BM) != 0 || (N % BN) != 0;
         // the ping-pong and producer / consumer kernels keep the padded-row form (rows of whole groups of 8 scale bytes)
         if (sr.row_bytes != 0) return HK_ERR_BAD_SHAPE;
         if (((uintptr_t)A_scales | (uintptr_t)B_scales) & 3u) return HK_ERR_BAD_ALIGNMENT;
@@ -609,15 +634,14 @@ static int mxfp4_gemm_impl(const void* A, const void* A_scales, int sa_pitch, co
         return edge ? launch_mxfp4_pingpong<true>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, s)
                     : launch_mxfp4_pingpong<false>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, s);
     }
-    return edge ? launch_mxfp4_4wave<true>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s)
-                : launch_mxfp4_4wave<false>(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s);
+    return launch_mxfp4_4wave(A, A_scales, B, B_scales, C, M, N, K, sa_pitch, sb_pitch, sr, s);
 }
 
 extern "C" int hk_mxfp4_gemm_variant(const void* A, const void* A_scales, const void* B,
                                      const void* B_scales, void* C, int M, int N, int K, int variant,
                                      void* stream) {
-    if (variant < 0) return HK_ERR_UNSUPPORTED;
-    return mxfp4_gemm_impl(A, A_scales, K / 32, B, B_scales, K / 32, C, M, N, K, variant, stream);
+    return variant < 0 ? HK_ERR_UNSUPPORTED
+                       : mxfp4_gemm_impl(A, A_scales, K / 32, B, B_scales, K / 32, C, M, N, K, variant > 6 ? -2 : variant, stream);
 }
 
 extern "C" int hk_mxfp4_gemm(const void* A, const void* A_scales, const void* B, const void* B_scales,

@@ -46,6 +46,10 @@ int hk_version(void);
  * reports the tile they would take otherwise. */
 int hk_gemm_tile_choice(int format, int M, int N, int K, int consult_table);
 
+/* Whether hk_fp8_gemm / hk_bf16_gemm / hk_mxfp4_gemm take one of the ring kernel's shorter tiles for a shape in the place
+ * of the tile that hk_gemm_tile_choice names: 0 = no, 1 = 192x256 (192 rows of A), 2 = 256x192. Negative: a status. */
+int hk_gemm_shorter_tile(int format, int M, int N, int K);
+
 /*
  * FP8 e4m3 (OCP e4m3fn) GEMM:  C[M,N] = bf16( (scale_a*scale_b) * sum_k A[m,k]*B[n,k] ).
  * A is [M,K] row-major, B is [N,K] row-major ("column-major B"), both 1 byte per
