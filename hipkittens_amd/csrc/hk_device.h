@@ -54,6 +54,32 @@ __device__ __forceinline__ void dma16(v4i srd, uint32_t lds_base, uint32_t voff,
         : "memory", "m0");
 }
 
+// dma16 / dma16_lanes to AT bytes behind lds_base: the sum is made in M0, so that no scalar register holds it.
+template <int AT>
+__device__ __forceinline__ void dma16_at(v4i srd, uint32_t lds_base, uint32_t voff, uint32_t soff) {
+    asm volatile(
+        "s_add_u32 m0, %0, %4\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, %3 offen lds"
+        :
+        : "s"(lds_base), "v"(voff), "s"(srd), "s"(soff), "n"(AT)
+        : "memory", "m0", "scc");
+}
+template <int AT>
+__device__ __forceinline__ void dma16_lanes_at(v4i srd, uint32_t lds_base, uint32_t voff, uint32_t soff, uint64_t mask) {
+    uint64_t saved;
+    asm volatile(
+        "s_mov_b64 %0, exec\n\t"
+        "s_mov_b64 exec, %5\n\t"
+        "s_add_u32 m0, %1, %6\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %2, %3, %4 offen lds\n\t"
+        "s_mov_b64 exec, %0"
+        : "=&s"(saved)
+        : "s"(lds_base), "v"(voff), "s"(srd), "s"(soff), "s"(mask), "n"(AT)
+        : "memory", "m0", "scc");
+}
+
 // dma16 with the non-temporal hint, for data that is read once (the weights of a decode GEMM): it need not
 // displace what the caches hold for re-use.
 __device__ __forceinline__ void dma16_nt(v4i srd, uint32_t lds_base, uint32_t voff, uint32_t soff) {

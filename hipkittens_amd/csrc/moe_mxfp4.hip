@@ -68,14 +68,18 @@ __device__ __forceinline__ v2i pack8_e4m3(const float (&v)[8], int e) {
     hi = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(hi, c[6], c[7], scale, true);
     return v2i{__builtin_bit_cast(int, lo), __builtin_bit_cast(int, hi)};
 }
-// Gated activation of the extended epilogues. act 0: SiLU(g) * u; act 1: the clamped SwiGLU of
-// the GPT-OSS experts, (clamp(u, -limit, limit) + 1) * g' * sigmoid(alpha * g') with
-// g' = min(g, limit).
-__device__ __forceinline__ float glu_act(int act, float g, float u, float alpha, float limit) {
-    if (act == 0) return silu_mul(g, u);
+// Gated activation of the extended epilogues: SiLU(g) * u, or (CLAMPED) the SwiGLU of the GPT-OSS
+// experts, (clamp(u, -limit, limit) + 1) * g' * sigmoid(alpha * g') with g' = min(g, limit). (A median
+// of three with a NaN is the minimum of the other two: -limit for u, as fmin(fmax()) gives.)
+template <bool CLAMPED>
+__device__ __forceinline__ float glu_act(float g, float u, float alpha, float limit) {
+    if constexpr (!CLAMPED) return silu_mul(g, u);
     g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
+    u = __builtin_amdgcn_fmed3f(u, -limit, limit);
     return (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + __expf(-alpha * g)));
+}
+__device__ __forceinline__ float glu_act(int act, float g, float u, float alpha, float limit) {
+    return act == 0 ? glu_act<false>(g, u, alpha, limit) : glu_act<true>(g, u, alpha, limit);
 }
 
 // MX codes of one row's block of 32 h columns held by the four lanes (r, g = 0..3) of the row: lane (r, g) has columns
@@ -89,11 +93,12 @@ __device__ __forceinline__ v4i mx_block_codes(const float (&h)[2][4], bool ok, i
 #pragma unroll
         for (int j = 0; j < 4; ++j) amax = fmaxf(amax, fabsf(h[o][j]));
     // maximum over the four lanes of the row: rows of 16 lanes swapped in registers
+    // (no NaN and no sign among the maxima: their bits compare as integers do)
     const uint32_t a = __float_as_uint(amax);
     const auto s16 = __builtin_amdgcn_permlane16_swap(a, a, false, false);
-    const uint32_t m1 = __float_as_uint(fmaxf(__uint_as_float(s16[0]), __uint_as_float(s16[1])));
+    const uint32_t m1 = max(s16[0], s16[1]);
     const auto s32 = __builtin_amdgcn_permlane32_swap(m1, m1, false, false);
-    amax = fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
+    amax = __uint_as_float(max(s32[0], s32[1]));
     e = A8 ? mx8_block_exponent(amax) : mx_block_exponent(amax);
     v4i o4;
     if (A8) {
@@ -824,13 +829,20 @@ __global__ __launch_bounds__(512) void moe_mxfp4_gemm_kernel(const MoeGemmParams
 // K-step's lanes for every load stood between the fragments' MFMAs with the matrix cores idle. Layer time before /
 // after: 16384 tokens (biases, clamped SwiGLU) 1470 / 1414 us, with MXFP8 activations 2080 / 1932, 4096 tokens 551 / 539.
 //
+// Where several items share an expert (prefill) neither the weight stream nor the MFMAs bound the kernel but what one wave
+// issues beside them. Gate+up at 16384 tokens, us: whole 985, without epilogues 708, loads alone 430, MFMAs on empty loads 538.
+// Hence: the activation is a template parameter (EXT 2 the clamped SwiGLU; a run-time test stood in front of each of
+// a lane's eight values of every fragment), half of an item's fragments share one branch (kFirst), the MFMA picks a
+// weight scale's byte itself, and LDS addresses of loads are made in M0. Layer before / after: 16384 tokens, biases and
+// clamped SwiGLU 1431 / 1284 us; 12175 tokens of 1792 x 2752, MXFP8, 512 / 453; 6243 of 2624 x 1280, plain 306 / 288.
+//
 // A8: the activations are MXFP8 (e4m3 elements, 256 bytes per row and K-step, same e8m0 scale
 // layout) and the MFMA is the mixed form (fp4 weights x fp8 activations, 32 cycles). The
 // activation tile is kept as two half-tiles of 128-byte rows (K halves), so that the LDS
 // swizzle, the load pieces and the fragment addressing stay those of the FP4 tile; a lane's
 // 32 bytes of a K half are the 16-byte chunks g and g + 4. Items have up to 128 rows then
 // (four 33 KiB stages), and the gate+up epilogue re-quantizes h to MXFP8.
-// EXT: biases / clamped SwiGLU / interleaved source rows in the epilogue.
+// EXT: biases / interleaved source rows in the epilogue, 1 with SiLU, 2 with the clamped SwiGLU.
 // GATHER (gate+up, plain epilogue): the item's rows are fetched by token from x quantized once per
 // token, and their scales once per 16 K-steps; see the kernel body. 16 loads per position then.
 // NT: the weight fragments are loaded with the non-temporal hint. When an expert's rows fit one
@@ -862,7 +874,7 @@ static_assert(S4Cfg<true, true>::kLds <= 160 * 1024 && S4Cfg<false, true>::kLds 
               S4Cfg<true, false>::kLds <= 160 * 1024 && S4Cfg<false, false>::kLds <= 160 * 1024, "LDS of a CU");
 constexpr int kS4Ahead = 3;  // positions between fetch and compute (two measure the same)
 
-template <int MODE, bool EXT, bool A8, bool GATHER = false, bool NT = false>
+template <int MODE, int EXT, bool A8, bool GATHER = false, bool NT = false>
 __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmParams p) {
     static_assert(!GATHER || (MODE == 0 && !EXT), "rows are gathered by the gate+up kernel with the plain epilogue only");
     using Cfg = S4Cfg<A8, GATHER>;
@@ -880,6 +892,9 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
     constexpr int kScaleLoads = GATHER ? 0 : 1;
     constexpr int kLoads = kPieces + kScaleLoads + 10;   // + 8 weight fragments, 2 weight scale dwords
     constexpr int MT = kBM / 16;
+    // The row fragments of an item that are multiplied under one branch; each of the others has its own. A branch between
+    // the MFMAs costs more than the MFMAs of a fragment that holds no rows where most items are more than half full.
+    constexpr int kFirst = NT ? 1 : MT / 2;
     extern __shared__ __attribute__((aligned(2048))) uint8_t smem[];
     const int lane = lane_id(), w = wave_id();
     const int n_items = scalar_load_x1(p.num_items);
@@ -1110,14 +1125,17 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
     auto fetch_load = [&]<int P, int L>() __attribute__((always_inline)) {
         if constexpr (L < kPieces) {
             constexpr int i = L % kGroups, khalf = L / kGroups;
-            uint32_t dst = lds_wave + (uint32_t)(P * kStage + khalf * (kBM * 128) + i * 4096);
-            // a piece past the tile's end (last, partial group of 32 rows): never holds rows, lands in the dump area
-            if constexpr (32 * i + 32 > kBM)
-                if (8 * (4 * i + w) >= kBM) dst = lds_wave + (uint32_t)(Cfg::kLds - Cfg::kDump);
-            if constexpr (GATHER) dma16(f_srd_a, dst, tok_cur[i], f_soff_a + (uint32_t)(khalf * 128));
-            else dma16(f_srd_a, dst, voff_a0 + (uint32_t)(i * 32 * kRow + khalf * 128), 0);
+            constexpr int at = P * kStage + khalf * (kBM * 128) + i * 4096;
+            const uint32_t voff = GATHER ? tok_cur[GATHER ? i : 0] : voff_a0 + (uint32_t)(i * 32 * kRow + khalf * 128);
+            const uint32_t soff = GATHER ? f_soff_a + (uint32_t)(khalf * 128) : 0u;
+            if constexpr (32 * i + 32 > kBM) {
+                // a piece past the tile's end (last, partial group of 32 rows): never holds rows, lands in the dump area
+                dma16(f_srd_a, 8 * (4 * i + w) >= kBM ? lds_wave + (uint32_t)(Cfg::kLds - Cfg::kDump) : lds_wave + (uint32_t)at, voff, soff);
+            } else {
+                dma16_at<at>(f_srd_a, lds_wave, voff, soff);
+            }
         } else if constexpr (L < kPieces + kScaleLoads) {
-            dma16_lanes(f_srd_sa, lds_sa_wave + (uint32_t)(P * kStage), voff_sa, 0, (1ull << (kBM / 8)) - 1ull);
+            dma16_lanes_at<P * kStage>(f_srd_sa, lds_sa_wave, voff_sa, 0, (1ull << (kBM / 8)) - 1ull);
         } else if constexpr (L < kPieces + kScaleLoads + 8) {
             constexpr int f = L - kPieces - kScaleLoads, pair = f >> 2, half = f & 1;
             const uint32_t voff = f_voff_b[half], soff = f_soff_b + (uint32_t)pair * 4096u;
@@ -1173,18 +1191,18 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int n = 0; n < 4; ++n) acc[m][n] = v4f{0.f, 0.f, 0.f, 0.f};
-    auto mfma = [&](v4f& c, const v4i& x, const v4i& y, int sx, int sy) __attribute__((always_inline)) {
+    auto mfma = [&]<int B>(v4f& c, const v4i& x, const v4i& y, int sx, int sy) __attribute__((always_inline)) {
         asm volatile(
-            "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0] cbsz:4 blgp:4"
+            "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,0,0] op_sel_hi:[%6,0,0] cbsz:4 blgp:4"
             : "+a"(c)
-            : "v"(x), "v"(y), "v"(sx), "v"(sy));
+            : "v"(x), "v"(y), "v"(sx), "v"(sy), "n"(B & 1), "n"(B >> 1));
     };
     // fp4 weights (4 registers) x fp8 activations (8 registers)
-    auto mfma8 = [&](v4f& c, const v4i& x, const v8i& y, int sx, int sy) __attribute__((always_inline)) {
+    auto mfma8 = [&]<int B>(v4f& c, const v4i& x, const v8i& y, int sx, int sy) __attribute__((always_inline)) {
         asm volatile(
-            "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel_hi:[0,0,0] cbsz:4"
+            "v_mfma_scale_f32_16x16x128_f8f6f4 %0, %1, %2, %0, %3, %4 op_sel:[%5,0,0] op_sel_hi:[%6,0,0] cbsz:4"
             : "+a"(c)
-            : "v"(x), "v"(y), "v"(sx), "v"(sy));
+            : "v"(x), "v"(y), "v"(sx), "v"(sy), "n"(B & 1), "n"(B >> 1));
     };
 
     // ---- epilogue of row fragment m of the compute item (its accumulators are final) -------------
@@ -1245,7 +1263,7 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
                 const v4f gt = acc[M][2 * o], up = acc[M][2 * o + 1];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    if (EXT) h[o][j] = glu_act(p.act, gt[j] + bias_a[o][j], up[j] + bias_b[o][j], p.alpha, p.limit);
+                    if (EXT) h[o][j] = glu_act<EXT == 2>(gt[j] + bias_a[o][j], up[j] + bias_b[o][j], p.alpha, p.limit);
                     else h[o][j] = silu_mul(gt[j], up[j]);
                 }
             }
@@ -1289,9 +1307,6 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
         if (last) {
             begin_epilogue();
         }
-        int bs[8];  // scale of weight fragment f = 4 pair + 2 n + half: byte 2 half + n of the pair's dword
-#pragma unroll
-        for (int f = 0; f < 8; ++f) bs[f] = (int)((uint32_t)bsc[P][f >> 2] >> (8 * (2 * (f & 1) + ((f >> 1) & 1))));
         uint32_t a_rd[2][2];
 #pragma unroll
         for (int hh = 0; hh < 2; ++hh)
@@ -1325,34 +1340,44 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
         auto loads = [&]<int L>() __attribute__((always_inline)) {
             if constexpr (L < kLoads) fetch_load.template operator()<PF, L>();
         };
+        // row fragment M: its MFMAs, the position's loads between them
         auto frag = [&]<int M>() __attribute__((always_inline)) {
-            if (M < mt) {
-                if (M + 2 < MT) rd(M + 2);  // rows past the tile's count are readable, never used
-                const int sa[2] = {(int)((uint32_t)as[M % 3].x >> sh), (int)((uint32_t)as[M % 3].y >> sh)};
-#pragma unroll
-                for (int half = 0; half < 2; ++half)
-#pragma unroll
-                    for (int n = 0; n < 4; ++n) {
-                        const int f = 4 * (n >> 1) + 2 * (n & 1) + half;
-                        if constexpr (A8) mfma8(acc[M][n], bw[P][f], af8[M % 3][half], bs[f], sa[half]);
-                        else mfma(acc[M][n], bw[P][f], af[M % 3][half], bs[f], sa[half]);
-                        if (half == 0 && n == 1) loads.template operator()<M>();
-                        if (half == 1 && n == 0) loads.template operator()<M + MT>();
-                        if (half == 1 && n == 2) loads.template operator()<M + 2 * MT>();
-                    }
-            } else {
-                loads.template operator()<M>();
-                loads.template operator()<M + MT>();
-                loads.template operator()<M + 2 * MT>();
-            }
-            if constexpr (M >= 1) {
-                if constexpr (P == 3)
-                    if (last && M - 1 < mt_item) epilogue.template operator()<M - 1>(M >= mt);
-            }
+            if (M + 2 < MT) rd(M + 2);  // rows past the tile's count are readable, never used
+            const int sa[2] = {(int)((uint32_t)as[M % 3].x >> sh), (int)((uint32_t)as[M % 3].y >> sh)};
+            [&]<int... X>(std::integer_sequence<int, X...>) __attribute__((always_inline)) {
+                ([&]() __attribute__((always_inline)) {
+                    constexpr int half = X >> 2, n = X & 3, f = 4 * (n >> 1) + 2 * (n & 1) + half;
+                    if constexpr (A8) mfma8.template operator()<2 * half + (n & 1)>(acc[M][n], bw[P][f], af8[M % 3][half], bsc[P][n >> 1], sa[half]);
+                    else mfma.template operator()<2 * half + (n & 1)>(acc[M][n], bw[P][f], af[M % 3][half], bsc[P][n >> 1], sa[half]);
+                    if constexpr (half == 0 && n == 1) loads.template operator()<M>();
+                    if constexpr (half == 1 && n == 0) loads.template operator()<M + MT>();
+                    if constexpr (half == 1 && n == 2) loads.template operator()<M + 2 * MT>();
+                }(), ...);
+            }(std::make_integer_sequence<int, 8>{});
         };
-        [&]<int... M>(std::integer_sequence<int, M...>) __attribute__((always_inline)) {
-            (frag.template operator()<M>(), ...);
-        }(std::make_integer_sequence<int, MT>{});
+        auto no_frag = [&]<int M>() __attribute__((always_inline)) {
+            loads.template operator()<M>();
+            loads.template operator()<M + MT>();
+            loads.template operator()<M + 2 * MT>();
+        };
+        // fragments A .. B - 1 under one branch; behind them the epilogues of fragments A - 1 .. B - 2
+        auto group = [&]<int A, int B>() __attribute__((always_inline)) {
+            const bool on = A < mt;
+            [&]<int... X>(std::integer_sequence<int, X...>) __attribute__((always_inline)) {
+                if (__builtin_expect(on, true)) (frag.template operator()<A + X>(), ...);
+                else (no_frag.template operator()<A + X>(), ...);
+                if constexpr (P == 3)
+                    if (last) ([&]() __attribute__((always_inline)) {
+                        constexpr int M = A + X - 1;
+                        if constexpr (M >= 0)
+                            if (M < mt_item) epilogue.template operator()<M>(!on);
+                    }(), ...);
+            }(std::make_integer_sequence<int, B - A>{});
+        };
+        group.template operator()<0, kFirst>();
+        [&]<int... X>(std::integer_sequence<int, X...>) __attribute__((always_inline)) {
+            (group.template operator()<kFirst + X, kFirst + X + 1>(), ...);
+        }(std::make_integer_sequence<int, MT - kFirst>{});
         advance_cf();
         if constexpr (P == 3)
             if (last && MT - 1 < mt_item) epilogue.template operator()<MT - 1>(true);
@@ -1473,7 +1498,7 @@ void moe_launch_build_items(const int32_t* expert_offsets, int E, int bm, int n_
     hipLaunchKernelGGL(moe_build_items_kernel, dim3(2, 8), dim3(512), 0, s, expert_offsets, E, b, num_items);
 }
 
-template <int MODE, bool EXT, bool A8, bool GATHER, bool NT>
+template <int MODE, int EXT, bool A8, bool GATHER, bool NT>
 static int launch_moe_stream_nt(MoeGemmParams p, int max_items, hipStream_t s) {
     constexpr int lds = S4Cfg<A8, GATHER>::kLds, threads = 256;
     const void* kern = (const void*)moe_mxfp4_stream4_kernel<MODE, EXT, A8, GATHER, NT>;
@@ -1486,7 +1511,7 @@ static int launch_moe_stream_nt(MoeGemmParams p, int max_items, hipStream_t s) {
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 // nt: non-temporal weight loads (see the kernel)
-template <int MODE, bool EXT, bool A8, bool GATHER = false>
+template <int MODE, int EXT, bool A8, bool GATHER = false>
 static int launch_moe_stream(MoeGemmParams p, int max_items, hipStream_t s, bool nt) {
     return nt ? launch_moe_stream_nt<MODE, EXT, A8, GATHER, true>(p, max_items, s)
               : launch_moe_stream_nt<MODE, EXT, A8, GATHER, false>(p, max_items, s);
@@ -1800,14 +1825,15 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
     if (few)
         st = launch_moe_few<0>(p, few, a8, ext, moe_few_max_items(S, E, few, p.n_tiles_n), s);
     else if (a8)
-        st = ext ? launch_moe_stream<0, true, true>(p, L.max_items1, s, nt)
-                 : gather ? launch_moe_stream<0, false, true, true>(p, L.max_items1, s, nt)
-                          : launch_moe_stream<0, false, true>(p, L.max_items1, s, nt);
+        st = ext ? (activation ? launch_moe_stream<0, 2, true>(p, L.max_items1, s, nt) : launch_moe_stream<0, 1, true>(p, L.max_items1, s, nt))
+                 : gather ? launch_moe_stream<0, 0, true, true>(p, L.max_items1, s, nt)
+                          : launch_moe_stream<0, 0, true>(p, L.max_items1, s, nt);
     else if (ext)
-        st = weight_layout ? launch_moe_stream<0, true, false>(p, L.max_items1, s, nt) : launch_moe_gemm<0, true>(p, L.max_items1, s);
+        st = !weight_layout ? launch_moe_gemm<0, true>(p, L.max_items1, s)
+             : activation ? launch_moe_stream<0, 2, false>(p, L.max_items1, s, nt) : launch_moe_stream<0, 1, false>(p, L.max_items1, s, nt);
     else
-        st = gather ? launch_moe_stream<0, false, false, true>(p, L.max_items1, s, nt)
-             : weight_layout ? launch_moe_stream<0, false, false>(p, L.max_items1, s, nt) : launch_moe_gemm<0, false>(p, L.max_items1, s);
+        st = gather ? launch_moe_stream<0, 0, false, true>(p, L.max_items1, s, nt)
+             : weight_layout ? launch_moe_stream<0, 0, false>(p, L.max_items1, s, nt) : launch_moe_gemm<0, false>(p, L.max_items1, s);
     if (st != HK_OK) return st;
 
     MoeGemmParams q{};
@@ -1826,11 +1852,11 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
     if (few)
         st = launch_moe_few<1>(q, few, a8, bias2 != nullptr, moe_few_max_items(S, E, few, q.n_tiles_n), s);
     else if (a8)
-        st = bias2 ? launch_moe_stream<1, true, true>(q, L.max_items2, s, nt) : launch_moe_stream<1, false, true>(q, L.max_items2, s, nt);
+        st = bias2 ? launch_moe_stream<1, 1, true>(q, L.max_items2, s, nt) : launch_moe_stream<1, 0, true>(q, L.max_items2, s, nt);
     else if (bias2)
-        st = weight_layout ? launch_moe_stream<1, true, false>(q, L.max_items2, s, nt) : launch_moe_gemm<1, true>(q, L.max_items2, s);
+        st = weight_layout ? launch_moe_stream<1, 1, false>(q, L.max_items2, s, nt) : launch_moe_gemm<1, true>(q, L.max_items2, s);
     else
-        st = weight_layout ? launch_moe_stream<1, false, false>(q, L.max_items2, s, nt) : launch_moe_gemm<1, false>(q, L.max_items2, s);
+        st = weight_layout ? launch_moe_stream<1, 0, false>(q, L.max_items2, s, nt) : launch_moe_gemm<1, false>(q, L.max_items2, s);
     if (st != HK_OK) return st;
 
     return hk_moe_unpermute(ws + L.o, topk_w, slot_to_pos, T, k, H, y_bf16, stream);
