@@ -832,9 +832,9 @@ __global__ __launch_bounds__(512) void moe_mxfp4_gemm_kernel(const MoeGemmParams
 // Where several items share an expert (prefill) neither the weight stream nor the MFMAs bound the kernel but what one wave
 // issues beside them. Gate+up at 16384 tokens, us: whole 985, without epilogues 708, loads alone 430, MFMAs on empty loads 538.
 // Hence: the activation is a template parameter (EXT 2 the clamped SwiGLU; a run-time test stood in front of each of
-// a lane's eight values of every fragment), half of an item's fragments share one branch (kFirst), the MFMA picks a
+// a lane's eight values of every fragment), two thirds of an item's fragments share one branch (kFirst), the MFMA picks a
 // weight scale's byte itself, and LDS addresses of loads are made in M0. Layer before / after: 16384 tokens, biases and
-// clamped SwiGLU 1431 / 1284 us; 12175 tokens of 1792 x 2752, MXFP8, 512 / 453; 6243 of 2624 x 1280, plain 306 / 288.
+// clamped SwiGLU 1417 / 1248 us; 12175 tokens of 1792 x 2752, MXFP8, 509 / 436; 6243 of 2624 x 1280, plain 305 / 276.
 //
 // A8: the activations are MXFP8 (e4m3 elements, 256 bytes per row and K-step, same e8m0 scale
 // layout) and the MFMA is the mixed form (fp4 weights x fp8 activations, 32 cycles). The
@@ -892,9 +892,11 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
     constexpr int kScaleLoads = GATHER ? 0 : 1;
     constexpr int kLoads = kPieces + kScaleLoads + 10;   // + 8 weight fragments, 2 weight scale dwords
     constexpr int MT = kBM / 16;
-    // The row fragments of an item that are multiplied under one branch; each of the others has its own. A branch between
-    // the MFMAs costs more than the MFMAs of a fragment that holds no rows where most items are more than half full.
-    constexpr int kFirst = NT ? 1 : MT / 2;
+    // The row fragments of an item that are multiplied under one branch; each of the others has its own. Where an expert has
+    // several items, each holds at least seven fragments of twelve (rows are spread evenly), and a branch between the MFMAs
+    // costs more than the MFMAs of one that holds no rows. Layer, us, 1 / 4 / 6 / 8 of 12: 16384 tokens 1316 / 1279 / 1266 /
+    // 1248, 12175 of 1792 x 2752 (MXFP8) 463 / 452 / 446 / 436, 2583 of 1088 x 3968 208 / 198 / 197 / 191.
+    constexpr int kFirst = NT ? 1 : MT * 8 / 12;
     extern __shared__ __attribute__((aligned(2048))) uint8_t smem[];
     const int lane = lane_id(), w = wave_id();
     const int n_items = scalar_load_x1(p.num_items);
@@ -1271,7 +1273,8 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
             const v4i o4 = mx_block_codes<A8>(h, st_ok[0], e);
             asm volatile("buffer_store_dwordx4 %0, %1, %2, 0 offen\n\ts_nop 1"
                          :: "v"(o4), "v"(st_voff0), "s"(st_srd0) : "memory");
-            asm volatile("buffer_store_byte %0, %1, %2, 0 offen"
+            // (s_nop 4: the descriptor may have been restored from a spill slot directly in front of the statement)
+            asm volatile("s_nop 4\n\tbuffer_store_byte %0, %1, %2, 0 offen"
                          :: "v"(e + 127), "v"(st_voff1), "s"(st_srd1) : "memory");
             st_voff0 += 16u * (uint32_t)kRow;
             st_voff1 += 16u * 8u;
