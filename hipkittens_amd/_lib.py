@@ -2,11 +2,16 @@
 from __future__ import annotations
 
 import ctypes
+import importlib.util
 from ctypes import c_float, c_int, c_size_t, c_void_p
 from pathlib import Path
 
 _LIB_PATH = Path(__file__).resolve().parent / "libhk355.so"
 _lib = None
+_DISPATCH_PATH = Path(__file__).resolve().parent / "_dispatch.so"
+_DISPATCH_ENTRIES = ("fp8_gemm", "fp8_gemm_ws", "bf16_gemm", "bf16_gemm_ws", "mxfp4_gemm", "mxfp4_gemm_ws",
+                     "mxfp4_gemm_pitched", "mxfp4_quantize_rows")   # the order of csrc/dispatch.cpp's Entries
+_dispatch = None
 
 # name -> (restype, argtypes); one entry per symbol declared in include/hk355.h
 SIGNATURES = {
@@ -112,6 +117,22 @@ def load_library() -> ctypes.CDLL:
         fn.argtypes = argtypes
     _lib = lib
     return lib
+
+
+def load_dispatch():
+    """The dispatchers' CPython module (csrc/dispatch.cpp), bound to the library. Raises RuntimeError if absent."""
+    global _dispatch
+    if _dispatch is not None:
+        return _dispatch
+    lib = load_library()
+    if not _DISPATCH_PATH.exists():
+        raise RuntimeError(f"{_DISPATCH_PATH} is missing: build it with `python -m hipkittens_amd.build`")
+    spec = importlib.util.spec_from_file_location("hipkittens_amd._dispatch", _DISPATCH_PATH)
+    module = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(module)
+    module.bind(*(ctypes.cast(getattr(lib, "hk_" + name), c_void_p).value for name in _DISPATCH_ENTRIES))
+    _dispatch = module
+    return module
 
 
 def check(status: int, what: str) -> None:

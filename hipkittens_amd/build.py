@@ -21,6 +21,9 @@ LIB_PATH = PKG_DIR / "libhk355.so"
 # nothing of it is exported by, or linked into, the product library; only bench.py loads it.
 BENCH_LIB_PATH = PKG_DIR / "libhk355_bench.so"
 
+# the dispatchers' CPython module (csrc/dispatch.cpp, host code only)
+DISPATCH_PATH = PKG_DIR / "_dispatch.so"
+
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
     "-O3",
@@ -69,7 +72,9 @@ def build(verbose: bool = True, extra_flags: list[str] | None = None, jobs: int 
         raise RuntimeError(f"no .hip sources under {CSRC}")
     bench_sources = sorted((CSRC / "bench").glob("*.hip"))
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
+        dispatch = pool.submit(_build_dispatch)
         all_objs = list(pool.map(lambda s: _compile_one(s, extra), sources + bench_sources))
+        dispatch.result()
     objs, bench_objs = all_objs[:len(sources)], all_objs[len(sources):]
     _link(objs, LIB_PATH)
     if bench_objs:
@@ -87,6 +92,23 @@ def build(verbose: bool = True, extra_flags: list[str] | None = None, jobs: int 
         if verbose:
             print("isa_check: 0 findings", file=sys.stderr)
     return LIB_PATH
+
+
+def _build_dispatch() -> None:
+    import sysconfig
+
+    from torch.utils import cpp_extension
+
+    tmp = DISPATCH_PATH.with_suffix(".so.tmp")
+    lib_dirs = cpp_extension.library_paths()
+    cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++20", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM",
+           "-D__HIP_PLATFORM_AMD__", *(f"-isystem{d}" for d in cpp_extension.include_paths()), "-isystem/opt/rocm/include",
+           f"-isystem{sysconfig.get_paths()['include']}", str(CSRC / "dispatch.cpp"), "-o", str(tmp),
+           *(f"-L{d}" for d in lib_dirs), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for dispatch.cpp:\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, DISPATCH_PATH)
 
 
 def _link(objs: list[Path], out: Path) -> None:

@@ -42,6 +42,13 @@ def _stream(t) -> int:
 
 
 _FP8 = (torch.float8_e4m3fn, torch.uint8)
+_native = None
+
+
+def _load_native():
+    global _native
+    _native = _lib.load_dispatch()
+    return _native
 
 
 def gemm_tile_choice(fmt: str, M: int, N: int, K: int, consult_table: bool = True) -> int:
@@ -68,6 +75,10 @@ def dispatch_fp8_gemm(A, B, C, scale_a: float = 1.0, scale_b: float = 1.0, varia
     `variant` -1 lets the library choose; 0..8 force a kernel (see include/hk355.h). `workspace`
     (uint8, fp8_gemm_workspace_bytes(M, N, K) bytes): lets the library split K for decode-like
     shapes (hk_fp8_gemm_ws)."""
+    if variant == -1:   # ordinary arguments are checked and launched natively; None: they are not
+        st = (_native or _load_native()).fp8_gemm(A, B, C, scale_a, scale_b, workspace)
+        if st is not None:
+            return _lib.check(st, "dispatch_fp8_gemm")
     _check_tensor(A, "A", _FP8, 2)
     _check_tensor(B, "B", _FP8, 2)
     _check_tensor(C, "C", (torch.bfloat16,), 2)
@@ -103,6 +114,10 @@ def dispatch_bf16_gemm(A, B, C, variant: int = -1, workspace=None) -> None:
     (include/hk355.h: hk_bf16_gemm). `variant` -1 lets the library choose; 0..6 force a kernel.
     `workspace` (uint8, bf16_gemm_workspace_bytes(M, N, K) bytes): lets the library split K for
     decode-like shapes (hk_bf16_gemm_ws)."""
+    if variant == -1:
+        st = (_native or _load_native()).bf16_gemm(A, B, C, workspace)
+        if st is not None:
+            return _lib.check(st, "dispatch_bf16_gemm")
     _check_tensor(A, "A", _BF16, 2)
     _check_tensor(B, "B", _BF16, 2)
     _check_tensor(C, "C", _BF16, 2)
@@ -152,6 +167,10 @@ def dispatch_mxfp4_gemm(A, A_scales, B, B_scales, C, variant: int = -1, workspac
     `variant` -1 lets the library choose; 0..6 force a kernel (see include/hk355.h).
     `workspace` (uint8, mxfp4_gemm_workspace_bytes(M, N, K) bytes): lets the library split K for
     decode-like shapes (hk_mxfp4_gemm_ws)."""
+    if variant == -1:
+        st = (_native or _load_native()).mxfp4_gemm(A, A_scales, B, B_scales, C, workspace)
+        if st is not None:
+            return _lib.check(st, "dispatch_mxfp4_gemm")
     _check_tensor(A, "A", _FP4, 2)
     _check_tensor(B, "B", _FP4, 2)
     _check_tensor(A_scales, "A_scales", _E8M0, 2)
@@ -256,6 +275,9 @@ _BF16 = (torch.bfloat16,)
 
 def dispatch_mxfp4_quantize_rows(x, packed, scales) -> None:
     """x [R,C] bf16 -> packed [R,C/2] uint8, scales [R,pitch] uint8 (pitch >= C/32, multiple of 8)."""
+    st = (_native or _load_native()).mxfp4_quantize_rows(x, packed, scales)
+    if st is not None:
+        return _lib.check(st, "dispatch_mxfp4_quantize_rows")
     _check_tensor(x, "x", _BF16, 2)
     _check_tensor(packed, "packed", _FP4, 2)
     _check_tensor(scales, "scales", _E8M0, 2)

@@ -1,0 +1,114 @@
+"""The native dispatchers (csrc/dispatch.cpp): they take what the Python dispatchers take, leave the rest to them, and give
+the same results."""
+import pytest
+import torch
+
+import hipkittens_amd as hk
+from hipkittens_amd import _lib
+
+tk = hk.tk_kernel
+
+
+def _needs_build():
+    if not hk.lib_path().exists():
+        pytest.skip("library not built")
+
+
+def test_cpu_tensors_and_wrong_types_are_left_to_python():
+    _needs_build()
+    nat = _lib.load_dispatch()
+    a, c = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(4, 4, dtype=torch.bfloat16)
+    u = torch.zeros(4, 64, dtype=torch.uint8)
+    assert nat.bf16_gemm(a, a, c, None) is None
+    assert nat.fp8_gemm(u, u, c, 1.0, 1.0, None) is None
+    assert nat.mxfp4_gemm(u, u, u, u, c, None) is None
+    assert nat.mxfp4_quantize_rows(a, u, u) is None
+    assert nat.bf16_gemm(a, a, c) is None and nat.bf16_gemm(None, 3, "x", a) is None
+    with pytest.raises(RuntimeError, match="GPU device"):
+        tk.dispatch_bf16_gemm(a, a, c)
+    with pytest.raises(RuntimeError, match="expected a torch.Tensor"):
+        tk.dispatch_fp8_gemm([1], u, c)
+
+
+def _python_only(monkeypatch):
+    class Off:
+        def __getattr__(self, name):
+            return lambda *args: None
+    monkeypatch.setattr(tk, "_native", Off())
+
+
+def _calls(dev):
+    g = torch.Generator(device=dev).manual_seed(3)
+    M, N, K = 33, 80, 544
+    x, w = (torch.randn(r, K, device=dev, generator=g).to(torch.bfloat16) for r in (M, N))
+    (x8, sx), (w8, sw) = hk.quant.quantize_fp8_per_tensor(x), hk.quant.quantize_fp8_per_tensor(w)
+    (x4, xs), (w4, ws) = hk.quant.quantize_mxfp4(x), hk.quant.quantize_mxfp4(w)
+    pad, space = hk.quant.pad_scales(xs), torch.empty(1 << 20, dtype=torch.uint8, device=dev)
+    new = lambda: torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=dev)
+    q = lambda: (torch.zeros(M, K // 2, dtype=torch.uint8, device=dev), torch.zeros(M, 24, dtype=torch.uint8, device=dev))
+    return {
+        "fp8": (tk.dispatch_fp8_gemm, lambda c: (x8, w8, c, sx, sw), {}, new),
+        "fp8 bytes": (tk.dispatch_fp8_gemm, lambda c: (x8.view(torch.uint8), w8, c), {}, new),
+        "fp8 int scales": (tk.dispatch_fp8_gemm, lambda c: (x8, w8, c, 2, 1), {}, new),   # (left to Python)
+        "fp8 workspace": (tk.dispatch_fp8_gemm, lambda c: (x8, w8, c, sx, sw), {"workspace": space}, new),
+        "bf16": (tk.dispatch_bf16_gemm, lambda c: (x, torch.nn.Parameter(w), c), {}, new),
+        "bf16 workspace": (tk.dispatch_bf16_gemm, lambda c: (x, w, c), {"workspace": space}, new),
+        "mxfp4": (tk.dispatch_mxfp4_gemm, lambda c: (x4, xs, w4, ws, c), {}, new),
+        "mxfp4 e8m0": (tk.dispatch_mxfp4_gemm, lambda c: (x4, xs.view(torch.float8_e8m0fnu), w4, ws, c), {}, new),
+        "mxfp4 pitched": (tk.dispatch_mxfp4_gemm, lambda c: (x4, pad, w4, ws, c), {}, new),
+        "mxfp4 workspace": (tk.dispatch_mxfp4_gemm, lambda c: (x4, pad, w4, ws, c), {"workspace": space}, new),
+        "quantize": (tk.dispatch_mxfp4_quantize_rows, lambda o: (x, *o), {}, q),
+    }
+
+
+_NAMES = ["fp8", "fp8 bytes", "fp8 int scales", "fp8 workspace", "bf16", "bf16 workspace", "mxfp4", "mxfp4 e8m0",
+          "mxfp4 pitched", "mxfp4 workspace", "quantize"]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", _NAMES)
+def test_same_results_as_the_python_dispatcher(monkeypatch, name):
+    fn, args, kw, new = _calls("cuda:0")[name]
+    out = [new(), new()]
+    with torch.cuda.stream(torch.cuda.Stream()):   # the current stream, not the default one
+        fn(*args(out[0]), **kw)
+        torch.cuda.current_stream().synchronize()
+    _python_only(monkeypatch)
+    fn(*args(out[1]), **kw)
+    torch.cuda.synchronize()
+    flat = lambda o: [t.view(torch.uint8) for t in (o if isinstance(o, tuple) else (o,))]
+    assert all(torch.equal(a, b) for a, b in zip(flat(out[0]), flat(out[1])))
+    assert not isinstance(out[0], torch.Tensor) or torch.isfinite(out[0].float()).all()
+
+
+@pytest.mark.gpu
+def test_refused_as_before():
+    dev = "cuda:0"
+    a = torch.zeros(32, 64, dtype=torch.bfloat16, device=dev)
+    c = torch.zeros(32, 32, dtype=torch.bfloat16, device=dev)
+    u = torch.zeros(32, 64, dtype=torch.uint8, device=dev)
+    for bad in [lambda: tk.dispatch_bf16_gemm(a, a, c[:, :16]), lambda: tk.dispatch_bf16_gemm(a.t(), a, c),
+                lambda: tk.dispatch_bf16_gemm(a, a.cpu(), c), lambda: tk.dispatch_bf16_gemm(a, a.float(), c),
+                lambda: tk.dispatch_bf16_gemm(a.view(-1)[4:4 + 32 * 60].view(32, 60), a[:, :60].contiguous(), c),
+                lambda: tk.dispatch_fp8_gemm(u, u[:, :48].contiguous(), c), lambda: tk.dispatch_fp8_gemm(u, u, c, workspace=a),
+                lambda: tk.dispatch_mxfp4_gemm(u, u[:, :2], u, u, c), lambda: tk.dispatch_mxfp4_gemm(u, u[:16], u, u, c),
+                lambda: tk.dispatch_mxfp4_quantize_rows(a, u, u),
+                lambda: torch.vmap(lambda t: tk.dispatch_bf16_gemm(t, a, c))(a.unsqueeze(0))]:
+        with pytest.raises(RuntimeError):
+            bad()
+
+
+@pytest.mark.gpu
+def test_captured_calls_replay():
+    fn, args, kw, new = _calls("cuda:0")["mxfp4 pitched"]
+    want, got = new(), new()
+    fn(*args(want), **kw)
+    torch.cuda.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        fn(*args(got), **kw)
+    for _ in range(3):
+        got.fill_(float("nan"))
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
