@@ -398,8 +398,9 @@ __global__ __launch_bounds__(512) void moe_fp8blk_gemm_kernel(const MoeFp8Params
 //     zeros in LDS and are never stored), because accumulators behind branches cost register copies.
 // The stream of (item, K-step) positions runs across item boundaries. All vector-memory loads are
 // inline asm and counted by hand: per position a wave issues 14 loads (5 activation pieces, the row
-// scales, 8 weight pieces; GATHER: 6 more per item for the slot ids), loads return in order, and the
-// wait for position p + 1 sits in step p behind the loads of position p + 3: vmcnt(2 x 14). (Four
+// scales, 8 weight pieces; GATHER: the row scales with every fourth position only, and 6 more per item for the
+// slot ids), loads return in order, and the wait for position p + 1 sits in step p behind the loads of position
+// p + 3: vmcnt(2 x 14), GATHER 26 or 27. (Four
 // positions ahead on five stages measured the same.) An item takes nk4 positions, nk rounded up to
 // a multiple of the four register sets: its last position then always falls on set 3 and the
 // epilogue code exists once (with a copy per set the kernel is 139 KB of code and every epilogue
@@ -414,9 +415,17 @@ constexpr int kF8BMShort = 144;
 constexpr int kF8sStages = 4;                           // LDS stages = weight register sets = positions per trip of the K loop
 constexpr int kF8sStage = 21504;                         // 160 x 128 B, then 16 x 12 row scales, padded to a multiple of 256 B
 constexpr int kF8sXch = kF8sStages * kF8sStage;          // epilogue exchange buffer: 160 x 4 floats
-constexpr int kF8sLds = kF8sXch + kF8BM * 16;            // 86.5 KiB
+// GATHER: the row scales of four K-steps (16 bytes per row) come in together, with the first of the four. A row's scales lie
+// in its token's row of the caller's array, so that a load touches a cache line per lane: 48 lines for 4 bytes each with
+// every K-step, where the eight weight and five activation pieces beside it touch 104. Two buffers of [row % 16][row / 16,
+// padded to 13] x 4 floats and one of zeros, which the padding positions read. A load per K-step / per four, layer, us:
+// DeepSeek-V3-like 8192 tokens 4199 / 4128; H = 7168, I = 2048, 64 experts, k = 6, 1479 tokens 773 / 741; H = 2816,
+// I = 1024, 64 experts, k = 4, 3000 tokens 241 / 236; 479 tokens of the first (HBM bound) 1827 / 1833.
+constexpr int kF8sSaBuf = 16 * 13 * 16;
+constexpr int kF8sSa = kF8sXch + kF8BM * 16;
+constexpr int kF8sLds = kF8sSa + 3 * kF8sSaBuf;          // 96.3 KiB
 constexpr int kF8sBTile = 256 * 128;                     // one (n-tile, K-step) block of the pre-shuffled weights
-constexpr int kF8sLoads = 14;                            // loads per wave and position
+constexpr int kF8sLoads = 14;                            // loads per wave and position (GATHER: 13 but for every fourth)
 static_assert(kF8sStage >= kF8ATile + 16 * 12 * 4 && kF8sStage % 256 == 0 && kF8sLds <= 160 * 1024, "LDS plan");
 static_assert((kF8sStages - 2) * kF8sLoads < 64 && kF8sStages == 4 && kF8sMT == 10 && kF8BMShort == 144, "vmcnt range; the slot plan below is written for nine or ten fragments");
 
@@ -475,9 +484,13 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
     auto piece_row = [&](int i) { return 40 * w + 8 * i + (lane >> 3); };
     // Row scales of a stage: [row % 16][row / 16, padded to 12] floats, so that a lane's scale of fragment
     // m sits at a fixed offset from its base. Wave w fetches slots [48 w, +48) with lanes 0..47.
-    const int sf = 48 * w + min(lane, 47);
-    const int scale_row = (sf % 12) < MT ? 16 * (sf % 12) + sf / 12 : -1;   // -1: padding slot, nothing fetched
-    constexpr uint64_t kSaMask = (1ull << 48) - 1ull;
+    // GATHER: [row % 16][row / 16, padded to 13], lanes 0..51.
+    constexpr int kSaCols = GATHER ? 13 : 12, kSaLanes = 4 * kSaCols;
+    const int sf = kSaLanes * w + min(lane, kSaLanes - 1);
+    const int scale_row = (sf % kSaCols) < MT ? 16 * (sf % kSaCols) + sf / kSaCols : -1;   // -1: padding slot, nothing fetched
+    constexpr uint64_t kSaMask = (1ull << kSaLanes) - 1ull;
+    // GATHER: first of the four K-steps whose scales come in with position kt (a multiple of four): inside the row
+    auto sa_first = [&](int kt) { return max(min(kt, nk - 4), 0); };
 
     // ---- cursors over this workgroup's stream of (item, K-step) positions -----------------------
     auto load_item = [&](F8Cursor& c) __attribute__((always_inline)) {
@@ -545,7 +558,7 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
         f_srd_b = make_srd(f_b_base, live ? (uint32_t)nk * kF8sBTile : 0u);
         const uint32_t row_base = (uint32_t)cf.kt * (uint32_t)p.S + (uint32_t)cf.row_start;
         f_soff_a = GATHER ? (uint32_t)cf.kt * 128u : row_base * 128u;
-        f_soff_sa = GATHER ? (uint32_t)cf.kt * 4u : row_base * 4u;
+        f_soff_sa = GATHER ? (uint32_t)sa_first(cf.kt) * 4u : row_base * 4u;   // (GATHER: used where cf.kt is a multiple of four)
         f_soff_b = (uint32_t)cf.kt * kF8sBTile + (uint32_t)w * 8192u;
         f_pieces = GATHER ? NA : (cf.rows - 40 * w + 7) >> 3;
     };
@@ -567,7 +580,8 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
 
     const uint32_t lds0 = (uint32_t)(uintptr_t)smem;
     const uint32_t lds_wave_a = to_sgpr(lds0 + (uint32_t)w * 5120u);
-    const uint32_t lds_wave_sa = to_sgpr(lds0 + kF8ATile + (uint32_t)w * 192u);
+    const uint32_t lds_wave_sa = to_sgpr(lds0 + (GATHER ? kF8sSa + (uint32_t)w * (kSaLanes * 16u) : kF8ATile + (uint32_t)w * 192u));
+    uint32_t f_sa = 0, c_sa = 0;   // GATHER: offset of the scale buffer that the next load fills / that holds the compute position's scales
     const uint32_t voff_b = lane * 16;
     struct BFrag { v4i lo, hi; };
     BFrag bw[kF8sStages][NT];   // weight fragments of four positions, in AGPRs
@@ -581,6 +595,11 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
             v4i s = f_srd_a;
             if (!GATHER && ai >= f_pieces) s.z = 0;
             dma16(s, lds_wave_a + PF * kF8sStage + ai * 1024, a_voff[ai], f_soff_a);
+        } else if constexpr (kind == 0 && GATHER) {
+            if constexpr (PF == 0) {
+                dma16_lanes(f_srd_sa, lds_wave_sa + f_sa, sa_voff, f_soff_sa, kSaMask);
+                f_sa = kF8sSaBuf - f_sa;
+            }
         } else if constexpr (kind == 0) {
             dma4_lanes(f_srd_sa, lds_wave_sa + PF * kF8sStage, sa_voff, f_soff_sa, kSaMask);
         } else {
@@ -621,7 +640,13 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
     const uint32_t r = lane & 15, g = lane >> 4;
     const uint32_t rd_lo = lds0 + r * 128u + swz_chunk(r, g) * 16u;
     const uint32_t rd_hi = lds0 + r * 128u + swz_chunk(r, g + 4) * 16u;
-    const uint32_t rd_sa = lds0 + kF8ATile + r * 48u;
+    const uint32_t rd_sa = GATHER ? lds0 + kF8sSa + r * (kSaCols * 16u) : lds0 + kF8ATile + r * 48u;
+    constexpr int kSaStep = GATHER ? 16 : 4;   // bytes between the scales of a lane's consecutive fragments
+    // base of the lane's scales of cursor c's position (stage P; GATHER: in the buffer at `buf`)
+    auto sa_base = [&]<int P>(const F8Cursor& c, uint32_t buf) __attribute__((always_inline)) {
+        if constexpr (!GATHER) return rd_sa + P * kF8sStage;
+        return rd_sa + (c.kt < nk ? buf + 4u * (uint32_t)(c.kt - sa_first(c.kt - P)) : 2u * kF8sSaBuf);
+    };
 
     float acc[MT][NT][4];
     auto zero_acc = [&]() __attribute__((always_inline)) {
@@ -761,14 +786,18 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
     ws_rows_of(cc);   // cn is still in this item (an item has at least four positions)
     request_ws(cc);
     zero_acc();
-    wait_vmcnt<(kF8sStages - 2) * kF8sLoads>();
+    if constexpr (GATHER) {
+        for (int i = threadIdx.x; i < kF8sSaBuf / 4; i += 256) *(lds_f32_mut_t*)(uintptr_t)(lds0 + kF8sSa + 2 * kF8sSaBuf + 4 * i) = 0.f;
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    wait_vmcnt<(kF8sStages - 2) * (GATHER ? kF8sLoads - 1 : kF8sLoads)>();
     block_barrier();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     asm volatile("" : "+s"(ws0_next), "+s"(ws1_next));   // the requested scales are in their registers from here on
     ws0 = ws0_next; ws1 = ws1_next;
     request_ws(cn);
     af[0] = lds_frag(rd_lo, rd_hi, 0);
-    xs_r[0] = *(lds_f32_t*)(uintptr_t)rd_sa;
+    xs_r[0] = *(lds_f32_t*)(uintptr_t)sa_base.template operator()<0>(cc, c_sa);
 
     // One stream position on LDS stage / weight register set P (both = position % 4). Every position
     // runs all ten fragments (rows past the item's count are zeros in LDS and are never stored): a
@@ -781,16 +810,20 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
         constexpr int PAR = (MT & 1) ? (P & 1) : 0, PAR_PREV = (MT & 1) ? (PAR ^ 1) : 0, PAR_NEXT = PAR_PREV;
         fetch_begin();
         landed.template operator()<P>();
-        const uint32_t a_lo = rd_lo + P * kF8sStage, a_hi = rd_hi + P * kF8sStage, a_sa = rd_sa + P * kF8sStage;
+        const uint32_t a_lo = rd_lo + P * kF8sStage, a_hi = rd_hi + P * kF8sStage, a_sa = sa_base.template operator()<P>(cc, c_sa);
+        // loads of the two positions behind the next one
+        constexpr int kBehind = (kF8sStages - 2) * kF8sLoads - (GATHER ? ((P + 2) % 4 != 0) + ((P + 3) % 4 != 0) : 0);
+        if constexpr (GATHER && PN == 0) c_sa = kF8sSaBuf - c_sa;   // the next position's
+        const uint32_t n_sa = sa_base.template operator()<PN>(cn, c_sa);
         // Behind fragment 8's third MFMA, when every LDS read of this position has been issued: the next
         // position's tile is waited for, its first fragment and scale are read, its weight scales arrive.
         auto transition = [&]() __attribute__((always_inline)) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this position's last LDS reads and the scale request
             asm volatile("" : "+s"(ws0_next), "+s"(ws1_next));
-            wait_vmcnt<(kF8sStages - 2) * kF8sLoads>();
+            wait_vmcnt<kBehind>();
             block_barrier();   // everyone's part of the next position's tile has landed; everyone has read this position's
             af[PAR_NEXT] = lds_frag(rd_lo + PN * kF8sStage, rd_hi + PN * kF8sStage, 0);
-            xs_r[PAR_NEXT] = *(lds_f32_t*)(uintptr_t)(rd_sa + PN * kF8sStage);
+            xs_r[PAR_NEXT] = *(lds_f32_t*)(uintptr_t)n_sa;
         };
         // Fragment M: four MFMA slots; the FMAs of an MFMA follow two slots later (fragment 0 starts with
         // those of fragment 9 of the previous K-step).
@@ -803,7 +836,7 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
             mfma.template operator()<P * NT + 0>(part[0], a_cur);
             if constexpr (M < MT - 2) {
                 af[BN] = lds_frag(a_lo, a_hi, (M + 1) * 2048);
-                xs_r[BN] = *(lds_f32_t*)(uintptr_t)(a_sa + (M + 1) * 4);
+                xs_r[BN] = *(lds_f32_t*)(uintptr_t)(a_sa + (M + 1) * kSaStep);
             }
             fma4(acc[MP][2], part[2], sc[BP][0]);
             if constexpr (M <= 6) fetch_load.template operator()<PF, 2 * M>();
@@ -821,7 +854,7 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
             if constexpr (M == MT - 2) {
                 // fragment 9 is read here, ahead of the barrier that frees this stage
                 af[BN] = lds_frag(a_lo, a_hi, (M + 1) * 2048);
-                xs_r[BN] = *(lds_f32_t*)(uintptr_t)(a_sa + (M + 1) * 4);
+                xs_r[BN] = *(lds_f32_t*)(uintptr_t)(a_sa + (M + 1) * kSaStep);
             }
             __builtin_amdgcn_sched_barrier(0);
             // slot 3
