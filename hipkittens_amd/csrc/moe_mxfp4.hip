@@ -133,41 +133,59 @@ __device__ __forceinline__ v4i mx_block_codes(const float (&h)[2][4], bool ok, i
 }
 
 // x [rows, cols] bf16 -> packed e2m1 [rows, cols/2] + e8m0 scales [rows, scale_pitch] (columns
-// >= cols/32 are filled with 127). One thread per 8 elements, 4 threads per MX block.
-template <bool A8>
+// >= cols/32 are filled with 127). One thread per 8 elements of ROWS consecutive rows, 4 threads per MX block. The loads of
+// a thread's rows go out together: with one row, 16 bytes a thread are too few in flight, and finding the row (a division
+// of 64 bits, which only grids of 2^31 threads and more need: Index) takes longer than the rest.
+// Back to back, us, one row and 64-bit index / now: 8192 x 8192 32.4 / 29.3, 4096 x 8192 18.2 / 15.9, 4096 x 2880 7.4 / 7.2.
+template <bool A8, int ROWS, typename Index>
 __global__ __launch_bounds__(256) void mx_quantize_rows_kernel(const uint16_t* __restrict__ x, int rows,
                                                                int cols, uint8_t* __restrict__ packed,
                                                                uint8_t* __restrict__ scales,
                                                                int scale_pitch) {
-    const int per_row = scale_pitch * 4;  // threads per row, a multiple of 4 (and of 32: pitch % 8 == 0)
-    const long long gid = (long long)blockIdx.x * 256 + threadIdx.x;
-    const int row = (int)(gid / per_row);
+    const Index per_row = (Index)scale_pitch * 4;  // threads per row, a multiple of 4 (and of 32: pitch % 8 == 0)
+    const Index gid = (Index)blockIdx.x * 256 + threadIdx.x;
+    const int row0 = (int)(gid / per_row) * ROWS;
     const int c8 = (int)(gid % per_row);  // which group of 8 elements
-    if (row >= rows) return;
-    float v[8];
+    if (row0 >= rows) return;
     const bool in = c8 * 8 < cols;
-    if (in) {
-        const v4i raw = *(const v4i*)(x + (size_t)row * cols + c8 * 8);
+    v4i raw[ROWS];
+#pragma unroll
+    for (int j = 0; j < ROWS; ++j)
+        raw[j] = in ? *(const v4i*)(x + (size_t)min(row0 + j, rows - 1) * cols + c8 * 8) : v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int j = 0; j < ROWS; ++j) {
+        const int row = row0 + j;
+        if (row >= rows) break;   // (uniform among the threads of a block of 32 elements)
+        float v[8];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            v[2 * i] = __uint_as_float((uint32_t)raw[i] << 16);
-            v[2 * i + 1] = __uint_as_float((uint32_t)raw[i] & 0xffff0000u);
+            v[2 * i] = __uint_as_float((uint32_t)raw[j][i] << 16);
+            v[2 * i + 1] = __uint_as_float((uint32_t)raw[j][i] & 0xffff0000u);
         }
-    } else {
+        float amax = 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = 0.f;
+        for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
+        amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
+        amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
+        const int e = A8 ? mx8_block_exponent(amax) : mx_block_exponent(amax);
+        if (in) {
+            if (A8) *(v2i*)(packed + (size_t)row * cols + c8 * 8) = pack8_e4m3(v, e);
+            else *(uint32_t*)(packed + (size_t)row * (cols / 2) + c8 * 4) = pack8_e2m1(v, e);
+        }
+        if ((c8 & 3) == 0) scales[(size_t)row * scale_pitch + (c8 >> 2)] = (uint8_t)(e + 127);
     }
-    float amax = 0.f;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(v[i]));
-    amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
-    amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
-    const int e = A8 ? mx8_block_exponent(amax) : mx_block_exponent(amax);
-    if (in) {
-        if (A8) *(v2i*)(packed + (size_t)row * cols + c8 * 8) = pack8_e4m3(v, e);
-        else *(uint32_t*)(packed + (size_t)row * (cols / 2) + c8 * 4) = pack8_e2m1(v, e);
-    }
-    if ((c8 & 3) == 0) scales[(size_t)row * scale_pitch + (c8 >> 2)] = (uint8_t)(e + 127);
+}
+template <bool A8>
+static int launch_mx_quantize_rows(const void* x, int rows, int cols, void* packed, void* scales, int scale_pitch, hipStream_t s) {
+    // four rows a thread while that still gives every CU four workgroups (5600 x 544, two of them: 3.9 us, 4.1 with four rows)
+    const long long four = ((long long)rows + 3) / 4 * scale_pitch * 4, one = (long long)rows * scale_pitch * 4;
+    const bool by4 = four >= 1024ll * moe_num_compute_units();
+    const long long threads = by4 ? four : one;
+    auto kern = threads >= (1ll << 31) ? (by4 ? mx_quantize_rows_kernel<A8, 4, long long> : mx_quantize_rows_kernel<A8, 1, long long>)
+                                       : (by4 ? mx_quantize_rows_kernel<A8, 4, unsigned> : mx_quantize_rows_kernel<A8, 1, unsigned>);
+    hipLaunchKernelGGL(kern, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, (const uint16_t*)x, rows, cols,
+                       (uint8_t*)packed, (uint8_t*)scales, scale_pitch);
+    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
 // Item lists of the two grouped GEMMs of a layer: list `which` (0 / 1) covers n_tiles[which] tiles
@@ -289,10 +307,19 @@ __device__ __forceinline__ void mx_quantize_tokens(const MxQuantizeArgs& a, int 
     const int S = T * topk;
     const int nk = (cols / 2 + 127) >> 7;
     // position of slot `slot`, or -1
-    auto position = [&](int slot) -> int {
-        if (!PERMUTE) return slot;
+    auto find = [&](int slot) -> int {
         const int pos = slot_to_pos[slot];
         return (unsigned)pos < (unsigned)S && sorted_slots[pos] == slot ? pos : -1;
+    };
+    // The positions of the token block's slots, found once, a slot per lane: two dependent loads in front of each of a
+    // slot's stores made the kernel wait sixteen times (layer, us, before / after: 842 tokens of 2880 x 2880, 32 experts, k = 4
+    // 153.6 / 147.9; 7232 of 1088 x 640, 64 experts, MXFP8 174.3 / 169.0). The two halves of a wave have the same tokens.
+    const bool held = PERMUTE && kQpRows * topk <= 32;
+    int mine = -1;
+    if (held && c < kQpRows * topk && t0 * topk + c < S) mine = find(t0 * topk + c);
+    auto position = [&](int slot) -> int {
+        if (!PERMUTE) return slot;
+        return held ? __builtin_amdgcn_readlane(mine, slot - t0 * topk) : find(slot);
     };
     if (pad && (K2 & 255)) {
         const int nk2 = (K2 + 255) >> 8;
@@ -1554,11 +1581,7 @@ extern "C" int hk_mxfp4_quantize_rows(const void* x_bf16, int rows, int cols, vo
     if (rows <= 0 || cols <= 0 || (cols % 32) != 0 || scale_pitch < cols / 32 || (scale_pitch % 8) != 0)
         return HK_ERR_BAD_SHAPE;
     if (((uintptr_t)x_bf16 | (uintptr_t)packed) & 15u) return HK_ERR_BAD_ALIGNMENT;
-    const long long threads = (long long)rows * scale_pitch * 4;
-    hipLaunchKernelGGL(mx_quantize_rows_kernel<false>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                       (hipStream_t)stream, (const uint16_t*)x_bf16, rows, cols, (uint8_t*)packed,
-                       (uint8_t*)scales, scale_pitch);
-    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
+    return launch_mx_quantize_rows<false>(x_bf16, rows, cols, packed, scales, scale_pitch, (hipStream_t)stream);
 }
 
 extern "C" int hk_mxfp8_quantize_rows(const void* x_bf16, int rows, int cols, void* codes, void* scales,
@@ -1567,11 +1590,7 @@ extern "C" int hk_mxfp8_quantize_rows(const void* x_bf16, int rows, int cols, vo
     if (rows <= 0 || cols <= 0 || (cols % 32) != 0 || scale_pitch < cols / 32 || (scale_pitch % 8) != 0)
         return HK_ERR_BAD_SHAPE;
     if (((uintptr_t)x_bf16 | (uintptr_t)codes) & 15u) return HK_ERR_BAD_ALIGNMENT;
-    const long long threads = (long long)rows * scale_pitch * 4;
-    hipLaunchKernelGGL(mx_quantize_rows_kernel<true>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0,
-                       (hipStream_t)stream, (const uint16_t*)x_bf16, rows, cols, (uint8_t*)codes,
-                       (uint8_t*)scales, scale_pitch);
-    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
+    return launch_mx_quantize_rows<true>(x_bf16, rows, cols, codes, scales, scale_pitch, (hipStream_t)stream);
 }
 
 extern "C" int hk_moe_unpermute_add(const void* o_bf16, const float* w, const int32_t* slot_to_pos, int T,
