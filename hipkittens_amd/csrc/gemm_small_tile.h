@@ -53,7 +53,7 @@ __device__ __forceinline__ void gemm_small_tile_body(
     constexpr int kTB = TILE * BK, kSB = 2 * kTB;    // bytes of one operand tile / of one stage
     constexpr int NDMA = kTB / (NW * 1024);          // loads per wave per operand per K-step
     constexpr bool kScaled = MMA::kScaled;
-    constexpr int LPT = 2 * NDMA + (kScaled ? 1 : 0);  // loads per wave per K-step
+    constexpr int LPT = 2 * NDMA;                    // operand loads per wave per K-step
     // scales: four slots, each the 16 bytes (two K-steps) of the TILE rows of A, then of B
     constexpr int kScaleSlot = 2 * TILE * 16, kScaleBase = STAGES * kSB;
     static_assert(STAGES >= 3 && STAGES <= 8 && (STAGES - 1) * LPT < 64, "vmcnt range");
@@ -94,11 +94,13 @@ __device__ __forceinline__ void gemm_small_tile_body(
     // this workgroup's K-steps: [kt0, kt0 + nkt)
     const int kt0 = SPLIT ? (int)blockIdx.y * kps : 0;
     const int nkt = SPLIT ? min(kps, nk - kt0) : nk;
-    // Scale loads (kScaled): wave w fetches operand w & 1 (0 = A), lane l the 16 bytes of row
-    // 64 (w >> 1) + l (TILE = 128; with TILE = 64 waves 2 and 3 repeat what 0 and 1 fetch), i.e. the
-    // scales of the pair of K-steps kt / 2. Every wave issues one such load with every K-step (on odd
-    // K-steps it repeats the pair's load into the same slot): the same number of loads per K-step in
-    // every wave keeps the counted waits uniform.
+    // Scale loads (kScaled): wave w fetches operand w & 1 (0 = A), lane l the 16 bytes of row 64 (w >> 1) + l (TILE = 64:
+    // waves 0 and 1 only), i.e. the scales of the pair of K-steps kt / 2, in front of the even K-step's operands. A scale
+    // load touches a cache line per lane, where the 1 KiB loads of operands touch eight: with every K-step and from every
+    // wave, which keeps the waits' counts the same, the scales cost more of a CU's vector-memory path than the operands.
+    // The waits leave the scale loads out: one among the loads behind a K-step makes its wait stricter, never weaker.
+    // (64x64 tiles, us before / after: 128 x 8192 x 8192 21.5 / 17.6, 200 x 8192 x 8192 27.2 / 22.6, 512 x 4096 x 4096 18.5 / 15.3,
+    // 128 x 4096 x 14336 34.6 / 27.0; 128x128 tiles 2 to 4 %.)
     v4i srd_s = {0, 0, 0, 0};
     uint32_t voff_s = 0, lds_s = 0;
     if (kScaled) {
@@ -117,13 +119,13 @@ __device__ __forceinline__ void gemm_small_tile_body(
         const uint32_t k0 = (uint32_t)kt * BK;
         const uint32_t dst = lds_wave + (uint32_t)stage * kSB;
         const uint32_t vor = kt == nk - 1 ? tail_or : 0u;
+        if (kScaled && (kt & 1) == 0 && (TILE == 128 || w < 2))
+            dma16(srd_s, lds_s + (uint32_t)((kt >> 1) & 3) * kScaleSlot, voff_s,
+                  (uint32_t)(kt >> 1) * 16u - ((kt >> 1) == sc.tail_pair ? (uint32_t)sc.tail_shift : 0u));
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) dma16(srd_a, dst + i * NW * 1024, voff_a[i] | vor, k0);
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) dma16(srd_b, dst + kTB + i * NW * 1024, voff_b[i] | vor, k0);
-        if (kScaled)
-            dma16(srd_s, lds_s + (uint32_t)((kt >> 1) & 3) * kScaleSlot, voff_s,
-                  (uint32_t)(kt >> 1) * 16u - ((kt >> 1) == sc.tail_pair ? (uint32_t)sc.tail_shift : 0u));
     };
     // wait until at most `tiles` of the most recently issued K-steps' loads are still in flight
     auto wait_tiles = [&](int tiles) {
@@ -353,8 +355,8 @@ static __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* 
 //     of the single round of 256 small tiles (the small tile wins by 60 %). Measured against the best of the
 //     three kernels, every launch on another copy of B (a model's weights come from HBM, not from the memory-side
 //     cache), the rule alone is more than 5 % behind on 7 / 6 of 414 shapes (FP8 / BF16; 42 / 40 with the constants
-//     that fitted these kernels before their loads and LDS reads were spread over the MFMAs) and on 20 of 360 (MXFP4),
-//     mostly by 5 to 10 % where a long B is read by several rows of small tiles;
+//     that fitted these kernels before their loads and LDS reads were spread over the MFMAs) and on 5 of 414 (MXFP4; 16 with
+//     the constants from before the scaled kernel's scale loads went from every K-step to every second);
 //  2. a generated table of the shapes on which a sweep found the rule's choice more than a few percent behind
 //     another tile (tile_table.inc, written by `python -m hipkittens_amd.tile_sweep FORMAT --emit`; the
 //     counterpart of the reference's per-shape analysis/baselines/gemm/utils/tuned.yaml). An entry is keyed by
@@ -389,30 +391,26 @@ static inline int pick_tile(int fmt, int M, int N, int nk, TileRule r, bool cons
         for (const TileTableEntry& e : kTileTable)
             if (e.fmt == fmt && e.m64 == m64 && e.n64 == n64 && e.nk == nk) return e.tile;
     }
-    // MXFP4, one row of 64x64 tiles and a wide output (128-column tiles for 7 of 8 CUs or more: N >= 28672 on 256
-    // CUs): every 64-row tile fetches its own scale pieces, and with B streaming from HBM the 128x128 tile measured
-    // 15 to 25 % faster at every K (M = 64, N = 32768, K = 16384: 85 -> 69 us), where the cost rule below, which
-    // knows rounds and not bytes, takes the small tile
-    if (fmt == kFmtMxfp4 && M <= kTinyTile && ((long long)N + kSmallTile - 1) / kSmallTile * 8 >= 7ll * cus) return kSmallTile;
     return pick_tile_rule(M, N, nk, r, cus);
 }
 // the formats' constants (K-steps: 128 bytes of an operand row)
 constexpr TileRule kTileRuleFp8{{7.10f, 3.28f, 2.02f}, {1.060f, 0.533f, 0.385f}};
 constexpr TileRule kTileRuleBf16{{8.57f, 2.79f, 2.20f}, {0.983f, 0.495f, 0.336f}};
-constexpr TileRule kTileRuleMxfp4{{7.71f, 3.13f, 1.94f}, {1.316f, 0.767f, 0.549f}};
+constexpr TileRule kTileRuleMxfp4{{7.51f, 3.07f, 1.185f}, {1.316f, 0.710f, 0.587f}};
 
 // The ring kernel's shorter tiles (gemm_ring.h): 192x256 or 256x192 in the place of the tile that pick_tile names, where
 // the same cost model, one workgroup per CU, gives them less time. The constants, and the factor on the estimate for a
 // 128- or 64-tile (which is high where it is compared with these), are fitted to 91 shapes per format on an MI355X
 // (M 500 ... 8192, (N, K) 4096 x 4096 ... 14336 x 4096, 2880 x 2880, 10000 x 1024, copies of B in rotation): no shape
 // is more than 3 % behind what it had, and the geometric mean falls by 5.5 (FP8), 6.3 (BF16) and 6.3 % (MXFP4), of 6.5,
-// 6.9 and 7.0 that the best kernel for every shape would give. Examples, us before / after: BF16 3001 x 4096 x 4096
+// 6.9 and 7.0 that the best kernel for every shape would give (MXFP4 as first fitted; fitted again to 112 shapes when its
+// small-tile kernels became faster: 3 more than 5 % behind the best kernel, before 4). Examples, us before / after: BF16 3001 x 4096 x 4096
 // 90.1 / 74.9 (192 tiles of 256x256 against 256 of 192x256), 4096 x 2880 x 2880 69.2 / 54.1; FP8 8192 x 2880 x 2880
 // 71.8 / 58.6; MXFP4 4096 x 2880 x 2880 35.2 / 27.8; and not taken: BF16 4096 x 4096 x 4096 96.3 / 130.9 (256 tiles of
 // 256x256, one round; 352 of 192x256, two).
 constexpr int kVariant192x256 = 100, kVariant256x192 = 101;   // the GEMM entry points' internal numbers for them
 struct ShorterTileRule { float fixed, per_step, small; };
-constexpr ShorterTileRule kShorterTileFp8{5.7f, 0.87f, 0.82f}, kShorterTileBf16{5.6f, 0.925f, 0.94f}, kShorterTileMxfp4{7.3f, 1.29f, 1.0f};
+constexpr ShorterTileRule kShorterTileFp8{5.7f, 0.87f, 0.82f}, kShorterTileBf16{5.6f, 0.925f, 0.94f}, kShorterTileMxfp4{7.37f, 1.057f, 0.974f};
 static inline int pick_shorter_tile(int M, int N, int nk, int tile, TileRule rule, ShorterTileRule shorter) {
     const long long cus = moe_num_compute_units();
     auto rounds = [&](int tm, int tn, long long capacity) {
