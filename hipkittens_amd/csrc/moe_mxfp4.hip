@@ -79,7 +79,10 @@ __device__ __forceinline__ float glu_act(float g, float u, float alpha, float li
     return (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + __expf(-alpha * g)));
 }
 __device__ __forceinline__ float glu_act(int act, float g, float u, float alpha, float limit) {
-    return act == 0 ? glu_act<false>(g, u, alpha, limit) : glu_act<true>(g, u, alpha, limit);
+    if (act == 0) return silu_mul(g, u);
+    g = fminf(g, limit);
+    u = fminf(fmaxf(u, -limit), limit);
+    return (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + __expf(-alpha * g)));
 }
 
 // MX codes of one row's block of 32 h columns held by the four lanes (r, g = 0..3) of the row: lane (r, g) has columns
