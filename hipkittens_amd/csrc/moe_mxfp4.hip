@@ -922,10 +922,13 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
     constexpr int kScaleLoads = GATHER ? 0 : 1;
     constexpr int kLoads = kPieces + kScaleLoads + 10;   // + 8 weight fragments, 2 weight scale dwords
     constexpr int MT = kBM / 16;
-    // The row fragments of an item that are multiplied under one branch; each of the others has its own. Where an expert has
-    // several items, each holds at least seven fragments of twelve (rows are spread evenly), and a branch between the MFMAs
-    // costs more than the MFMAs of one that holds no rows. Layer, us, 1 / 4 / 6 / 8 of 12: 16384 tokens 1316 / 1279 / 1266 /
-    // 1248, 12175 of 1792 x 2752 (MXFP8) 463 / 452 / 446 / 436, 2583 of 1088 x 3968 208 / 198 / 197 / 191.
+    // The row fragments of an item that are multiplied under one branch; each of the others has its own. Where experts have
+    // several items on the average, most items hold six fragments of twelve or more (an expert's rows are spread evenly over its
+    // items: two items of 193 rows have seven and six; an expert of few rows has one item of any size), and a branch between the
+    // MFMAs costs more than the MFMAs of a fragment that holds no rows. Layer, us, 1 / 4 / 6 / 8 of 12: 16384 tokens 1316 /
+    // 1279 / 1266 / 1248, 12175 of 1792 x 2752 (MXFP8) 463 / 452 / 446 / 436, 2583 of 1088 x 3968 208 / 198 / 197 / 191. Uneven
+    // routing, before these branches and the template parameter of the activation / now: 16384 tokens, 128 experts of 0 to 8044
+    // rows, half of them below 66, 1543 / 1344; 2583 tokens, 32 experts of 0 to 2583 rows, half of them empty, 228 / 205.
     constexpr int kFirst = NT ? 1 : MT * 8 / 12;
     extern __shared__ __attribute__((aligned(2048))) uint8_t smem[];
     const int lane = lane_id(), w = wave_id();
@@ -1313,6 +1316,17 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
         for (int n = 0; n < 4; ++n) acc[M][n] = v4f{0.f, 0.f, 0.f, 0.f};
     };
 
+    // Accumulators of the fragments under one branch, at the end of an item that has fewer (those with rows are clear).
+    auto clear_first = [&]() __attribute__((always_inline)) {
+        asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");   // (the last MFMAs: see epilogue)
+#pragma unroll
+        for (int m = 1; m < kFirst; ++m) {
+            asm volatile("" : "+a"(acc[m][0]), "+a"(acc[m][1]), "+a"(acc[m][2]), "+a"(acc[m][3]));
+#pragma unroll
+            for (int n = 0; n < 4; ++n) acc[m][n] = v4f{0.f, 0.f, 0.f, 0.f};
+        }
+    };
+
     // ---- prologue: positions 0..2 -----------------------------------------------------------------
     fetch_all.template operator()<0>();
     fetch_all.template operator()<1>();
@@ -1414,6 +1428,10 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
         advance_cf();
         if constexpr (P == 3)
             if (last && MT - 1 < mt_item) epilogue.template operator()<MT - 1>(true);
+        // Fragments without rows that shared the branch: their products are zero only while the expert's weight scales are
+        // numbers (0 times an e8m0 NaN is NaN), and the next item, another expert's, must not start from them.
+        if constexpr (P == 3 && kFirst > 1)
+            if (last && mt_item < kFirst) clear_first();
         if (++cc.kt == nk4) {
             // the fetch cursor entered this item three positions ago and is still in it (nk4 >= 4)
             cc = cf; cc.kt = 0;
