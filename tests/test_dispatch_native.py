@@ -65,19 +65,22 @@ _NAMES = ["fp8", "fp8 bytes", "fp8 int scales", "fp8 workspace", "bf16", "bf16 w
           "mxfp4 pitched", "mxfp4 workspace", "quantize"]
 
 
+def _same(a, b):
+    flat = lambda o: [t.view(torch.uint8) for t in (o if isinstance(o, tuple) else (o,))]
+    return all(torch.equal(x, y) for x, y in zip(flat(a), flat(b)))
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", _NAMES)
 def test_same_results_as_the_python_dispatcher(monkeypatch, name):
     fn, args, kw, new = _calls("cuda:0")[name]
     out = [new(), new()]
-    with torch.cuda.stream(torch.cuda.Stream()):   # the current stream, not the default one
-        fn(*args(out[0]), **kw)
-        torch.cuda.current_stream().synchronize()
+    fn(*args(out[0]), **kw)
+    torch.cuda.synchronize()
     _python_only(monkeypatch)
     fn(*args(out[1]), **kw)
     torch.cuda.synchronize()
-    flat = lambda o: [t.view(torch.uint8) for t in (o if isinstance(o, tuple) else (o,))]
-    assert all(torch.equal(a, b) for a, b in zip(flat(out[0]), flat(out[1])))
+    assert _same(out[0], out[1])
     assert not isinstance(out[0], torch.Tensor) or torch.isfinite(out[0].float()).all()
 
 
@@ -99,8 +102,35 @@ def test_refused_as_before():
 
 
 @pytest.mark.gpu
-def test_captured_calls_replay():
-    fn, args, kw, new = _calls("cuda:0")["mxfp4 pitched"]
+@pytest.mark.parametrize("name", _NAMES)
+def test_the_current_stream_is_used(name):
+    """The call waits for what its own stream does to an operand: milliseconds of products, then the operand's final
+    values. On another stream it would see the values from before."""
+    fn, args, kw, new = _calls("cuda:0")[name]
+    outs = [new() for _ in range(3)]   # of the first values, of the final ones, from the side stream
+    a = args(outs[0])[0].view(torch.uint8)
+    first, final = a.clone(), a.flip(0).contiguous()
+    for values, out in zip((first, final), outs):
+        a.copy_(values)
+        fn(*args(out), **kw)
+    a.copy_(first)
+    busy = torch.randn(4096, 4096, device="cuda:0")
+    torch.cuda.synchronize()
+    assert not _same(outs[0], outs[1])
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        for _ in range(8):
+            torch.mm(busy, busy)
+        a.copy_(final)
+        fn(*args(outs[2]), **kw)
+    side.synchronize()
+    assert _same(outs[2], outs[1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", _NAMES)
+def test_captured_calls_replay(name):
+    fn, args, kw, new = _calls("cuda:0")[name]
     want, got = new(), new()
     fn(*args(want), **kw)
     torch.cuda.synchronize()
@@ -108,7 +138,8 @@ def test_captured_calls_replay():
     with torch.cuda.graph(g):
         fn(*args(got), **kw)
     for _ in range(3):
-        got.fill_(float("nan"))
+        for t in got if isinstance(got, tuple) else (got,):
+            t.zero_()
         g.replay()
         torch.cuda.synchronize()
-        assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+        assert _same(got, want)
