@@ -119,8 +119,17 @@ def load_library() -> ctypes.CDLL:
     return lib
 
 
+def dispatch_build_tag() -> str:
+    """What the dispatchers' module is compiled against: its calls into torch and Python are not stable between versions."""
+    import sys
+
+    import torch
+    return f"torch {torch.__version__}, Python {sys.version_info.major}.{sys.version_info.minor}"
+
+
 def load_dispatch():
-    """The dispatchers' CPython module (csrc/dispatch.cpp), bound to the library. Raises RuntimeError if absent."""
+    """The dispatchers' CPython module (csrc/dispatch.cpp), bound to the library. Raises RuntimeError or ImportError where
+    it is absent, built for another torch or Python, or cannot be loaded (tk_kernel then does without it)."""
     global _dispatch
     if _dispatch is not None:
         return _dispatch
@@ -130,6 +139,8 @@ def load_dispatch():
     spec = importlib.util.spec_from_file_location("hipkittens_amd._dispatch", _DISPATCH_PATH)
     module = importlib.util.module_from_spec(spec)
     spec.loader.exec_module(module)
+    if module.build_tag != dispatch_build_tag():
+        raise RuntimeError(f"{_DISPATCH_PATH} is built for {module.build_tag}, this is {dispatch_build_tag()}")
     module.bind(*(ctypes.cast(getattr(lib, "hk_" + name), c_void_p).value for name in _DISPATCH_ENTRIES))
     _dispatch = module
     return module

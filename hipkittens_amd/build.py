@@ -74,7 +74,11 @@ def build(verbose: bool = True, extra_flags: list[str] | None = None, jobs: int 
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
         dispatch = pool.submit(_build_dispatch)
         all_objs = list(pool.map(lambda s: _compile_one(s, extra), sources + bench_sources))
-        dispatch.result()
+        try:
+            dispatch.result()
+        except (RuntimeError, OSError, ImportError) as e:   # g++ or headers missing: the library serves without it
+            DISPATCH_PATH.unlink(missing_ok=True)
+            print(f"{DISPATCH_PATH.name} not built, GEMM calls check their arguments in Python: {e}", file=sys.stderr)
     objs, bench_objs = all_objs[:len(sources)], all_objs[len(sources):]
     _link(objs, LIB_PATH)
     if bench_objs:
@@ -99,10 +103,12 @@ def _build_dispatch() -> None:
 
     from torch.utils import cpp_extension
 
+    from . import _lib
+
     tmp = DISPATCH_PATH.with_suffix(".so.tmp")
     lib_dirs = cpp_extension.library_paths()
     cmd = [shutil.which("g++") or "g++", "-O2", "-std=c++20", "-fPIC", "-shared", "-fvisibility=hidden", "-DUSE_ROCM",
-           "-D__HIP_PLATFORM_AMD__", *(f"-isystem{d}" for d in cpp_extension.include_paths()), "-isystem/opt/rocm/include",
+           "-D__HIP_PLATFORM_AMD__", f'-DHK_BUILD_TAG="{_lib.dispatch_build_tag()}"', *(f"-isystem{d}" for d in cpp_extension.include_paths()), "-isystem/opt/rocm/include",
            f"-isystem{sysconfig.get_paths()['include']}", str(CSRC / "dispatch.cpp"), "-o", str(tmp),
            *(f"-L{d}" for d in lib_dirs), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
     res = subprocess.run(cmd, capture_output=True, text=True)

@@ -7,7 +7,8 @@
 //
 // Every function returns the library's status, or None where an argument is not what it knows (another type or device, a
 // shape that does not fit, a subclass or a wrapper of a transform): the Python dispatcher then runs its own checks, which
-// accept or refuse the call with their messages. No call is refused here.
+// accept or refuse the call with their messages. No call is refused here. The module is not a condition either: where it is
+// absent or built for another torch or Python (build_tag), every call is left to the Python dispatchers.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -197,5 +198,7 @@ PyMODINIT_FUNC PyInit__dispatch(void) {
     Py_DECREF(nn);
     if (!parameter) return nullptr;
     parameter_type = reinterpret_cast<PyTypeObject*>(parameter);   // (kept for the life of the process)
-    return PyModule_Create(&module_def);
+    PyObject* module = PyModule_Create(&module_def);
+    if (module && PyModule_AddStringConstant(module, "build_tag", HK_BUILD_TAG) < 0) Py_CLEAR(module);
+    return module;
 }

@@ -11,6 +11,8 @@ stream (the reference uses the null stream).
 """
 from __future__ import annotations
 
+import warnings
+
 import torch
 
 from . import _lib
@@ -45,9 +47,25 @@ _FP8 = (torch.float8_e4m3fn, torch.uint8)
 _native = None
 
 
+class _NoNative:
+    """In the place of the native dispatchers where their module cannot be loaded: leaves every call to the Python ones."""
+
+    @staticmethod
+    def fp8_gemm(*_):
+        return None
+
+    bf16_gemm = mxfp4_gemm = mxfp4_quantize_rows = fp8_gemm
+
+
 def _load_native():
     global _native
-    _native = _lib.load_dispatch()
+    if not _lib.lib_path().exists():
+        return _NoNative   # (the Python dispatcher says so, behind its checks)
+    try:
+        _native = _lib.load_dispatch()
+    except (RuntimeError, ImportError) as e:
+        warnings.warn(f"GEMM calls check their arguments in Python, 3 to 6 us a call more: {e}", RuntimeWarning, stacklevel=3)
+        _native = _NoNative
     return _native
 
 

@@ -1,5 +1,8 @@
 """The native dispatchers (csrc/dispatch.cpp): they take what the Python dispatchers take, leave the rest to them, and give
 the same results."""
+import warnings
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -30,11 +33,33 @@ def test_cpu_tensors_and_wrong_types_are_left_to_python():
         tk.dispatch_fp8_gemm([1], u, c)
 
 
-def _python_only(monkeypatch):
-    class Off:
-        def __getattr__(self, name):
-            return lambda *args: None
-    monkeypatch.setattr(tk, "_native", Off())
+def _python_only(monkeypatch, path="/nonexistent/_dispatch.so"):
+    monkeypatch.setattr(_lib, "_DISPATCH_PATH", Path(path))
+    monkeypatch.setattr(_lib, "_dispatch", None)
+    monkeypatch.setattr(tk, "_native", None)
+
+
+@pytest.mark.parametrize("how", ["absent", "not a module", "another torch"])
+def test_without_the_module_the_python_dispatchers_take_every_call(monkeypatch, tmp_path, how):
+    """What the module does not load for (it is missing, broken, or compiled against another torch) is no call's failure."""
+    _needs_build()
+    built = _lib._DISPATCH_PATH
+    (tmp_path / "_dispatch.so").write_text("no shared object")
+    _python_only(monkeypatch, {"absent": tmp_path / "none.so", "not a module": tmp_path / "_dispatch.so"}.get(how, built))
+    if how == "another torch":
+        monkeypatch.setattr(torch, "__version__", "0.1")
+    with pytest.raises((RuntimeError, ImportError)):
+        _lib.load_dispatch()
+    a, c = torch.zeros(4, 64, dtype=torch.bfloat16), torch.zeros(4, 4, dtype=torch.bfloat16)
+    u = torch.zeros(4, 64, dtype=torch.uint8)
+    calls = [lambda: tk.dispatch_bf16_gemm(a, a, c), lambda: tk.dispatch_fp8_gemm(u, u, c),
+             lambda: tk.dispatch_mxfp4_gemm(u, u, u, u, c), lambda: tk.dispatch_mxfp4_quantize_rows(a, u, u)]
+    for i, call in enumerate(calls):
+        with warnings.catch_warnings(record=True) as said:
+            warnings.simplefilter("always")
+            with pytest.raises(RuntimeError, match="GPU device"):   # the Python dispatcher's own check
+                call()
+        assert [w.category for w in said] == ([RuntimeWarning] if i == 0 else [])   # said once
 
 
 def _calls(dev):
@@ -78,7 +103,8 @@ def test_same_results_as_the_python_dispatcher(monkeypatch, name):
     fn(*args(out[0]), **kw)
     torch.cuda.synchronize()
     _python_only(monkeypatch)
-    fn(*args(out[1]), **kw)
+    with pytest.warns(RuntimeWarning, match="in Python"):
+        fn(*args(out[1]), **kw)
     torch.cuda.synchronize()
     assert _same(out[0], out[1])
     assert not isinstance(out[0], torch.Tensor) or torch.isfinite(out[0].float()).all()
