@@ -278,15 +278,18 @@ extern "C" int hk_bf16_gemm_variant(const void* A, const void* B, void* C, int M
     return bf16_gemm_impl(A, B, C, M, N, K, variant > 6 ? -1 : variant, stream);
 }
 
+extern "C" int hk_bf16_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K, int tile, void* stream) {
+    return bf16_gemm_impl(A, B, C, M, N, K, hk::variant_of_tile(tile, 1, 2, 3), stream);
+}
+
 extern "C" int hk_bf16_gemm(const void* A, const void* B, void* C, int M, int N, int K, void* stream) {
     using namespace hk;
     if (gemm_dims_too_large(M, N, K)) return HK_ERR_BAD_SHAPE;
     const bool tile_ok = K > 0 && (long long)2 * K * BM < (1ll << 31);
-    // the same choice of tile as hk_fp8_gemm (pick_tile), with this format's measured corrections
-    const int tile = pick_tile(kFmtBf16, M, N, (int)((2ll * K + BK - 1) / BK), kTileRuleBf16);
+    // the same choice of tile as hk_fp8_gemm, with this format's measured corrections
+    const int tile = pick_gemm_tile(kFmtBf16, M, N, (int)((2ll * K + BK - 1) / BK));
     const bool skinny = tile_ok && use_skinny(M, N, (int)((2ll * K + BK - 1) / BK), false, moe_num_compute_units());
-    const int shorter = pick_shorter_tile(M, N, (int)((2ll * K + BK - 1) / BK), tile, kTileRuleBf16, kShorterTileBf16);
-    const int variant = !tile_ok ? 0 : skinny ? 6 : shorter ? shorter : tile == kTinyTile ? 3 : tile == kSmallTile ? 2 : 1;
+    const int variant = !tile_ok ? 0 : skinny ? 6 : tile > BM ? tile : tile == kTinyTile ? 3 : tile == kSmallTile ? 2 : 1;
     return bf16_gemm_impl(A, B, C, M, N, K, variant, stream);
 }
 

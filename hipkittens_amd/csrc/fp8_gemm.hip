@@ -259,6 +259,11 @@ extern "C" int hk_fp8_gemm_variant(const void* A, const void* B, void* C, int M,
     return fp8_gemm_impl(A, B, C, M, N, K, scale_a, scale_b, variant > 8 ? -1 : variant, stream);
 }
 
+extern "C" int hk_fp8_gemm_tile(const void* A, const void* B, void* C, int M, int N, int K, float scale_a, float scale_b,
+                                int tile, void* stream) {
+    return fp8_gemm_impl(A, B, C, M, N, K, scale_a, scale_b, hk::variant_of_tile(tile, 4, 5, 6), stream);
+}
+
 extern "C" size_t hk_fp8_gemm_workspace_bytes(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0 || hk::gemm_dims_too_large(M, N, K)) return 0;
     const int s = hk::splitk_ranges(M, N, K);
@@ -335,24 +340,37 @@ extern "C" int hk_fp8_gemm_static_ws(const void* A, const void* B, void* C, int 
     return hk_fp8_gemm_ws(A, B, C, M, N, K, scale_a, scale_b, ws, kStaticScratchBytes, stream);
 }
 
+// K-steps of a shape (128 bytes of an operand row each); 0: no such shape.
+static int tile_k_steps(int format, int M, int N, int K) {
+    using namespace hk;
+    if (format < 0 || format > 2 || M <= 0 || N <= 0 || K <= 0 || gemm_dims_too_large(M, N, K)) return 0;
+    const long long row_bytes = format == kFmtFp8 ? K : format == kFmtBf16 ? 2ll * K : K / 2;
+    return (int)((row_bytes + BK - 1) / BK);
+}
+
 extern "C" int hk_gemm_tile_choice(int format, int M, int N, int K, int consult_table) {
     using namespace hk;
-    if (format < 0 || format > 2 || M <= 0 || N <= 0 || K <= 0 || gemm_dims_too_large(M, N, K)) return HK_ERR_BAD_SHAPE;
-    const long long row_bytes = format == kFmtFp8 ? K : format == kFmtBf16 ? 2ll * K : K / 2;
-    const int nk = (int)((row_bytes + BK - 1) / BK);
-    const TileRule rule = format == kFmtFp8 ? kTileRuleFp8 : format == kFmtBf16 ? kTileRuleBf16 : kTileRuleMxfp4;
-    return pick_tile(format, M, N, nk, rule, consult_table != 0);
+    const int nk = tile_k_steps(format, M, N, K);
+    if (!nk) return HK_ERR_BAD_SHAPE;
+    const int listed = consult_table ? table_tile(format, M, N, nk) : 0;
+    return listed == BM || listed == kSmallTile || listed == kTinyTile ? listed
+                                                                      : pick_tile_rule(M, N, nk, kTileRules[format], moe_num_compute_units());
 }
 
 extern "C" int hk_gemm_shorter_tile(int format, int M, int N, int K) {
     using namespace hk;
-    if (format < 0 || format > 2 || M <= 0 || N <= 0 || K <= 0 || gemm_dims_too_large(M, N, K)) return HK_ERR_BAD_SHAPE;
-    const long long row_bytes = format == kFmtFp8 ? K : format == kFmtBf16 ? 2ll * K : K / 2;
-    const int nk = (int)((row_bytes + BK - 1) / BK);
-    const TileRule rule = format == kFmtFp8 ? kTileRuleFp8 : format == kFmtBf16 ? kTileRuleBf16 : kTileRuleMxfp4;
-    const ShorterTileRule sr = format == kFmtFp8 ? kShorterTileFp8 : format == kFmtBf16 ? kShorterTileBf16 : kShorterTileMxfp4;
-    const int v = pick_shorter_tile(M, N, nk, pick_tile(format, M, N, nk, rule), rule, sr);
+    const int nk = tile_k_steps(format, M, N, K);
+    if (!nk) return HK_ERR_BAD_SHAPE;
+    const int v = pick_gemm_tile(format, M, N, nk);
     return v == kVariant192x256 ? 1 : v == kVariant256x192 ? 2 : 0;
+}
+
+extern "C" int hk_gemm_tile_shape(int format, int M, int N, int K, int consult_table) {
+    using namespace hk;
+    const int nk = tile_k_steps(format, M, N, K);
+    if (!nk) return HK_ERR_BAD_SHAPE;
+    const int v = pick_gemm_tile(format, M, N, nk, consult_table != 0);
+    return v > BM ? v : 1001 * v;   // (256 -> 256256)
 }
 
 extern "C" int hk_fp8_gemm(const void* A, const void* B, void* C, int M, int N, int K,
@@ -360,11 +378,10 @@ extern "C" int hk_fp8_gemm(const void* A, const void* B, void* C, int M, int N, 
     using namespace hk;
     if (gemm_dims_too_large(M, N, K)) return HK_ERR_BAD_SHAPE;
     const bool tile_ok = K > 0 && (long long)K * BM < (1ll << 31);
-    // 256x256 tiles (five-slot ring kernel), 128x128 or 64x64: see pick_tile
-    const int tile = pick_tile(kFmtFp8, M, N, (K + BK - 1) / BK, kTileRuleFp8);
+    // see pick_gemm_tile
+    const int tile = pick_gemm_tile(kFmtFp8, M, N, (K + BK - 1) / BK);
     // few rows: one pass over B by the skinny kernel where that is faster (use_skinny)
     const bool skinny = tile_ok && use_skinny(M, N, (K + BK - 1) / BK, false, moe_num_compute_units());
-    const int shorter = pick_shorter_tile(M, N, (K + BK - 1) / BK, tile, kTileRuleFp8, kShorterTileFp8);
-    const int variant = !tile_ok ? 0 : skinny ? 8 : shorter ? shorter : tile == kTinyTile ? 6 : tile == kSmallTile ? 5 : 4;
+    const int variant = !tile_ok ? 0 : skinny ? 8 : tile > BM ? tile : tile == kTinyTile ? 6 : tile == kSmallTile ? 5 : 4;
     return fp8_gemm_impl(A, B, C, M, N, K, scale_a, scale_b, variant, stream);
 }

@@ -342,9 +342,14 @@ static __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* 
     }
 }
 
-// Which tile a GEMM gets when the caller does not pin a kernel: 256 (the large-tile kernels), 128 or
-// 64. Two layers:
-//  1. a rule: the tile with the smallest estimated time. A tile kernel's workgroups run in rounds over the
+// Which tile a GEMM gets when the caller does not pin a kernel (pick_gemm_tile): 256, 128 or 64 square, or one of the ring
+// kernel's 192x256 and 256x192. A table, then a rule in two steps:
+//  1. a generated table of the shapes on which a sweep found the rule's choice more than a few percent behind
+//     another tile (tile_table.inc, written by `python -m hipkittens_amd.tile_sweep FORMAT --emit`; the
+//     counterpart of the reference's per-shape analysis/baselines/gemm/utils/tuned.yaml). An entry is keyed by
+//     the format, the numbers of 64-row / 64-column blocks of M and N and the K-step count, applies on
+//     devices with the CU count the sweep ran on, and is final: it corrects the rule's estimates, so they do not judge it again;
+//  2. the square tile with the smallest estimated time (pick_tile_rule). A tile kernel's workgroups run in rounds over the
 //     device's CUs (one workgroup per CU for the 256- and 128-tiles, two for the 64-tile), every round costs
 //     the same whether it is full or not, and a workgroup's time is a fixed part (prologue, epilogue, launch)
 //     plus a part per K-step:  time = ceil(tiles / (CUs x workgroups per CU)) x (fixed + per_step x K-steps).
@@ -352,21 +357,16 @@ static __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* 
 //     enter only through their ratios, the CU count through the rounds). This captures what a threshold on the
 //     tile count cannot: 72 tiles of 256 are one round where their 288 tiles of 128 are two (the large tile
 //     wins by 4-12 % from a K of about 4096 elements on), 64 tiles of 256 are one round of four times the work
-//     of the single round of 256 small tiles (the small tile wins by 60 %). Measured against the best of the
-//     three kernels, every launch on another copy of B (a model's weights come from HBM, not from the memory-side
-//     cache), the rule alone is more than 5 % behind on 7 / 6 of 414 shapes (FP8 / BF16; 42 / 40 with the constants
-//     that fitted these kernels before their loads and LDS reads were spread over the MFMAs) and on 5 of 414 (MXFP4; 16 with
-//     the constants from before the scaled kernel's scale loads went from every K-step to every second);
-//  2. a generated table of the shapes on which a sweep found the rule's choice more than a few percent behind
-//     another tile (tile_table.inc, written by `python -m hipkittens_amd.tile_sweep FORMAT --emit`; the
-//     counterpart of the reference's per-shape analysis/baselines/gemm/utils/tuned.yaml). An entry is keyed by
-//     the format, the numbers of 64-row / 64-column blocks of M and N and the K-step count, and applies on
-//     devices with the CU count the sweep ran on.
+//     of the single round of 256 small tiles (the small tile wins by 60 %);
+//  3. a shorter tile in its place where that is estimated faster (pick_shorter_tile).
+// Measured against the best of the five kernels, every launch on another copy of B (a model's weights come from HBM, not from
+// the memory-side cache), the rule alone is more than 5 % behind on 36 / 16 / 21 of the sweep's 414 shapes (FP8 / BF16 /
+// MXFP4), with the table on 0 / 1 / 1, and on 24 / 37 / 9 of 450 shapes drawn between the sweep's points.
 struct TileRule {
     float fixed[3], per_step[3];   // 256-, 128-, 64-tile
 };
 enum TileFormat { kFmtFp8 = 0, kFmtBf16 = 1, kFmtMxfp4 = 2 };
-struct TileTableEntry { unsigned char fmt; unsigned short m64, n64, nk, tile; };
+struct TileTableEntry { unsigned char fmt; unsigned short m64, n64, nk; int tile; };
 #include "tile_table.inc"   // kTileTableCus, kTileTable[]
 
 int moe_num_compute_units();  // number of CUs of the current device, cached (moe_mxfp4.hip)
@@ -384,33 +384,35 @@ static inline int pick_tile_rule(int M, int N, int nk, TileRule r, int cus) {
     }
     return tile[best];
 }
-static inline int pick_tile(int fmt, int M, int N, int nk, TileRule r, bool consult_table = true) {
-    const int cus = moe_num_compute_units();   // 256 when no device can be queried
-    if (consult_table && cus == kTileTableCus) {
-        const long long m64 = ((long long)M + 63) / 64, n64 = ((long long)N + 63) / 64;
-        for (const TileTableEntry& e : kTileTable)
-            if (e.fmt == fmt && e.m64 == m64 && e.n64 == n64 && e.nk == nk) return e.tile;
-    }
-    return pick_tile_rule(M, N, nk, r, cus);
+// The table's entry for a shape: 256, 128, 64 or one of the ring kernel's shorter tiles; 0: none.
+static inline int table_tile(int fmt, int M, int N, int nk) {
+    if (moe_num_compute_units() != kTileTableCus) return 0;   // (256 when no device can be queried)
+    const long long m64 = ((long long)M + 63) / 64, n64 = ((long long)N + 63) / 64;
+    for (const TileTableEntry& e : kTileTable)
+        if (e.fmt == fmt && e.m64 == m64 && e.n64 == n64 && e.nk == nk) return e.tile;
+    return 0;
 }
 // the formats' constants (K-steps: 128 bytes of an operand row)
-constexpr TileRule kTileRuleFp8{{7.10f, 3.28f, 2.02f}, {1.060f, 0.533f, 0.385f}};
-constexpr TileRule kTileRuleBf16{{8.57f, 2.79f, 2.20f}, {0.983f, 0.495f, 0.336f}};
-constexpr TileRule kTileRuleMxfp4{{7.51f, 3.07f, 1.185f}, {1.316f, 0.710f, 0.587f}};
+constexpr TileRule kTileRules[3] = {{{7.10f, 3.28f, 2.02f}, {1.060f, 0.533f, 0.385f}},      // FP8
+                                    {{8.57f, 2.79f, 2.20f}, {0.983f, 0.495f, 0.336f}},      // BF16
+                                    {{7.51f, 3.07f, 1.185f}, {1.316f, 0.710f, 0.587f}}};    // MXFP4
 
-// The ring kernel's shorter tiles (gemm_ring.h): 192x256 or 256x192 in the place of the tile that pick_tile names, where
+// The ring kernel's shorter tiles (gemm_ring.h): 192x256 or 256x192 in the place of the rule's square tile, where
 // the same cost model, one workgroup per CU, gives them less time. The constants, and the factor on the estimate for a
 // 128- or 64-tile (which is high where it is compared with these), are fitted to 91 shapes per format on an MI355X
-// (M 500 ... 8192, (N, K) 4096 x 4096 ... 14336 x 4096, 2880 x 2880, 10000 x 1024, copies of B in rotation): no shape
-// is more than 3 % behind what it had, and the geometric mean falls by 5.5 (FP8), 6.3 (BF16) and 6.3 % (MXFP4), of 6.5,
-// 6.9 and 7.0 that the best kernel for every shape would give (MXFP4 as first fitted; fitted again to 112 shapes when its
-// small-tile kernels became faster: 3 more than 5 % behind the best kernel, before 4). Examples, us before / after: BF16 3001 x 4096 x 4096
-// 90.1 / 74.9 (192 tiles of 256x256 against 256 of 192x256), 4096 x 2880 x 2880 69.2 / 54.1; FP8 8192 x 2880 x 2880
-// 71.8 / 58.6; MXFP4 4096 x 2880 x 2880 35.2 / 27.8; and not taken: BF16 4096 x 4096 x 4096 96.3 / 130.9 (256 tiles of
-// 256x256, one round; 352 of 192x256, two).
-constexpr int kVariant192x256 = 100, kVariant256x192 = 101;   // the GEMM entry points' internal numbers for them
+// (M 500 ... 8192, (N, K) 4096 x 4096 ... 14336 x 4096, 2880 x 2880, 10000 x 1024, copies of B in rotation; MXFP4 again to 112
+// when its small-tile kernels became faster). Over the 414 shapes of the sweep and 450 drawn ones a shorter tile is more than 3 %
+// behind the square one on 5 / 1 / 5 (FP8 / BF16 / MXFP4; those of the sweep are in the table), and the geometric mean of the
+// drawn ones falls by 1.1 / 1.4 / 1.7 %, of 1.8 / 2.2 / 2.0 that the best kernel for every shape would give. (A fit to all of
+// them, {6.84, 0.882, 0.882}, {6.75, 0.816, 0.881}, {6.73, 1.07, 0.873}, gained 4 % where FP8 and BF16 choose otherwise with it, but
+// lost up to 14 % on single shapes, 0.6 % on the average for MXFP4.) Examples, us before /
+// after: BF16 3001 x 4096 x 4096 90.1 / 74.9 (192 tiles of 256x256 against 256 of 192x256), 4096 x 2880 x 2880 69.2 / 54.1; FP8
+// 8192 x 2880 x 2880 71.8 / 58.6; MXFP4 4096 x 2880 x 2880 35.2 / 27.8; and not taken: BF16 4096 x 4096 x 4096 96.3 / 130.9
+// (256 tiles of 256x256, one round; 352 of 192x256, two). Equal estimates go to 256x192: with the one that pads less instead, 5
+// more shapes of FP8 and 16 of BF16 are behind.
+constexpr int kVariant192x256 = 192256, kVariant256x192 = 256192;   // the GEMM entry points' internal numbers for them
 struct ShorterTileRule { float fixed, per_step, small; };
-constexpr ShorterTileRule kShorterTileFp8{5.7f, 0.87f, 0.82f}, kShorterTileBf16{5.6f, 0.925f, 0.94f}, kShorterTileMxfp4{7.37f, 1.057f, 0.974f};
+constexpr ShorterTileRule kShorterTileRules[3] = {{5.7f, 0.87f, 0.82f}, {5.6f, 0.925f, 0.94f}, {7.37f, 1.057f, 0.974f}};
 static inline int pick_shorter_tile(int M, int N, int nk, int tile, TileRule rule, ShorterTileRule shorter) {
     const long long cus = moe_num_compute_units();
     auto rounds = [&](int tm, int tn, long long capacity) {
@@ -424,6 +426,21 @@ static inline int pick_shorter_tile(int M, int N, int nk, int tile, TileRule rul
     const double t0 = rounds(192, 256, cus) * one, t1 = rounds(256, 192, cus) * one;
     if ((t0 < t1 ? t0 : t1) > now) return 0;
     return t0 < t1 ? kVariant192x256 : kVariant256x192;
+}
+// The tile kernel of a shape: 256, 128, 64, kVariant192x256 or kVariant256x192. A measured entry of the table is final.
+static inline int pick_gemm_tile(int fmt, int M, int N, int nk, bool consult_table = true) {
+    const int listed = consult_table ? table_tile(fmt, M, N, nk) : 0;
+    if (listed) return listed;
+    const TileRule& rule = kTileRules[fmt];
+    const int square = pick_tile_rule(M, N, nk, rule, moe_num_compute_units());
+    const int shorter = pick_shorter_tile(M, N, nk, square, rule, kShorterTileRules[fmt]);
+    return shorter ? shorter : square;
+}
+
+// The GEMM entry points' variant number for a tile as hk_gemm_tile_shape names it (rows * 1000 + columns); -1: there is none.
+static inline int variant_of_tile(int tile, int v256, int v128, int v64) {
+    return tile == kVariant192x256 || tile == kVariant256x192 ? tile
+           : tile == 256256 ? v256 : tile == 128128 ? v128 : tile == 64064 ? v64 : -1;
 }
 
 // Number of K ranges the split-K path would use: as many as fill the CUs, each at least 4

@@ -588,10 +588,9 @@ static int mxfp4_gemm_impl(const void* A, const void* A_scales, int sa_pitch, co
     const Mxfp4ScaleRows sr = mxfp4_scale_rows(K, sa_pitch, sb_pitch);
     const bool size_ok = (long long)(K / 2) * BM < (1ll << 31) && (long long)BM * max(sa_pitch, sb_pitch) < (1ll << 31);
     if (variant < 0) {
-        // the choice of tile of hk_fp8_gemm (pick_tile); a K-step is 256 elements here
-        const int tile = pick_tile(kFmtMxfp4, M, N, (K / 2 + BK - 1) / BK, kTileRuleMxfp4);
-        const int shorter = pick_shorter_tile(M, N, (K / 2 + BK - 1) / BK, tile, kTileRuleMxfp4, kShorterTileMxfp4);
-        variant = !(sr.ok && size_ok) ? 0 : shorter ? shorter : tile == kTinyTile ? 3 : tile == kSmallTile ? 2 : 1;
+        // the choice of tile of hk_fp8_gemm; a K-step is 256 elements here
+        const int tile = pick_gemm_tile(kFmtMxfp4, M, N, (K / 2 + BK - 1) / BK);
+        variant = !(sr.ok && size_ok) ? 0 : tile > BM ? tile : tile == kTinyTile ? 3 : tile == kSmallTile ? 2 : 1;
         // few rows: one pass over B by the skinny kernel where that is faster (use_skinny); it takes any scale rows
         if (size_ok && use_skinny(M, N, (K / 2 + BK - 1) / BK, false, moe_num_compute_units(), kSkinnyMaxMScaled, 2)) variant = 6;
     }
@@ -642,6 +641,12 @@ extern "C" int hk_mxfp4_gemm_variant(const void* A, const void* A_scales, const 
                                      void* stream) {
     return variant < 0 ? HK_ERR_UNSUPPORTED
                        : mxfp4_gemm_impl(A, A_scales, K / 32, B, B_scales, K / 32, C, M, N, K, variant > 6 ? -2 : variant, stream);
+}
+
+extern "C" int hk_mxfp4_gemm_tile(const void* A, const void* A_scales, int a_scale_pitch, const void* B, const void* B_scales,
+                                  int b_scale_pitch, void* C, int M, int N, int K, int tile, void* stream) {
+    const int v = hk::variant_of_tile(tile, 1, 2, 3);
+    return mxfp4_gemm_impl(A, A_scales, a_scale_pitch, B, B_scales, b_scale_pitch, C, M, N, K, v < 0 ? -2 : v, stream);
 }
 
 extern "C" int hk_mxfp4_gemm(const void* A, const void* A_scales, const void* B, const void* B_scales,

@@ -4,21 +4,25 @@ and writes the per-shape table that the library's choice of tile consults.
     python -m hipkittens_amd.tile_sweep fp8|bf16|mxfp4            report on the 110-shape grid
     python -m hipkittens_amd.tile_sweep fp8|bf16|mxfp4 --emit     sweep the larger grid, rewrite the format's
                                                                   entries of csrc/tile_table.inc, then rebuild
+    python -m hipkittens_amd.tile_sweep fp8|bf16|mxfp4 --draw N   report on N drawn shapes (what a rule fitted to a
+                                                                  grid does between the grid's points)
 
 For each shape it prints the GPU time (a HIP graph of 20 launches between two events, the launches rotating
 over copies of B that exceed the memory-side cache, as a model's weights do; best of three replays, in two passes over the kernels, forwards and backwards) of the default choice (variant -1; with at
 most 64 rows of A that can be the skinny kernel, csrc/gemm_skinny.h, instead of a tile kernel), of the 256x256,
-128x128 and 64x64 tile kernels, and of the call with a workspace where the library would split K without the
-skinny kernel, and marks the shapes where the default is more than 5 % behind the best tile kernel.
+128x128, 64x64, 192x256 and 256x192 tile kernels, and of the call with a workspace where the library would split K
+without the skinny kernel, and marks the shapes where the default is more than 5 % behind the best tile kernel.
 
-The choice of tile (`pick_tile`, csrc/gemm_small_tile.h) is a rule plus a generated table of exceptions,
+The choice of tile (`pick_gemm_tile`, csrc/gemm_small_tile.h) is a rule plus a generated table of exceptions,
 the counterpart of the reference's tuned.yaml (analysis/baselines/gemm/utils/tuned.yaml: one tuned solution
-per shape). `--emit` measures the three tile kernels on every shape of the larger grid and records the
-shapes where the rule's choice (`hk_gemm_tile_choice(..., consult_table=0)`) is more than 3 % slower than
+per shape). `--emit` measures the five tile kernels on every shape of the larger grid and records the
+shapes where the rule's choice (`hk_gemm_tile_shape(..., consult_table=0)`) is more than 3 % slower than
 the fastest tile, keyed as the library looks them up: format, ceil(M / 64), ceil(N / 64), K-steps. The
 table applies on devices with the CU count it was measured on; run it again after changing a tile kernel
 or on another device, and rebuild the library.
 """
+import math
+import random
 import re
 import sys
 from pathlib import Path
@@ -86,25 +90,43 @@ def _problem(fmt, M, N, K, dev):
             return items[turn[0]]
         return nxt
 
+    lib = _lib.load_library()
+
+    def pinned(st):
+        _lib.check(st, "tile_sweep")
+
     if fmt == "fp8":
         A = torch.randn(M, K, device=dev).to(torch.float8_e4m3fn)
         B = rotating([torch.randn(N, K, device=dev).to(torch.float8_e4m3fn) for _ in range(_copies(N * K))])
-        return (lambda v, ws=None: tk.dispatch_fp8_gemm(A, B(), C, 1.0, 1.0, variant=v, workspace=ws),
-                tk.fp8_gemm_workspace_bytes(M, N, K))
+
+        def run(tile=None, ws=None):
+            if tile is None:
+                return tk.dispatch_fp8_gemm(A, B(), C, 1.0, 1.0, workspace=ws)
+            pinned(lib.hk_fp8_gemm_tile(A.data_ptr(), B().data_ptr(), C.data_ptr(), M, N, K, 1.0, 1.0, tile, tk._stream(A)))
+
+        return run, tk.fp8_gemm_workspace_bytes(M, N, K)
     if fmt == "bf16":
         A = torch.randn(M, K, device=dev, dtype=torch.bfloat16)
         B = rotating([torch.randn(N, K, device=dev, dtype=torch.bfloat16) for _ in range(_copies(2 * N * K))])
-        return (lambda v, ws=None: tk.dispatch_bf16_gemm(A, B(), C, variant=v, workspace=ws),
-                tk.bf16_gemm_workspace_bytes(M, N, K))
+
+        def run(tile=None, ws=None):
+            if tile is None:
+                return tk.dispatch_bf16_gemm(A, B(), C, workspace=ws)
+            pinned(lib.hk_bf16_gemm_tile(A.data_ptr(), B().data_ptr(), C.data_ptr(), M, N, K, tile, tk._stream(A)))
+
+        return run, tk.bf16_gemm_workspace_bytes(M, N, K)
     A = torch.randint(0, 256, (M, K // 2), dtype=torch.uint8, device=dev)
     As = torch.randint(120, 130, (M, K // 32), dtype=torch.uint8, device=dev)
     B = rotating([(torch.randint(0, 256, (N, K // 2), dtype=torch.uint8, device=dev),
                    torch.randint(120, 130, (N, K // 32), dtype=torch.uint8, device=dev))
                   for _ in range(_copies(N * (K // 2 + K // 32)))])
 
-    def run(v, ws=None):
+    def run(tile=None, ws=None):
         b, bs = B()
-        tk.dispatch_mxfp4_gemm(A, As, b, bs, C, variant=v, workspace=ws)
+        if tile is None:
+            return tk.dispatch_mxfp4_gemm(A, As, b, bs, C, workspace=ws)
+        pinned(lib.hk_mxfp4_gemm_tile(A.data_ptr(), As.data_ptr(), K // 32, b.data_ptr(), bs.data_ptr(), K // 32, C.data_ptr(),
+                                      M, N, K, tile, tk._stream(A)))
 
     return run, tk.mxfp4_gemm_workspace_bytes(M, N, K)
 
@@ -125,8 +147,9 @@ def _write_table(fmt, entries, cus):
     rows = sorted(set(kept) | {(code,) + e for e in entries})
     lines = [
         "// Generated by `python -m hipkittens_amd.tile_sweep FORMAT --emit` (one run per format; each run rewrites its",
-        "// format's entries). Shapes on which the rule of pick_tile (gemm_small_tile.h) was measured more than 3 % behind",
-        "// another tile kernel: {format, ceil(M / 64), ceil(N / 64), K-steps, tile}.",
+        "// format's entries). Shapes on which the rule of pick_gemm_tile (gemm_small_tile.h) was measured more than 3 % behind",
+        "// another tile kernel: {format, ceil(M / 64), ceil(N / 64), K-steps, tile}; 192256 and 256192: the ring kernel's shorter",
+        "// tiles.",
         f"constexpr int kTileTableCus = {cus};   // CU count of the device the sweeps ran on",
         "static const TileTableEntry kTileTable[] = {",
         "    {255, 0, 0, 0, 0},   // (keeps the array non-empty)",
@@ -137,58 +160,90 @@ def _write_table(fmt, entries, cus):
     return len(rows)
 
 
+# the tile kernels as hk_gemm_tile_shape names them: rows * 1000 + columns
+TILES = (256256, 128128, 64064, 192256, 256192)
+
+
+def _table_tile(tile):
+    """A tile as the table names it: 256, 128 and 64 for the square ones."""
+    return tile % 1000 if tile // 1000 == tile % 1000 else tile
+
+
+def _drawn(n, rng):
+    """Shapes over the range of the grids, log-uniform, in whole multiples of 64 columns and 128 elements of K mostly."""
+    log = lambda lo, hi: int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+    while n:
+        M, N, K = log(1, 8192), -(-log(512, 65536) // 64) * 64, -(-log(512, 16384) // 128) * 128
+        N -= rng.choice((0, 0, 0, 16, 40))
+        if M * N * K <= 6144 ** 3 and N * K <= 5e8:
+            n -= 1
+            yield M, N, K
+
+
+def measure(run):
+    """GPU time, us, of the default choice (None) and of every tile kernel. Every kernel is timed in two passes, the second
+    in reverse order, and the faster one counts: single timings of one and the same kernel differ by 2-6 % with their
+    position in the sequence (cold operands first, a warm chip last)."""
+    order = (None,) + TILES
+    t = {v: _time_us(lambda: run(v)) for v in order}
+    for v in reversed(order):
+        t[v] = min(t[v], _time_us(lambda: run(v)))
+    return t
+
+
+def _entries(measured):
+    """Table entries from [(key, the rule's tile, {tile: us})]. A key stands for every shape with the same counts of blocks and
+    K-steps (16 and 64 rows among them): it is listed where the rule is behind by the margin on one of its shapes, with the
+    tile that is, and only if that tile is not the slower one on another."""
+    by_key = {}
+    for key, rule, t in measured:
+        by_key.setdefault(key, []).append((rule, t))
+    out = set()
+    for key, shapes in by_key.items():
+        rule, t = max(shapes, key=lambda s: s[1][s[0]] / min(s[1].values()))
+        best = min(t, key=t.get)
+        if t[rule] > EMIT_MARGIN * t[best] and all(s[best] <= 1.01 * s[r] for r, s in shapes):
+            out.add(key + (_table_tile(best),))
+    return out
+
+
 def main(argv):
     args = [a for a in argv[1:] if not a.startswith("--")]
     flags = [a for a in argv[1:] if a.startswith("--")]
-    if len(args) != 1 or args[0] not in FORMATS or any(f != "--emit" for f in flags):
+    draw = int(args.pop()) if flags == ["--draw"] and len(args) == 2 else 0
+    if len(args) != 1 or args[0] not in FORMATS or flags not in ([], ["--emit"], ["--draw"]) or (flags == ["--draw"]) != (draw > 0):
         print(__doc__)
         return 2
     if not torch.cuda.is_available():
         raise RuntimeError("tile_sweep needs a GPU")
     fmt, dev, emit = args[0], "cuda:0", "--emit" in flags
     lib = _lib.load_library()
-    tiles = {"fp8": (4, 5, 6), "bf16": (1, 2, 3), "mxfp4": (1, 2, 3)}[fmt]   # 256, 128, 64
-    size_of = dict(zip(tiles, (256, 128, 64)))
-    behind = total = 0
-    entries = set()
-    for M in (M_GRID_EMIT if emit else M_GRID):
-        for N, K in (NK_GRID_EMIT if emit else NK_GRID):
-            run, ws_bytes = _problem(fmt, M, N, K, dev)
-            # every kernel is timed in two passes, the second in reverse order, and the faster one counts: single
-            # timings of one and the same kernel differ by 2-6 % with their position in the sequence (cold operands
-            # first, a warm chip last)
-            order = tiles + ((-1,) if not emit else ())
-            t = {v: _time_us(lambda: run(v)) for v in order}
-            for v in reversed(order):
-                t[v] = min(t[v], _time_us(lambda: run(v)))
-            best_v = min(tiles, key=lambda v: t[v])
-            if emit:
-                rule = int(lib.hk_gemm_tile_choice(FORMATS[fmt], M, N, K, 0))
-                t_rule = t[[v for v in tiles if size_of[v] == rule][0]]
-                line = (f"M={M} N={N} K={K}: rule {rule} {t_rule:.1f} us | 256x256 {t[tiles[0]]:.1f}  128x128 "
-                        f"{t[tiles[1]]:.1f}  64x64 {t[tiles[2]]:.1f}")
-                if t_rule > EMIT_MARGIN * t[best_v]:
-                    entries.add(((M + 63) // 64, (N + 63) // 64, _k_steps(fmt, K), size_of[best_v]))
-                    line += f"  -> table: {size_of[best_v]}"
-                print(line, flush=True)
-                continue
-            line = (f"M={M} N={N} K={K}: default {t[-1]:.1f} us | 256x256 {t[tiles[0]]:.1f}  128x128 "
-                    f"{t[tiles[1]]:.1f}  64x64 {t[tiles[2]]:.1f}")
-            if ws_bytes:
-                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-                line += f" | split-K {_time_us(lambda: run(-1, ws)):.1f}"
-            total += 1
-            if t[-1] > 1.05 * t[best_v]:
-                behind += 1
-                line += "  <-- default more than 5 % behind"
-            print(line, flush=True)
+    grid = lambda ms, nks: [(M, N, K) for M in ms for N, K in nks]
+    shapes = grid(M_GRID_EMIT, NK_GRID_EMIT) if emit else list(_drawn(draw, random.Random())) if draw else grid(M_GRID, NK_GRID)
+    behind = rule_behind = 0
+    measured = []
+    for M, N, K in shapes:
+        run, ws_bytes = _problem(fmt, M, N, K, dev)
+        t = measure(run)
+        best = min(TILES, key=lambda v: t[v])
+        rule = int(lib.hk_gemm_tile_shape(FORMATS[fmt], M, N, K, 0))
+        line = f"{fmt} {M} {N} {K}: default {t[None]:.1f} us, rule {rule} {t[rule]:.1f} |" + "".join(f" {v}: {t[v]:.1f}" for v in TILES)
+        if ws_bytes and not emit:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+            line += f" | split-K {_time_us(lambda: run(None, ws)):.1f}"
+        if t[None] > 1.05 * t[best]:
+            behind += 1
+            line += "  <-- default more than 5 % behind"
+        rule_behind += t[rule] > 1.05 * t[best]
+        measured.append((((M + 63) // 64, (N + 63) // 64, _k_steps(fmt, K)), rule, {v: t[v] for v in TILES}))
+        print(line, flush=True)
+    print(f"{fmt}: more than 5 % behind the best tile kernel on {behind} (default) / {rule_behind} (rule alone) of {len(shapes)} shapes")
     if emit:
+        entries = _entries(measured)
         cus = torch.cuda.get_device_properties(0).multi_processor_count
         n = _write_table(fmt, entries, cus)
         print(f"{len(entries)} entries for {fmt}; {TABLE_PATH} now holds {n}: rebuild the library "
               f"(python -m hipkittens_amd.build)")
-    else:
-        print(f"default more than 5 % behind the best tile kernel on {behind} of {total} shapes")
     return 0
 
 

@@ -70,8 +70,9 @@ def _load_native():
 
 
 def gemm_tile_choice(fmt: str, M: int, N: int, K: int, consult_table: bool = True) -> int:
-    """Tile (256, 128 or 64) the library picks for a GEMM of format "fp8", "bf16" or "mxfp4" on the current
-    device; consult_table False: the rule alone, without the generated per-shape table (tile_sweep.py)."""
+    """Square tile (256, 128 or 64) the library picks for a GEMM of format "fp8", "bf16" or "mxfp4" on the current
+    device; consult_table False: the rule alone, without the generated per-shape table (tile_sweep.py). The ring
+    kernel's 192x256 or 256x192 tile may run in its place: hk_gemm_shorter_tile and hk_gemm_tile_shape say whether."""
     code = {"fp8": 0, "bf16": 1, "mxfp4": 2}.get(fmt)
     if code is None:
         raise RuntimeError(f"unknown GEMM format {fmt!r}")

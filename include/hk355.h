@@ -50,6 +50,18 @@ int hk_gemm_tile_choice(int format, int M, int N, int K, int consult_table);
  * of the tile that hk_gemm_tile_choice names: 0 = no, 1 = 192x256 (192 rows of A), 2 = 256x192. Negative: a status. */
 int hk_gemm_shorter_tile(int format, int M, int N, int K);
 
+/* Both answers in one: rows * 1000 + columns of the tile that they take (256256, 128128, 64064, 192256 or 256192);
+ * consult_table as for hk_gemm_tile_choice. Negative: a status. hk_*_gemm_tile: the same GEMM, pinned to the tile kernel
+ * that such a number names (for tests and tuning, like hk_*_gemm_variant; any other number: HK_ERR_UNSUPPORTED). All five
+ * give identical bits. */
+int hk_gemm_tile_shape(int format, int M, int N, int K, int consult_table);
+int hk_fp8_gemm_tile(const void* A_e4m3, const void* B_e4m3, void* C_bf16, int M, int N, int K, float scale_a,
+                     float scale_b, int tile, void* stream);
+int hk_bf16_gemm_tile(const void* A_bf16, const void* B_bf16, void* C_bf16, int M, int N, int K, int tile, void* stream);
+int hk_mxfp4_gemm_tile(const void* A_e2m1, const void* A_scales_e8m0, int A_scale_pitch, const void* B_e2m1,
+                       const void* B_scales_e8m0, int B_scale_pitch, void* C_bf16, int M, int N, int K, int tile,
+                       void* stream);
+
 /*
  * FP8 e4m3 (OCP e4m3fn) GEMM:  C[M,N] = bf16( (scale_a*scale_b) * sum_k A[m,k]*B[n,k] ).
  * A is [M,K] row-major, B is [N,K] row-major ("column-major B"), both 1 byte per

@@ -188,9 +188,27 @@ def test_tile_choice_rule_and_generated_table():
     entries = [e for e in entries if e[0] != 255]
     assert entries and len(set(e[:4] for e in entries)) == len(entries)     # one tile per key
     k_per_step = {0: 128, 1: 64, 2: 256}
+    lib = hk.load_library()
     for code, m64, n64, nk, tile in entries:
-        assert tile in (256, 128, 64)
+        assert tile in (256, 128, 64, 192256, 256192)
         fmt = ("fp8", "bf16", "mxfp4")[code]
         M, N, K = 64 * m64 - 5, 64 * n64, nk * k_per_step[code]
-        assert tk.gemm_tile_choice(fmt, M, N, K) == tile
-        assert tk.gemm_tile_choice(fmt, M, N, K, False) != tile             # an entry that repeats the rule is noise
+        shape = tile if tile > 256 else 1001 * tile
+        assert lib.hk_gemm_tile_shape(code, M, N, K, 1) == shape            # final: the rule does not judge it again
+        assert lib.hk_gemm_tile_shape(code, M, N, K, 0) != shape            # an entry that repeats the rule is noise
+        assert lib.hk_gemm_shorter_tile(code, M, N, K) == {192256: 1, 256192: 2}.get(tile, 0)
+        if tile <= 256:
+            assert tk.gemm_tile_choice(fmt, M, N, K) == tile
+        else:
+            assert tk.gemm_tile_choice(fmt, M, N, K) == tk.gemm_tile_choice(fmt, M, N, K, False)
+
+
+def test_shorter_tile_rule():
+    """192x256 and 256x192 where they fill a round of 256 CUs that square tiles leave idle, 256x256 where that does."""
+    lib = hk.load_library()
+    for code in (0, 1, 2):
+        assert lib.hk_gemm_tile_shape(code, 3001, 4096, 4096, 0) == 192256
+        assert lib.hk_gemm_tile_shape(code, 4096, 2880, 2880, 0) == 256192
+        assert lib.hk_gemm_tile_shape(code, 4096, 4096, 4096, 0) == 256256
+        assert lib.hk_gemm_tile_shape(code, 1024, 1024, 1024, 0) == 64064
+        assert lib.hk_gemm_tile_shape(code, 0, 4096, 4096, 0) < 0 and lib.hk_gemm_tile_shape(3, 64, 64, 64, 0) < 0

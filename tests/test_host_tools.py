@@ -94,3 +94,17 @@ def test_tile_table_rewrite_keeps_the_other_formats(tmp_path, monkeypatch):
                     "{1, 12, 45, 23, 64},", "{2, 9, 9, 9, 256},"]
     assert tile_sweep._k_steps("fp8", 8192) == 64 and tile_sweep._k_steps("bf16", 8192) == 128
     assert tile_sweep._k_steps("mxfp4", 2880) == 12
+
+
+def test_table_entries_from_measured_times():
+    """An entry where the rule's tile is behind by the margin, with the fastest of the five tiles; none where another shape
+    of the same key (16 and 64 rows) would be slower with it."""
+    from hipkittens_amd import tile_sweep as ts
+
+    times = lambda *us: dict(zip(ts.TILES, us))
+    measured = [((1, 8, 4), 64064, times(9, 5.0, 6.0, 8, 8)), ((1, 8, 4), 64064, times(9, 5.0, 5.5, 8, 8)),   # both gain
+                ((1, 9, 4), 64064, times(9, 5.0, 6.0, 8, 8)), ((1, 9, 4), 64064, times(9, 5.5, 5.0, 8, 8)),   # one loses
+                ((4, 4, 4), 128128, times(9, 5.0, 6, 8, 4.9)),                                               # inside the margin
+                ((16, 16, 9), 128128, times(9, 8.0, 9, 7.0, 7.5))]
+    assert ts._entries(measured) == {(1, 8, 4, 128), (16, 16, 9, 192256)}
+    assert len({s for s in ts._drawn(50, __import__("random").Random(1))}) > 45
