@@ -137,16 +137,16 @@ __device__ __forceinline__ v4i mx_block_codes(const float (&h)[2][4], bool ok, i
 
 // x [rows, cols] bf16 -> packed e2m1 [rows, cols/2] + e8m0 scales [rows, scale_pitch] (columns
 // >= cols/32 are filled with 127). One thread per 8 elements of ROWS consecutive rows, 4 threads per MX block. The loads of
-// a thread's rows go out together: with one row, 16 bytes a thread are too few in flight, and finding the row (a division
-// of 64 bits, which only grids of 2^31 threads and more need: Index) takes longer than the rest.
+// a thread's rows go out together: with one row, 16 bytes a thread are too few in flight, and finding the row by a division
+// of 64 bits (a grid has fewer than 2^32 threads) takes longer than the rest.
 // Back to back, us, one row and 64-bit index / now: 8192 x 8192 32.4 / 29.3, 4096 x 8192 18.2 / 15.9, 4096 x 2880 7.4 / 7.2.
-template <bool A8, int ROWS, typename Index>
+template <bool A8, int ROWS>
 __global__ __launch_bounds__(256) void mx_quantize_rows_kernel(const uint16_t* __restrict__ x, int rows,
                                                                int cols, uint8_t* __restrict__ packed,
                                                                uint8_t* __restrict__ scales,
                                                                int scale_pitch) {
-    const Index per_row = (Index)scale_pitch * 4;  // threads per row, a multiple of 4 (and of 32: pitch % 8 == 0)
-    const Index gid = (Index)blockIdx.x * 256 + threadIdx.x;
+    const unsigned per_row = (unsigned)scale_pitch * 4;  // threads per row, a multiple of 4 (and of 32: pitch % 8 == 0)
+    const unsigned gid = blockIdx.x * 256 + threadIdx.x;
     const int row0 = (int)(gid / per_row) * ROWS;
     const int c8 = (int)(gid % per_row);  // which group of 8 elements
     if (row0 >= rows) return;
@@ -184,8 +184,8 @@ static int launch_mx_quantize_rows(const void* x, int rows, int cols, void* pack
     const long long four = ((long long)rows + 3) / 4 * scale_pitch * 4, one = (long long)rows * scale_pitch * 4;
     const bool by4 = four >= 1024ll * moe_num_compute_units();
     const long long threads = by4 ? four : one;
-    auto kern = threads >= (1ll << 31) ? (by4 ? mx_quantize_rows_kernel<A8, 4, long long> : mx_quantize_rows_kernel<A8, 1, long long>)
-                                       : (by4 ? mx_quantize_rows_kernel<A8, 4, unsigned> : mx_quantize_rows_kernel<A8, 1, unsigned>);
+    if (threads > 0xffffff00ll) return HK_ERR_LAUNCH;   // (more than a grid can have)
+    auto kern = by4 ? mx_quantize_rows_kernel<A8, 4> : mx_quantize_rows_kernel<A8, 1>;
     hipLaunchKernelGGL(kern, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, (const uint16_t*)x, rows, cols,
                        (uint8_t*)packed, (uint8_t*)scales, scale_pitch);
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;

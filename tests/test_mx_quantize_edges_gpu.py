@@ -10,21 +10,27 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
+@pytest.mark.parametrize("fmt", ["mxfp4", "mxfp8"])
 @pytest.mark.parametrize("cols", [96, 2880])
 @pytest.mark.parametrize("rows", [1, 1023, 2730, 4096, 4097, 4098, 4099, 32771])
-def test_rows_of_every_remainder(hk, rows, cols):
+def test_rows_of_every_remainder(hk, rows, cols, fmt):
     rng = np.random.default_rng(rows + cols)
     x = F.bf16_to_f32(F.bf16_round(rng.standard_normal((rows, cols)).astype(np.float32)))
     xt = torch.from_numpy(x).to(DEV).to(torch.bfloat16)
-    pitch = -(-cols // 256) * 8
+    pitch, width = -(-cols // 256) * 8, cols if fmt == "mxfp8" else cols // 2
     guard = 64
-    packed = torch.full((rows * cols // 2 + guard,), 0xAA, dtype=torch.uint8, device=DEV)
+    packed = torch.full((rows * width + guard,), 0xAA, dtype=torch.uint8, device=DEV)
     scales = torch.full((rows * pitch + guard,), 0xAA, dtype=torch.uint8, device=DEV)
-    hk.tk_kernel.dispatch_mxfp4_quantize_rows(xt, packed[:rows * cols // 2].view(rows, -1), scales[:rows * pitch].view(rows, pitch))
+    out = packed[:rows * width].view(rows, width), scales[:rows * pitch].view(rows, pitch)
+    if fmt == "mxfp8":
+        hk.tk_kernel.dispatch_mxfp8_quantize_rows(xt, out[0].view(torch.float8_e4m3fn), out[1])
+        want_p, want_s = F.quantize_mxfp8(x)
+    else:
+        hk.tk_kernel.dispatch_mxfp4_quantize_rows(xt, *out)
+        want_p, want_s = F.quantize_mxfp4(x)
     torch.cuda.synchronize()
-    want_p, want_s = F.quantize_mxfp4(x)
-    assert np.array_equal(packed[:-guard].view(rows, -1).cpu().numpy(), want_p)
-    got = scales[:-guard].view(rows, pitch).cpu().numpy()
+    assert np.array_equal(out[0].cpu().numpy(), want_p)
+    got = out[1].cpu().numpy()
     assert np.array_equal(got[:, :cols // 32], want_s) and (got[:, cols // 32:] == 127).all()
     assert (packed[-guard:] == 0xAA).all() and (scales[-guard:] == 0xAA).all()
 
