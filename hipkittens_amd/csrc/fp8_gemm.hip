@@ -352,9 +352,9 @@ extern "C" int hk_gemm_tile_choice(int format, int M, int N, int K, int consult_
     using namespace hk;
     const int nk = tile_k_steps(format, M, N, K);
     if (!nk) return HK_ERR_BAD_SHAPE;
-    const int listed = consult_table ? table_tile(format, M, N, nk) : 0;
-    return listed == BM || listed == kSmallTile || listed == kTinyTile ? listed
-                                                                      : pick_tile_rule(M, N, nk, kTileRules[format], moe_num_compute_units());
+    const int cus = moe_num_compute_units();
+    const int listed = consult_table ? table_tile(format, M, N, nk, cus) : 0;
+    return listed == BM || listed == kSmallTile || listed == kTinyTile ? listed : pick_tile_rule(M, N, nk, kTileRules[format], cus);
 }
 
 extern "C" int hk_gemm_shorter_tile(int format, int M, int N, int K) {

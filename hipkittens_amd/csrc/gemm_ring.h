@@ -46,9 +46,10 @@ constexpr int kRingScaleSlot = 2 * 256 * 16;   // A's rows, then B's (256 of eac
 constexpr int ring_lds_bytes(int tile_m, int tile_n, bool scaled) {
     return (2 * tile_m + 3 * tile_n) * BK + (scaled ? 2 * kRingScaleSlot : 0);
 }
-// Rows past M or N are not clamped: they lie outside the descriptors, fetch nothing and arrive as zeros (with a row address
-// per load, clamped to the last row, ragged problems had a register and a vector instruction per load more: BF16 3001 x
-// 4096 x 4096 on 192x256 tiles 79.0 us, now 74.9).
+// Rows past M or N are not clamped: they lie outside the descriptors, fetch nothing and arrive as zeros. This depends on the
+// buffers' range check counting the scalar offset, which holds the K offset and the rows of a load (i * dma_row_stride): seen with
+// an offset that wrapped, whose loads returned zeros. (With a row address per load, clamped to the last row, ragged problems had
+// a register and a vector instruction per load more: BF16 3001 x 4096 x 4096 on 192x256 tiles 79.0 us, now 74.9.)
 // EDGE: M or N is not a multiple of the tile (only the epilogue needs to know).
 template <typename MMA, bool EDGE, bool STREAM_C = false, int TILE_M = BM, int TILE_N = BN>
 __device__ __forceinline__ void gemm_ring_body(uint8_t* smem, const uint8_t* __restrict__ A,

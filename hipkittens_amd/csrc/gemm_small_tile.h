@@ -384,12 +384,34 @@ static inline int pick_tile_rule(int M, int N, int nk, TileRule r, int cus) {
     }
     return tile[best];
 }
-// The table's entry for a shape: 256, 128, 64 or one of the ring kernel's shorter tiles; 0: none.
-static inline int table_tile(int fmt, int M, int N, int nk) {
-    if (moe_num_compute_units() != kTileTableCus) return 0;   // (256 when no device can be queried)
+// The table's entry for a shape: 256, 128, 64 or one of the ring kernel's shorter tiles; 0: none. (The entries behind the
+// first are in order; a walk over all of them, on every call, is a tenth of a microsecond.)
+constexpr unsigned long long tile_key(unsigned long long fmt, unsigned long long m64, unsigned long long n64, unsigned long long nk) {
+    return fmt << 48 | m64 << 32 | n64 << 16 | nk;
+}
+constexpr int kTileTableSize = sizeof(kTileTable) / sizeof(kTileTable[0]);
+constexpr bool tile_table_in_order() {
+    for (int i = 2; i < kTileTableSize; ++i) {
+        const TileTableEntry &a = kTileTable[i - 1], &b = kTileTable[i];
+        if (tile_key(a.fmt, a.m64, a.n64, a.nk) >= tile_key(b.fmt, b.m64, b.n64, b.nk)) return false;
+    }
+    return true;
+}
+static_assert(tile_table_in_order(), "table_tile searches it by halves");
+static inline int table_tile(int fmt, int M, int N, int nk, int cus) {
+    if (cus != kTileTableCus) return 0;
     const long long m64 = ((long long)M + 63) / 64, n64 = ((long long)N + 63) / 64;
-    for (const TileTableEntry& e : kTileTable)
-        if (e.fmt == fmt && e.m64 == m64 && e.n64 == n64 && e.nk == nk) return e.tile;
+    if (m64 > 0xffff || n64 > 0xffff || nk > 0xffff) return 0;
+    const unsigned long long key = tile_key(fmt, m64, n64, nk);
+    int lo = 1, hi = kTileTableSize;
+    while (lo < hi) {
+        const int mid = (lo + hi) / 2;
+        const TileTableEntry& e = kTileTable[mid];
+        const unsigned long long k = tile_key(e.fmt, e.m64, e.n64, e.nk);
+        if (k == key) return e.tile;
+        if (k < key) lo = mid + 1;
+        else hi = mid;
+    }
     return 0;
 }
 // the formats' constants (K-steps: 128 bytes of an operand row)
@@ -413,8 +435,7 @@ constexpr TileRule kTileRules[3] = {{{7.10f, 3.28f, 2.02f}, {1.060f, 0.533f, 0.3
 constexpr int kVariant192x256 = 192256, kVariant256x192 = 256192;   // the GEMM entry points' internal numbers for them
 struct ShorterTileRule { float fixed, per_step, small; };
 constexpr ShorterTileRule kShorterTileRules[3] = {{5.7f, 0.87f, 0.82f}, {5.6f, 0.925f, 0.94f}, {7.37f, 1.057f, 0.974f}};
-static inline int pick_shorter_tile(int M, int N, int nk, int tile, TileRule rule, ShorterTileRule shorter) {
-    const long long cus = moe_num_compute_units();
+static inline int pick_shorter_tile(int M, int N, int nk, int tile, TileRule rule, ShorterTileRule shorter, long long cus) {
     auto rounds = [&](int tm, int tn, long long capacity) {
         const long long tiles = (((long long)M + tm - 1) / tm) * (((long long)N + tn - 1) / tn);
         return (double)((tiles + capacity - 1) / capacity);
@@ -429,11 +450,12 @@ static inline int pick_shorter_tile(int M, int N, int nk, int tile, TileRule rul
 }
 // The tile kernel of a shape: 256, 128, 64, kVariant192x256 or kVariant256x192. A measured entry of the table is final.
 static inline int pick_gemm_tile(int fmt, int M, int N, int nk, bool consult_table = true) {
-    const int listed = consult_table ? table_tile(fmt, M, N, nk) : 0;
+    const int cus = moe_num_compute_units();   // 256 when no device can be queried
+    const int listed = consult_table ? table_tile(fmt, M, N, nk, cus) : 0;
     if (listed) return listed;
     const TileRule& rule = kTileRules[fmt];
-    const int square = pick_tile_rule(M, N, nk, rule, moe_num_compute_units());
-    const int shorter = pick_shorter_tile(M, N, nk, square, rule, kShorterTileRules[fmt]);
+    const int square = pick_tile_rule(M, N, nk, rule, cus);
+    const int shorter = pick_shorter_tile(M, N, nk, square, rule, kShorterTileRules[fmt], cus);
     return shorter ? shorter : square;
 }
 

@@ -78,6 +78,8 @@ __device__ __forceinline__ float glu_act(float g, float u, float alpha, float li
     u = __builtin_amdgcn_fmed3f(u, -limit, limit);
     return (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + __expf(-alpha * g)));
 }
+// The same with the activation chosen at run time, for the kernel on plain weights (two instantiations of it instead of three).
+// Here fmin(fmax()) on purpose: with the median that kernel spills 62 scalar registers, 56 without.
 __device__ __forceinline__ float glu_act(int act, float g, float u, float alpha, float limit) {
     if (act == 0) return silu_mul(g, u);
     g = fminf(g, limit);

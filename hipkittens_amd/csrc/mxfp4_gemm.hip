@@ -50,7 +50,8 @@ __device__ __forceinline__ void mfma_fp4_acc(v4f& acc, const v4i& x, const v4i& 
         : "v"(x), "v"(y), "v"(sx), "v"(sy));
 }
 
-// (Rows past M or N: outside the descriptors, as in gemm_ring.h; EDGE is the epilogue's.)
+// (Rows past M or N: outside the descriptors, whose range check counts the scalar offset with a load's rows in it, as in
+// gemm_ring.h; EDGE is the epilogue's.)
 template <bool EDGE>
 __global__ __launch_bounds__(256) void mxfp4_gemm_4wave_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ SA, const uint8_t* __restrict__ B,

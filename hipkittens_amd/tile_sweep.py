@@ -151,7 +151,7 @@ def _write_table(fmt, entries, cus):
         "// another tile kernel: {format, ceil(M / 64), ceil(N / 64), K-steps, tile}; 192256 and 256192: the ring kernel's shorter",
         "// tiles.",
         f"constexpr int kTileTableCus = {cus};   // CU count of the device the sweeps ran on",
-        "static const TileTableEntry kTileTable[] = {",
+        "static constexpr TileTableEntry kTileTable[] = {",
         "    {255, 0, 0, 0, 0},   // (keeps the array non-empty)",
     ]
     lines += [f"    {{{e[0]}, {e[1]}, {e[2]}, {e[3]}, {e[4]}}}," for e in rows]
