@@ -7,10 +7,10 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-# rows per expert: around the edges of fragments (16 rows), of the fragments under one branch (64, 72, 96) and of items
-# (128, 144, 192); the mean has to stay above one item
-ROWS = [1, 16, 17, 63, 65, 72, 73, 95, 96, 97, 112, 113, 128, 129, 144, 145, 176, 177, 191, 192, 193, 208, 288, 384, 385,
-        400, 577, 900]
+# rows per expert: around the edges of fragments (16 rows), of the fragments under one branch (80, 96 and 128 rows for items of
+# up to 128, 144 and 192) and of items (128, 144, 192); the mean has to stay above one item
+ROWS = [1, 16, 17, 63, 65, 79, 80, 81, 95, 96, 97, 112, 113, 127, 128, 129, 144, 145, 176, 177, 191, 192, 193, 208, 288, 384,
+        385, 400, 577, 900]
 
 
 def _layer(hk, E, H, I, seed):
