@@ -360,8 +360,9 @@ static __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* 
 //     of the single round of 256 small tiles (the small tile wins by 60 %);
 //  3. a shorter tile in its place where that is estimated faster (pick_shorter_tile).
 // Measured against the best of the five kernels, every launch on another copy of B (a model's weights come from HBM, not from
-// the memory-side cache), the rule alone is more than 5 % behind on 36 / 16 / 21 of the sweep's 414 shapes (FP8 / BF16 /
-// MXFP4), with the table on 0 / 1 / 1, and on 24 / 37 / 9 of 450 shapes drawn between the sweep's points.
+// the memory-side cache), the rule alone is more than 5 % behind on 36 / 16 / 20 of the sweep's 414 shapes (FP8 / BF16 /
+// MXFP4; without the about 40 that the skinny kernel takes), with the table on none (all 414 on another device: 2 / 2 / 1), and on
+// 24 / 37 / 9 of 450 shapes drawn between the sweep's points.
 struct TileRule {
     float fixed[3], per_step[3];   // 256-, 128-, 64-tile
 };

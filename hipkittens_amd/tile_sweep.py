@@ -235,7 +235,10 @@ def main(argv):
             behind += 1
             line += "  <-- default more than 5 % behind"
         rule_behind += t[rule] > 1.05 * t[best]
-        measured.append((((M + 63) // 64, (N + 63) // 64, _k_steps(fmt, K)), rule, {v: t[v] for v in TILES}))
+        choice = int(lib.hk_gemm_tile_shape(FORMATS[fmt], M, N, K, 1))
+        # (up to 64 rows the default can be the skinny kernel, which a time of its own shows: no tile to list there)
+        if M > 64 or abs(t[None] / t[choice] - 1.0) <= 0.05:
+            measured.append((((M + 63) // 64, (N + 63) // 64, _k_steps(fmt, K)), rule, {v: t[v] for v in TILES}))
         print(line, flush=True)
     print(f"{fmt}: more than 5 % behind the best tile kernel on {behind} (default) / {rule_behind} (rule alone) of {len(shapes)} shapes")
     if emit:
