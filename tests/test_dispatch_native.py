@@ -62,6 +62,23 @@ def test_without_the_module_the_python_dispatchers_take_every_call(monkeypatch, 
         assert [w.category for w in said] == ([RuntimeWarning] if i == 0 else [])   # said once
 
 
+def test_the_build_goes_on_without_a_host_compiler(monkeypatch, tmp_path, capsys):
+    from hipkittens_amd import build
+
+    def no_compiler():
+        raise FileNotFoundError("g++")
+
+    stale = tmp_path / "_dispatch.so"
+    stale.write_text("of an earlier build")
+    monkeypatch.setattr(build, "DISPATCH_PATH", stale)
+    monkeypatch.setattr(build, "_build_dispatch", no_compiler)
+    monkeypatch.setattr(build, "_compile_one", lambda src, extra: src)
+    linked = []
+    monkeypatch.setattr(build, "_link", lambda objs, out: linked.append(out))
+    assert build.build(check=False) == build.LIB_PATH and build.LIB_PATH in linked
+    assert not stale.exists() and "not built" in capsys.readouterr().err
+
+
 def _calls(dev):
     g = torch.Generator(device=dev).manual_seed(3)
     M, N, K = 33, 80, 544
