@@ -944,6 +944,7 @@ __global__ __launch_bounds__(256) void moe_fp8blk_preshuffle_kernel(const uint8_
 
 }  // namespace hk
 #include "moe_fp8blk_few.h"
+#include "moe_fp8blk_tall.h"
 namespace hk {
 
 // The few-rows kernel for as many items as the list can hold (the workgroups past its actual length leave at once).
@@ -976,9 +977,20 @@ static int launch_fp8blk_stream_nt(const MoeFp8Params& p, int max_items, hipStre
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
+template <int MODE>
+static int launch_fp8blk_tall(const MoeFp8Params& p, int max_items, hipStream_t s) {
+    auto kern = moe_fp8blk_tall_kernel<MODE>;
+    static DeviceOnce configured;
+    if (!set_lds_limit_once((const void*)kern, kF8tLds, configured)) return HK_ERR_LAUNCH;
+    const int grid = min(max_items, moe_num_compute_units());
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(512), kF8tLds, s, p);
+    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
+}
+
 // bm: rows per work item the item lists were built for (kF8BM or kF8BMShort)
 template <int MODE, bool GATHER>
 static int launch_fp8blk_stream(const MoeFp8Params& p, int max_items, hipStream_t s, bool nt, int bm) {
+    if (bm == kF8tBM) return launch_fp8blk_tall<MODE>(p, max_items, s);
     constexpr int kShort = kF8BMShort / 16;
     if (bm == kF8BMShort)
         return nt ? launch_fp8blk_stream_nt<MODE, GATHER, true, kShort>(p, max_items, s)
@@ -987,13 +999,25 @@ static int launch_fp8blk_stream(const MoeFp8Params& p, int max_items, hipStream_
               : launch_fp8blk_stream_nt<MODE, GATHER, false, kF8sMT>(p, max_items, s);
 }
 
-// Rows per work item of the streaming kernels for a layer of T * k slots over E experts: 144 unless
-// that costs a pass over the weights that 160 would not (judged at mean + two standard deviations of
-// an expert's rows under uniform routing).
-static int moe_fp8blk_item_rows(int T, int k, int E) {
+// Rows per work item of the kernels for pre-shuffled weights, for a layer of T * k slots over E experts, judged at mean +
+// two standard deviations of an expert's rows under uniform routing. 144 unless that costs a pass over the weights that
+// 160 would not (streaming kernel); 288 (tall kernel) where that saves a third of the rounds in which the gate+up GEMM's
+// items go over the CUs: by fewer passes over the weights, unless there are too few items for that to matter. us,
+// streaming / tall kernel, even routing: H = 7168, I = 2048, 256 experts, k = 8 (rows per expert) 128 2377 / 2492,
+// 140 2777 / 2544, 178 3440 / 2714, 256 3760 / 3269, and with experts asked for unevenly (standard deviation 0.8 of the
+// mean) 256 4078 / 3689; H = 4096, I = 1536, 64 experts, k = 4: 125 285 / 299, 169 404 / 328, 281 479 / 483, 312 590 / 531,
+// 512 798 / 693; one expert, H = 7168, I = 2048: 1400 rows 93 / 123 (one round either way), 3000 197 / 152 (two rounds
+// and one), 6000 308 / 307 (three and two), 8192 396 / 355.
+static int moe_fp8blk_item_rows(int T, int H, int I, int E, int k) {
     const double mu = (double)T * k / E, hi = mu + 2.0 * __builtin_sqrt(mu);
     const long long n_short = (long long)((hi + kF8BMShort - 1) / kF8BMShort);
     const long long n_long = (long long)((hi + kF8BM - 1) / kF8BM);
+    const long long n_tall = (long long)((hi + kF8tBM - 1) / kF8tBM);
+    const long long cus = moe_num_compute_units();
+    auto rounds = [&](long long passes) { return (E * passes * (I / 128) + cus - 1) / cus; };
+    // (the tall kernel needs three K-steps, and row offsets that leave bit 31 free)
+    if (H >= 384 && I >= 384 && (long long)T * H < (1ll << 31) && 3 * rounds(n_tall) <= 2 * rounds(std::min(n_short, n_long)))
+        return kF8tBM;
     return n_short <= n_long ? kF8BMShort : kF8BM;
 }
 
@@ -1140,7 +1164,7 @@ static int fp8blk_grouped_gemms(const void* x_e4m3, const float* x_scales, const
     const bool few = weight_layout == 1 && moe_fp8blk_few(T, H, I, E, k);
     const bool identity = !sorted_slots, lists = !few || !identity;
     int32_t* nitems = (int32_t*)(ws + L.nitems);
-    const int bm = few ? kF8FewRows : weight_layout == 1 ? moe_fp8blk_item_rows(T, k, E) : kF8BM;
+    const int bm = few ? kF8FewRows : weight_layout == 1 ? moe_fp8blk_item_rows(T, H, I, E, k) : kF8BM;
     if (identity && lists) {
         hipLaunchKernelGGL(moe_identity_routing_kernel, dim3((T + 255) / 256), dim3(256), 0, s, T,
                            (int32_t*)(ws + L.sorted), (int32_t*)(ws + L.offsets));
