@@ -1453,6 +1453,7 @@ __global__ __launch_bounds__(256) void moe_mxfp4_stream4_kernel(const MoeGemmPar
 
 }  // namespace hk
 #include "moe_mxfp4_few.h"
+#include "moe_mxfp4_tall.h"
 namespace hk {
 
 // ------------------------------------------------------------------------------ un-permute
@@ -1568,6 +1569,15 @@ template <int MODE, int EXT, bool A8, bool GATHER = false>
 static int launch_moe_stream(MoeGemmParams p, int max_items, hipStream_t s, bool nt) {
     return nt ? launch_moe_stream_nt<MODE, EXT, A8, GATHER, true>(p, max_items, s)
               : launch_moe_stream_nt<MODE, EXT, A8, GATHER, false>(p, max_items, s);
+}
+
+template <int MODE, int EXT>
+static int launch_moe_tall(const MoeGemmParams& p, int max_items, hipStream_t s) {
+    auto kern = moe_mxfp4_tall_kernel<MODE, EXT>;
+    static DeviceOnce configured;
+    if (!set_lds_limit_once((const void*)kern, kTlLds, configured)) return HK_ERR_LAUNCH;
+    hipLaunchKernelGGL(kern, dim3(min(max_items, moe_num_compute_units())), dim3(512), kTlLds, s, p);
+    return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
 // The few-rows kernel on items of `rows` rows (16, or 32 with MXFP4 activations): four one-wave workgroups per item that the list can hold (the
@@ -1759,9 +1769,9 @@ static int moe_mxfp4_check(int T, int H, int I, int E, int k, int w13_scale_pitc
     return HK_OK;
 }
 
-static MoeBuildItems moe_items_args(uint8_t* ws, const MoeWs& L, int I, int H, bool a8, int weight_layout, bool gather, int few) {
+static MoeBuildItems moe_items_args(uint8_t* ws, const MoeWs& L, int I, int H, bool a8, int weight_layout, bool gather, int few, bool tall) {
     MoeBuildItems b;
-    b.bm = few ? few : a8 ? (gather ? S4Cfg<true, true>::kBM : S4Cfg<true, false>::kBM) : weight_layout ? kStBM : kMoeBM;
+    b.bm = few ? few : tall ? kTlBM : a8 ? (gather ? S4Cfg<true, true>::kBM : S4Cfg<true, false>::kBM) : weight_layout ? kStBM : kMoeBM;
     b.items[0] = (MoeItem*)(ws + L.items1); b.items[1] = (MoeItem*)(ws + L.items2);
     b.n_tiles[0] = (I + 127) / 128; b.n_tiles[1] = (H + 255) / 256;
     return b;
@@ -1782,6 +1792,21 @@ static MxQuantizeArgs moe_quantize_args(const void* x_bf16, const int32_t* sorte
 // 4096 tokens of 2880 MXFP4 columns, 1024 of MXFP8).
 static bool moe_gathers(int weight_layout, bool ext, bool a8, int T, int H) {
     return weight_layout == 1 && !ext && (long long)T * H * (a8 ? 2 : 1) <= 12ll << 20;
+}
+
+// Whether a layer on pre-shuffled weights takes the tall kernel (items of up to 288 rows; MXFP4 activations): from a mean of
+// 400 rows per expert on, where it needs fewer rounds of the gate+up GEMM's items over the CUs (judged at mean + two standard
+// deviations of an expert's rows under uniform routing). Layer, us, streaming / tall kernel, at the mean number of rows, `~`
+// with experts asked for unevenly: 2880 x 2880, 128 experts, biases and clamped SwiGLU ~188 578 / 599, 344 851 / 873, 406
+// 1016 / 966, 512 1181 / 1118, ~512 1226 / 1173; 32 experts, plain ~250 192 / 199, ~500 310 / 306, ~750 447 / 415, ~2048 1100 /
+// 1017; 1792 x 1024, 64 experts, plain ~219 118 / 118, ~500 215 / 190, ~1024 375 / 328.
+constexpr int kTallMinMean = 400;
+static bool moe_tall(int T, int H, int I, int E, int k, int weight_layout, bool a8) {
+    if (weight_layout != 1 || a8 || H <= 512 || I <= 512) return false;   // (the kernel needs three K-steps)
+    const double mu = (double)T * k / E, hi = mu + 2.0 * __builtin_sqrt(mu);
+    const long long cus = moe_num_compute_units();
+    auto rounds = [&](int bm) { return (E * (long long)((hi + bm - 1) / bm) * ((I + 127) / 128) + cus - 1) / cus; };
+    return (long long)T * k >= (long long)kTallMinMean * E && rounds(kTlBM) < rounds(kStBM);
 }
 
 // Every argument check of the expert MLP, made before the first launch of a call (the forward entry points run
@@ -1838,13 +1863,14 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
 
     int32_t* nitems = (int32_t*)(ws + L.nitems);
     const int few = weight_layout == 1 ? moe_few_rows(T, H, I, E, k, a8, ext) : 0;
-    const bool gather = few || moe_gathers(weight_layout, ext, a8, T, H);
+    const bool tall = !few && moe_tall(T, H, I, E, k, weight_layout, a8);
+    const bool gather = few || (!tall && moe_gathers(weight_layout, ext, a8, T, H));
     // non-temporal weight loads while most experts' rows fit one work item (their weights are then read
     // once): mean + one standard deviation of the rows per expert under uniform routing
     const bool nt = moe_rows_fit_one_item(T, k, E, a8 ? (gather ? S4Cfg<true, true>::kBM : S4Cfg<true, false>::kBM) : kStBM);
     if (!x_quantized) {   // (the forward pass of a small layer has done this in its sort launch)
         const int nk1 = (H / 2 + 127) / 128;
-        const MoeBuildItems b = moe_items_args(ws, L, I, H, a8, weight_layout, gather, few);
+        const MoeBuildItems b = moe_items_args(ws, L, I, H, a8, weight_layout, gather, few, tall);
         const MxQuantizeArgs qa = moe_quantize_args(x_bf16, sorted_slots, slot_to_pos, k, T, H, I, ws, L);
         auto qp = a8 ? (gather ? mx_quantize_permute_kernel<true, false> : mx_quantize_permute_kernel<true, true>)
                      : (gather ? mx_quantize_permute_kernel<false, false> : mx_quantize_permute_kernel<false, true>);
@@ -1869,6 +1895,9 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
     p.bias = bias13; p.bias_bytes = (uint32_t)((size_t)E * 2 * I * 4); p.act = activation; p.alpha = alpha; p.limit = limit; p.interleaved = w13_interleaved != 0;
     if (few)
         st = launch_moe_few<0>(p, few, a8, ext, moe_few_max_items(S, E, few, p.n_tiles_n), s);
+    else if (tall)
+        st = !ext ? launch_moe_tall<0, 0>(p, L.max_items1, s)
+             : activation ? launch_moe_tall<0, 2>(p, L.max_items1, s) : launch_moe_tall<0, 1>(p, L.max_items1, s);
     else if (a8)
         st = ext ? (activation ? launch_moe_stream<0, 2, true>(p, L.max_items1, s, nt) : launch_moe_stream<0, 1, true>(p, L.max_items1, s, nt))
                  : gather ? launch_moe_stream<0, 0, true, true>(p, L.max_items1, s, nt)
@@ -1896,6 +1925,8 @@ static int moe_mxfp4_experts_impl(const void* x_bf16, const void* w13, const voi
     q.bias = bias2; q.bias_bytes = (uint32_t)((size_t)E * H * 4);
     if (few)
         st = launch_moe_few<1>(q, few, a8, bias2 != nullptr, moe_few_max_items(S, E, few, q.n_tiles_n), s);
+    else if (tall)
+        st = bias2 ? launch_moe_tall<1, 1>(q, L.max_items2, s) : launch_moe_tall<1, 0>(q, L.max_items2, s);
     else if (a8)
         st = bias2 ? launch_moe_stream<1, 1, true>(q, L.max_items2, s, nt) : launch_moe_stream<1, 0, true>(q, L.max_items2, s, nt);
     else if (bias2)
@@ -1964,12 +1995,13 @@ static int moe_mxfp4_forward_impl(const void* x_bf16, const float* router_logits
     const bool ext = bias13 || bias2 || activation != 0 || w13_interleaved;
     bool fused = false;
     const int few = weight_layout == 1 ? moe_few_rows(T, H, I, E, k, a8, ext) : 0;
-    if ((few || moe_gathers(weight_layout, ext, a8, T, H)) && (long long)T * k <= kSortSmallMax && x_bf16 &&
+    const bool tall = !few && moe_tall(T, H, I, E, k, weight_layout, a8);
+    if ((few || (!tall && moe_gathers(weight_layout, ext, a8, T, H))) && (long long)T * k <= kSortSmallMax && x_bf16 &&
         (((uintptr_t)x_bf16 | (uintptr_t)workspace) & 15u) == 0) {
         // sort, item lists and the quantization of x in one launch (moe_sort_quantize_kernel)
         const int S = T * k, nchunks = (S + kSortChunk - 1) / kSortChunk;
         const int nk1 = (H / 2 + 127) / 128;
-        const MoeBuildItems b = moe_items_args(ws, L, I, H, a8, weight_layout, true, few);
+        const MoeBuildItems b = moe_items_args(ws, L, I, H, a8, weight_layout, true, few, tall);
         const MxQuantizeArgs qa = moe_quantize_args(x_bf16, nullptr, nullptr, k, T, H, I, ws, L);
         const int grid = nchunks + 2 * kFusedItemParts + (T + kQpRows - 1) / kQpRows * ((nk1 + 7) / 8);
         auto kern = a8 ? moe_sort_quantize_kernel<true> : moe_sort_quantize_kernel<false>;
