@@ -280,9 +280,12 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 __device__ __forceinline__ int xcd_chunk_order(int wg, int num_wg, int chunk) {
     const int span = kNumXcd * chunk;
     const int full = (num_wg / span) * span;
-    if (wg >= full) return wg;
     const int xcd = wg % kNumXcd;
     const int local = wg / kNumXcd;
+    if (wg >= full) {   // the last, partial span: equal runs, the first `longer` XCDs have one id more
+        const int rest = num_wg - full, run = rest / kNumXcd, longer = rest % kNumXcd;
+        return full + xcd * run + min(xcd, longer) + (local - full / kNumXcd);
+    }
     return (local / chunk) * span + xcd * chunk + (local % chunk);
 }
 
