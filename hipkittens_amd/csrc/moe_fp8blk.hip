@@ -903,7 +903,9 @@ __global__ __launch_bounds__(256) void moe_fp8blk_stream_kernel(const MoeFp8Para
                 epilogue(cc);
                 zero_acc();
                 // what the next K-step adds for "the last fragment of the previous K-step"
+                // (the partial sums too: zero times a NaN would reach a row of the next item)
                 sc[(MT - 1 + PAR) & 1][0] = 0.f; sc[(MT - 1 + PAR) & 1][1] = 0.f;
+                part[2] = v4f{0.f, 0.f, 0.f, 0.f}; part[3] = v4f{0.f, 0.f, 0.f, 0.f};
             }
         }
         cc = cn;
