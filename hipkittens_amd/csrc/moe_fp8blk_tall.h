@@ -8,7 +8,7 @@
 // patch instead of 96. Both operands go through LDS, two slots each of 36 KiB of activations and 32 KiB of weights:
 //   * a wave's four weight fragments are read into registers over the last twelve MFMAs of the position before, which go
 //     through the last three row fragments column by column, so that one weight fragment after the other is done with
-//     (read in one go behind the last MFMA, 64 reads of the eight waves met in front of the next one: 1.5 % of the layer);
+//     (read in one go behind the last MFMA, 64 reads of the eight waves met in front of the next one: 1 % of the layer);
 //     a barrier then frees the slot, and the weights of the position after the next are requested into it: they have
 //     more than a K-step to arrive from HBM;
 //   * the activation tile of the position after the next is requested when everyone has read this one's, ahead of the
@@ -19,7 +19,7 @@
 // The K loop exists for items of five to nine pairs of row fragments: rows of experts that are asked for unevenly fill two
 // thirds of their items (all items through the nine: 4319 us instead of 3895). The epilogue, shared, tests each fragment.
 // No non-temporal hint on the weights, which an expert's second item wants from L2 (3907 / 3831 us with / without it).
-// DeepSeek-V3-like layer, 8192 tokens, rows per expert 256 +- 206: 4118 us with the streaming kernel, 3728 with this one
+// DeepSeek-V3-like layer, 8192 tokens, rows per expert 256 +- 206: 4118-4201 us with the streaming kernel, 3728-3838 with this one
 // (gate+up 2603 -> 2307, down 1458 -> 1311); 256 +- 16: 3760 / 3269. What bounds it now is power as much as latency: the
 // clock is 1.64-1.79 GHz where the streaming kernel's is 1.84-1.93, the matrix cores are busy 51-53 % of the time.
 // Same MFMA, K order and scaling FMAs as the other two kernels: the same bits.

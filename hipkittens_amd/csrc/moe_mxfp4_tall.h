@@ -10,8 +10,8 @@
 // loads is vmcnt(5): everything but the weights and weight scales of the position after the next. A row's scale byte is read
 // from LDS as a byte (no shift), a weight's is picked by the MFMA. The K loop exists for items of five to nine pairs of row
 // fragments; the epilogue, shared, tests each fragment.
-// GPT-OSS-like layer, 16384 tokens, biases and clamped SwiGLU: 1239-1257 us with the streaming kernel, 1163-1190 with this one (gate+up
-// 808 -> 750, down 390 -> 380). What bounds it (development builds, layer, us): without epilogues 1015, on empty loads 1022, both
+// GPT-OSS-like layer, 16384 tokens, biases and clamped SwiGLU: 1239-1274 us with the streaming kernel, 1163-1201 with this one (gate+up
+// 860 -> 793, down 418 -> 401, traced). What bounds it (development builds, layer, us): without epilogues 1015, on empty loads 1022, both
 // 866, of which 140 are not GEMMs: MFMAs, LDS reads and two barriers a position take 1.7 times the MFMAs' own time, the epilogue of
 // all eight waves at once 150, and what loads cost on top 150; matrix cores busy 41 % at 1.83 GHz.
 // Same MFMA and K order as the other kernels: the same bits.
