@@ -332,9 +332,10 @@ __global__ __launch_bounds__(512) void moe_mxfp4_tall_kernel(const MoeGemmParams
                 if constexpr (J == 20) read_frag.template operator()<0>();
                 if constexpr (J == 17) read_bf.template operator()<2>();
                 if constexpr (J == 23) { read_bf.template operator()<3>(); read_sb.template operator()<1>(); }
-                // loads: the weights two positions on, when everyone holds its fragments of this one's; the activations two
-                // positions on, when everyone has read this one's
-                if constexpr (I == 6) { block_barrier(); slot_fence(); }
+                // loads: the weights two positions on, when everyone holds its fragments of this one's (slot 7 is the first to
+                // use, and so to wait for, the last of them: there is no other wait in front of the barrier); the activations
+                // two positions on, when everyone has read this one's
+                if constexpr (I == 7) { block_barrier(); slot_fence(); }
                 if constexpr (I == 8) load_b.template operator()<0>();
                 if constexpr (I == 10) load_b.template operator()<1>();
                 if constexpr (I == 12) load_b.template operator()<2>();

@@ -183,3 +183,52 @@ def test_scalar_register_spills_do_not_grow(assembly):
             if res.get("sgpr_spills", 0) > ceiling:
                 over.append(f"{src} {name}: {res['sgpr_spills']} scalar registers spilled (ceiling {ceiling})")
     assert not over, "\n".join(over)
+
+
+def _loops_with_two_barriers(text, kernel):
+    """(function, instructions) of the innermost loops of `kernel`'s instantiations that hold two barriers, with the blocks
+    that several ways back to the loop's head enclose."""
+    import re
+
+    lines = [raw.split(";")[0].strip() for raw in text.split("\n")]
+    function, labels, spans = "", {}, {}
+    for n, line in enumerate(lines):
+        label = re.match(r"^([.$\w]+):$", line)
+        back = re.match(r"s_c?branch\S*\s+(\S+)", line)
+        if label and not label.group(1).startswith(".L"):
+            function, labels = label.group(1), {}
+        elif label:
+            labels[label.group(1)] = n
+        elif back and kernel in function and back.group(1) in labels:
+            first = labels[back.group(1)]
+            barriers = tuple(i for i in range(first, n) if lines[i] == "s_barrier")
+            if len(barriers) == 2:
+                lo, hi = spans.get((function, barriers), (first, n))
+                spans[function, barriers] = (min(lo, first), max(hi, n))
+    return [(f, [isa_check._instruction(x) for x in lines[lo:hi] if re.match(r"[a-z]", x)])
+            for (f, _), (lo, hi) in spans.items()]
+
+
+@pytest.mark.parametrize("source,kernel,instances,weights", [("moe_fp8blk.hip", "moe_fp8blk_tall_kernel", 2, 8),
+                                                             ("moe_mxfp4.hip", "moe_mxfp4_tall_kernel", 5, 8)])
+def test_tall_kernels_hold_their_weights_before_the_slot_is_free(assembly, source, kernel, instances, weights):
+    """A barrier of the K loops of the kernels for items of up to 288 rows lets the next weights be written over the ones
+    that the waves have read, and no wait for LDS reads stands in front of it: every weight fragment and weight scale that
+    comes out of LDS is used by a matrix instruction, and so has arrived, before the next barrier."""
+    loops = _loops_with_two_barriers(assembly[source], kernel)
+    assert len(loops) == 5 * instances, [f for f, _ in loops]   # items of five to nine pairs of row fragments
+    for function, body in loops:
+        regs = isa_check._vector_registers
+        held = {r for op, _, o in body if op.startswith("v_mfma") for t in o[1:2] + o[4:5] for r in regs(t.split()[0])}
+        pending, reads = set(), set()
+        for op, _, operands in body + body:   # (twice: the reads of one K-step are used in the next)
+            if op.startswith("ds_read"):
+                landed_in = [r for r in regs(operands[0]) if r in held]
+                pending.update(landed_in)
+                if len(landed_in) == 4:
+                    reads.add(operands[0])
+            elif op.startswith("v_mfma"):
+                pending.difference_update(r for t in operands[1:6] for r in regs(t.split()[0]))
+            elif op == "s_barrier":
+                assert not pending, f"{function}: {sorted(pending)} may not have been read when a barrier frees their slot"
+        assert len(reads) == weights, f"{function}: weights by way of {sorted(reads)}"
