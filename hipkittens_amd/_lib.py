@@ -24,7 +24,9 @@ SIGNATURES = {
     "hk_bf16_gemm_tile": (c_int, [c_void_p] * 3 + [c_int] * 4 + [c_void_p]),
     "hk_mxfp4_gemm_tile": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_void_p, c_int, c_void_p] + [c_int] * 4 + [c_void_p]),
     "hk_moe_mxfp4_few_rows": (c_int, [c_int] * 7),
+    "hk_moe_mxfp4_item_rows": (c_int, [c_int] * 7),
     "hk_moe_fp8blk_few_rows": (c_int, [c_int] * 5),
+    "hk_moe_fp8blk_item_rows": (c_int, [c_int] * 5),
     "hk_fp8_gemm": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_void_p]),
     "hk_fp8_gemm_variant": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_float, c_int, c_void_p]),
     "hk_fp8_quantize_tensor_workspace_bytes": (c_size_t, []),

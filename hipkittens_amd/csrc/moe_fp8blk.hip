@@ -989,7 +989,7 @@ static int launch_fp8blk_tall(const MoeFp8Params& p, int max_items, hipStream_t 
     return hipGetLastError() == hipSuccess ? HK_OK : HK_ERR_LAUNCH;
 }
 
-// bm: rows per work item the item lists were built for (kF8BM or kF8BMShort)
+// bm: rows per work item the item lists were built for (kF8BM or kF8BMShort; kF8tBM: the tall kernel's)
 template <int MODE, bool GATHER>
 static int launch_fp8blk_stream(const MoeFp8Params& p, int max_items, hipStream_t s, bool nt, int bm) {
     if (bm == kF8tBM) return launch_fp8blk_tall<MODE>(p, max_items, s);
@@ -1002,7 +1002,8 @@ static int launch_fp8blk_stream(const MoeFp8Params& p, int max_items, hipStream_
 }
 
 // Rows per work item of the kernels for pre-shuffled weights, for a layer of T * k slots over E experts, judged at mean +
-// two standard deviations of an expert's rows under uniform routing. 144 unless that costs a pass over the weights that
+// two standard deviations of an expert's rows under uniform routing, rounded down to whole rows (288.9 rows are one pass of
+// 288). 144 unless that costs a pass over the weights that
 // 160 would not (streaming kernel); 288 (tall kernel) where that saves a third of the rounds in which the gate+up GEMM's
 // items go over the CUs: by fewer passes over the weights, unless there are too few items for that to matter. us,
 // streaming / tall kernel, even routing: H = 7168, I = 2048, 256 experts, k = 8 (rows per expert) 128 2377 / 2492,
@@ -1124,6 +1125,10 @@ extern "C" size_t hk_moe_fp8blk_workspace_bytes(int T, int H, int I, int E, int 
 extern "C" int hk_moe_fp8blk_few_rows(int T, int H, int I, int E, int k) {
     if (fp8blk_check(T, H, I, E, k) != HK_OK) return HK_ERR_BAD_SHAPE;
     return moe_fp8blk_few(T, H, I, E, k) ? kF8FewRows : 0;
+}
+extern "C" int hk_moe_fp8blk_item_rows(int T, int H, int I, int E, int k) {
+    if (fp8blk_check(T, H, I, E, k) != HK_OK) return HK_ERR_BAD_SHAPE;
+    return moe_fp8blk_few(T, H, I, E, k) ? kF8FewRows : moe_fp8blk_item_rows(T, H, I, E, k);
 }
 
 extern "C" int hk_moe_fp8blk_preshuffle_bytes(int E, int N, int K, int mode, size_t* w_bytes) {

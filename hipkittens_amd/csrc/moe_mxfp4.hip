@@ -1769,9 +1769,13 @@ static int moe_mxfp4_check(int T, int H, int I, int E, int k, int w13_scale_pitc
     return HK_OK;
 }
 
+// Rows per work item.
+static int moe_item_rows(bool a8, int weight_layout, bool gather, int few, bool tall) {
+    return few ? few : tall ? kTlBM : a8 ? (gather ? S4Cfg<true, true>::kBM : S4Cfg<true, false>::kBM) : weight_layout ? kStBM : kMoeBM;
+}
 static MoeBuildItems moe_items_args(uint8_t* ws, const MoeWs& L, int I, int H, bool a8, int weight_layout, bool gather, int few, bool tall) {
     MoeBuildItems b;
-    b.bm = few ? few : tall ? kTlBM : a8 ? (gather ? S4Cfg<true, true>::kBM : S4Cfg<true, false>::kBM) : weight_layout ? kStBM : kMoeBM;
+    b.bm = moe_item_rows(a8, weight_layout, gather, few, tall);
     b.items[0] = (MoeItem*)(ws + L.items1); b.items[1] = (MoeItem*)(ws + L.items2);
     b.n_tiles[0] = (I + 127) / 128; b.n_tiles[1] = (H + 255) / 256;
     return b;
@@ -1796,7 +1800,7 @@ static bool moe_gathers(int weight_layout, bool ext, bool a8, int T, int H) {
 
 // Whether a layer on pre-shuffled weights takes the tall kernel (items of up to 288 rows; MXFP4 activations): from a mean of
 // 400 rows per expert on, where it needs fewer rounds of the gate+up GEMM's items over the CUs (judged at mean + two standard
-// deviations of an expert's rows under uniform routing). Layer, us, streaming / tall kernel, at the mean number of rows, `~`
+// deviations of an expert's rows under uniform routing, in whole rows as in moe_fp8blk_item_rows). Layer, us, streaming / tall kernel, at the mean number of rows, `~`
 // with experts asked for unevenly: 2880 x 2880, 128 experts, biases and clamped SwiGLU ~188 578 / 599, 344 851 / 873, 406
 // 1016 / 966, 512 1181 / 1118, ~512 1226 / 1173; 32 experts, plain ~250 192 / 199, ~500 310 / 306, ~750 447 / 415, ~2048 1100 /
 // 1017; 1792 x 1024, 64 experts, plain ~219 118 / 118, ~500 215 / 190, ~1024 375 / 328.
@@ -1807,6 +1811,12 @@ static bool moe_tall(int T, int H, int I, int E, int k, int weight_layout, bool 
     const long long cus = moe_num_compute_units();
     auto rounds = [&](int bm) { return (E * (long long)((hi + bm - 1) / bm) * ((I + 127) / 128) + cus - 1) / cus; };
     return (long long)T * k >= (long long)kTallMinMean * E && rounds(kTlBM) < rounds(kStBM);
+}
+extern "C" int hk_moe_mxfp4_item_rows(int T, int H, int I, int E, int k, int mxfp8, int ext) {
+    if (!moe_mxfp4_shape_ok(T, H, I, E, k)) return HK_ERR_BAD_SHAPE;
+    const bool a8 = mxfp8 != 0;
+    const int few = moe_few_rows(T, H, I, E, k, a8, ext != 0);
+    return moe_item_rows(a8, 1, moe_gathers(1, ext != 0, a8, T, H), few, !few && moe_tall(T, H, I, E, k, 1, a8));
 }
 
 // Every argument check of the expert MLP, made before the first launch of a call (the forward entry points run

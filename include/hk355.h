@@ -284,9 +284,11 @@ int hk_moe_unpermute_add(const void* o_bf16, const float* w, const int32_t* slot
 size_t hk_moe_mxfp4_workspace_bytes(int T, int H, int I, int E, int k);
 
 /* Rows per work item (16 or 32) where a layer on pre-shuffled weights takes the few-rows kernel on the current
- * device, 0 where it takes the streaming kernel; negative: a status. mxfp8: MXFP8 activations; ext: biases, clamped
- * SwiGLU or interleaved rows. (Host only; for tests and tuning, like hk_gemm_tile_choice.) */
+ * device, 0 where it takes the streaming or the tall kernel; negative: a status. mxfp8: MXFP8 activations; ext: biases,
+ * clamped SwiGLU or interleaved rows. (Host only; for tests and tuning, like hk_gemm_tile_choice.) */
 int hk_moe_mxfp4_few_rows(int T, int H, int I, int E, int k, int mxfp8, int ext);
+/* Likewise, rows per work item whichever kernel it is: 16 or 32 few rows, 128, 144 or 192 streaming, 288 tall. */
+int hk_moe_mxfp4_item_rows(int T, int H, int I, int E, int k, int mxfp8, int ext);
 
 /* Offline weight pre-shuffle (weight_layout = 1 below). For every expert, n-tile and K-step the
  * 256 x 128-byte weight tile is stored contiguously in the order the kernel keeps it in LDS
@@ -386,6 +388,8 @@ int hk_fp8_quantize_rows_1x128(const void* x_bf16, int rows, int cols, void* q_e
 size_t hk_moe_fp8blk_workspace_bytes(int T, int H, int I, int E, int k);
 /* As hk_moe_mxfp4_few_rows, for the block-scaled layer: 16 or 0. */
 int hk_moe_fp8blk_few_rows(int T, int H, int I, int E, int k);
+/* As hk_moe_mxfp4_item_rows: 16 few rows, 144 or 160 streaming, 288 tall. */
+int hk_moe_fp8blk_item_rows(int T, int H, int I, int E, int k);
 
 /* Expert MLP for routed and sorted tokens (outputs of hk_moe_topk_* and hk_moe_sort). */
 int hk_moe_fp8blk_experts(const void* x_e4m3, const float* x_scales, const void* w13,

@@ -1,5 +1,5 @@
-"""Which layers take the few-rows kernel (host only; without a GPU the rules assume 256 CUs). Both sides of each line are
-layers that were timed on both kernels."""
+"""Which layers take the few-rows kernel, and which the one for items of 288 rows (host only; without a GPU the rules assume
+256 CUs). Both sides of each line of the few-rows rule are layers that were timed on both kernels."""
 import pytest
 
 import hipkittens_amd
@@ -37,7 +37,28 @@ def test_fp8blk(H, I, E, k, T, rows):
     assert lib.hk_moe_fp8blk_few_rows(T, H, I, E, k) == rows
 
 
+@pytest.mark.parametrize("H,I,E,k,T,mxfp8,ext,rows", [
+    (2880, 2880, 128, 4, 16384, 0, 1, 288), (2880, 2880, 128, 4, 12800, 0, 1, 288), (2880, 2880, 128, 4, 12799, 0, 1, 192),
+    (2880, 2880, 128, 4, 16384, 1, 0, 144), (2880, 2880, 128, 4, 1000, 1, 0, 128), (2880, 2880, 128, 4, 4, 0, 1, 16),
+    (512, 2880, 128, 4, 16384, 0, 0, 192), (544, 2880, 128, 4, 16384, 0, 0, 288),     # three K-steps
+    (2880, 512, 128, 4, 16384, 0, 0, 192)])
+def test_mxfp4_item_rows(H, I, E, k, T, mxfp8, ext, rows):
+    assert lib.hk_moe_mxfp4_item_rows(T, H, I, E, k, mxfp8, ext) == rows
+
+
+@pytest.mark.parametrize("H,I,E,k,T,rows", [
+    (7168, 2048, 256, 8, 8192, 288), (7168, 2048, 256, 8, 64, 16), (7168, 2048, 256, 8, 2048, 144),
+    # whole rows of mean + two standard deviations: 144 and 145, 160 and 161, 288 and 289 (there two items of either length)
+    (7168, 2048, 256, 8, 3930, 144), (7168, 2048, 256, 8, 3931, 160), (7168, 2048, 256, 8, 4401, 160),
+    (7168, 2048, 256, 8, 4402, 288), (7168, 2048, 256, 8, 8222, 288), (7168, 2048, 256, 8, 8223, 160),
+    (256, 2048, 256, 8, 8192, 144), (384, 2048, 256, 8, 8192, 288), (7168, 256, 256, 8, 8192, 144),   # three K-steps
+    (7168, 2048, 1, 1, 1400, 160), (7168, 2048, 1, 1, 3000, 288)])   # one round either way; two rounds and one
+def test_fp8blk_item_rows(H, I, E, k, T, rows):
+    assert lib.hk_moe_fp8blk_item_rows(T, H, I, E, k) == rows
+
+
 def test_refused_shapes():
     assert lib.hk_moe_mxfp4_few_rows(0, 2880, 2880, 128, 4, 0, 0) == -2
     assert lib.hk_moe_mxfp4_few_rows(4, 2880, 2880, 4, 8, 0, 0) == -2
     assert lib.hk_moe_fp8blk_few_rows(4, 100, 128, 4, 2) == -2
+    assert lib.hk_moe_mxfp4_item_rows(4, 2880, 2880, 4, 8, 0, 0) == -2 and lib.hk_moe_fp8blk_item_rows(4, 100, 128, 4, 2) == -2

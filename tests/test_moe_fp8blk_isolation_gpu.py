@@ -26,7 +26,7 @@ def test_nan_weights_of_an_expert_of_few_rows(hk, long):
     logits = torch.full((T, E), -30.0, device=DEV)
     logits[torch.arange(T, device=DEV), ids] = 30.0
     ws = torch.empty(hk.tk_kernel.moe_fp8blk_workspace_bytes(T, H, I, E, 1), dtype=torch.uint8, device=DEV)
-    assert hk.load_library().hk_moe_fp8blk_few_rows(T, H, I, E, 1) == 0
+    assert hk.load_library().hk_moe_fp8blk_item_rows(T, H, I, E, 1) == long
 
     def run(a, b):
         W = hk.tk_kernel.MoeFp8BlkShuffledWeights.from_plain(a, s13, b, s2)

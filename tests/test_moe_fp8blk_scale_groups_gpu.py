@@ -13,7 +13,7 @@ DEV = "cuda:0"
 def test_row_scales_in_groups_of_four(hk, T, E, H):
     I, k = 512, 2
     print(f"fp8blk scale groups T={T} E={E} H={H}", flush=True)
-    assert hk.load_library().hk_moe_fp8blk_few_rows(T, H, I, E, k) == 0   # the streaming kernel
+    assert hk.load_library().hk_moe_fp8blk_item_rows(T, H, I, E, k) in (144, 160)   # the streaming kernel
     g = torch.Generator(device=DEV).manual_seed(H + E)
     e4m3 = lambda *s: (torch.randn(*s, device=DEV, generator=g) * 40).to(torch.float8_e4m3fn)
     scales = lambda *s: torch.exp2(torch.randint(-12, -4, s, device=DEV, generator=g).float())
