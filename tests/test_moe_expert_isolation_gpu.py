@@ -6,7 +6,6 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-LONG = 600
 # rows of the experts of few rows: one fragment of 16, and up to the last that leaves a shared branch's fragments without rows
 SHORT = [1, 16, 17, 33, 48, 49, 64, 65, 80, 81, 96, 97, 111, 112, 5, 30]
 
@@ -22,13 +21,16 @@ def _weights(hk, g, E, rows, cols, short):
 
 @pytest.mark.parametrize("act_format", ["mxfp4", "mxfp8"])
 @pytest.mark.parametrize("options", [{}, {"bias": True}, {"activation": "swiglu_oai", "bias": True}], ids=["plain", "biases", "swiglu"])
-@pytest.mark.parametrize("H", [512, 1024])   # (plain: rows gathered by token up to 512, MXFP4 up to 1024; else permuted)
-def test_nan_scale_of_an_expert_of_few_rows(hk, H, options, act_format):
-    print(f"moe expert isolation H={H} {options} {act_format}", flush=True)
+# (plain: rows gathered by token up to 512, MXFP4 up to 1024; else permuted; MXFP4 with experts of 1000 rows: items of 288)
+@pytest.mark.parametrize("H,long", [(512, 600), (1024, 600), (1024, 1000)])
+def test_nan_scale_of_an_expert_of_few_rows(hk, H, long, options, act_format):
+    print(f"moe expert isolation H={H} long={long} {options} {act_format}", flush=True)
     # 512 and more items of gate+up and, at H = 1024, more than 256 of down: a workgroup's next item is the 32nd behind
-    I, rows = 1024, [r for s in SHORT for r in (s, LONG)]
+    I, rows = 1024, [r for s in SHORT for r in (s, long)]
     E, T = len(rows), sum(rows)
     short = list(range(0, E, 2))
+    tall = hk.load_library().hk_moe_mxfp4_item_rows(T, H, I, E, 1, act_format == "mxfp8", bool(options)) == 288
+    assert tall == (long == 1000 and act_format == "mxfp4")
     g = torch.Generator(device=DEV).manual_seed(H)
     p13, s13, bad13 = _weights(hk, g, E, 2 * I, H, short)
     p2, s2, bad2 = _weights(hk, g, E, H, I, short)

@@ -1,8 +1,6 @@
 """The MXFP4 MoE's kernel for items of up to 288 rows: every number of row fragments per item, one and more items per expert,
 all epilogues, K of three K-steps and of a part of the last one. A token's result does not depend on the tokens beside it,
 so the whole batch has to equal, bit for bit, the same tokens in batches small enough for the other kernels."""
-import math
-
 import pytest
 import torch
 
@@ -11,14 +9,6 @@ DEV = "cuda:0"
 # rows per expert: around the edges of fragments (16 and 32 rows), of the K loops (160 to 288 rows) and of items
 ROWS = [0, 1, 15, 16, 17, 31, 33, 128, 159, 160, 161, 176, 177, 192, 193, 224, 225, 256, 257, 272, 273, 287, 288, 289, 305, 321,
         385, 448, 512, 576, 577, 640, 863, 865, 1000, 1152, 1153, 1700, 2000, 2500]
-
-
-def _takes_tall_kernel(T, H, I, E, k):
-    """The rule of moe_tall."""
-    hi = T * k / E + 2 * math.sqrt(T * k / E)
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    rounds = lambda bm: math.ceil(E * math.ceil(hi / bm) * math.ceil(I / 128) / cus)
-    return min(H, I) > 512 and T * k >= 400 * E and rounds(288) < rounds(192)
 
 
 def _run(hk, x, logits, W, H, I, E, **options):
@@ -36,8 +26,9 @@ def _run(hk, x, logits, W, H, I, E, **options):
 def test_items_of_up_to_288_rows(hk, H, I, biases, activation, interleaved):
     print(f"mxfp4 tall H={H} I={I} {biases} {activation} {interleaved}", flush=True)
     E, T = len(ROWS), sum(ROWS)
-    if not _takes_tall_kernel(T, H, I, E, 1):
-        pytest.skip("this device's rule takes the streaming kernel")
+    ext = biases or interleaved or activation != "silu"
+    item_rows = lambda tokens: hk.load_library().hk_moe_mxfp4_item_rows(tokens, H, I, E, 1, 0, ext)
+    assert item_rows(T) == 288 and item_rows(2048) == 192
     g = torch.Generator(device=DEV).manual_seed(H + I)
     w13 = hk.quant.quantize_mxfp4(torch.randn(E * 2 * I, H, device=DEV, generator=g) * 0.2)
     w2 = hk.quant.quantize_mxfp4(torch.randn(E * H, I, device=DEV, generator=g) * 0.2)
@@ -55,6 +46,5 @@ def test_items_of_up_to_288_rows(hk, H, I, biases, activation, interleaved):
         options["bias2"] = torch.randn(E, H, device=DEV, generator=g)
     whole = _run(hk, x, logits, W, H, I, E, **options)
     parts = [_run(hk, x[t:t + 2048], logits[t:t + 2048], W, H, I, E, **options) for t in range(0, T, 2048)]
-    assert not _takes_tall_kernel(2048, H, I, E, 1)
     assert torch.isfinite(whole.float()).all()
     assert torch.equal(whole.view(torch.int16), torch.cat(parts).view(torch.int16))
