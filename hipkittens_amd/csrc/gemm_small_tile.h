@@ -363,9 +363,12 @@ static __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* 
 //     of the single round of 256 small tiles (the small tile wins by 60 %);
 //  3. a shorter tile in its place where that is estimated faster (pick_shorter_tile).
 // Measured against the best of the five kernels, every launch on another copy of B (a model's weights come from HBM, not from
-// the memory-side cache), the rule alone is more than 5 % behind on 36 / 16 / 20 of the sweep's 414 shapes (FP8 / BF16 /
-// MXFP4; without the about 40 that the skinny kernel takes), with the table on none (all 414 on another device: 2 / 2 / 1), and on
-// 24 / 37 / 9 of 450 shapes drawn between the sweep's points.
+// the memory-side cache), the rule alone is more than 5 % behind on 38 / 21 / 26 of the sweep's 414 shapes (FP8 / BF16 /
+// MXFP4; without the about 40 that the skinny kernel takes), with the table on 3 / 4 / 4, by 9 % at most, and on
+// 24 / 28 / 9 of 450 shapes drawn between the sweep's points (without the about 155 of the skinny kernel): the more of two sweeps.
+// Table and constants were measured when a launch's last, partial span of tiles still went round robin over the XCDs (xcd_chunk_order).
+// Of the 100 swept shapes that have an entry 78 are still more than 3 % ahead of the rule's choice in both sweeps, and none that a tile
+// kernel takes is more than 1.1 % behind it in either; 8 / 8 / 5 shapes without one would get one in both.
 struct TileRule {
     float fixed[3], per_step[3];   // 256-, 128-, 64-tile
 };
@@ -427,15 +430,14 @@ constexpr TileRule kTileRules[3] = {{{7.10f, 3.28f, 2.02f}, {1.060f, 0.533f, 0.3
 // the same cost model, one workgroup per CU, gives them less time. The constants, and the factor on the estimate for a
 // 128- or 64-tile (which is high where it is compared with these), are fitted to 91 shapes per format on an MI355X
 // (M 500 ... 8192, (N, K) 4096 x 4096 ... 14336 x 4096, 2880 x 2880, 10000 x 1024, copies of B in rotation; MXFP4 again to 112
-// when its small-tile kernels became faster). Over the 414 shapes of the sweep and 450 drawn ones a shorter tile is more than 3 %
-// behind the square one on 5 / 1 / 5 (FP8 / BF16 / MXFP4; those of the sweep are in the table), and the geometric mean of the
-// drawn ones falls by 1.1 / 1.4 / 1.7 %, of 1.8 / 2.2 / 2.0 that the best kernel for every shape would give. (A fit to all of
-// them, {6.84, 0.882, 0.882}, {6.75, 0.816, 0.881}, {6.73, 1.07, 0.873}, gained 4 % where FP8 and BF16 choose otherwise with it, but
-// lost up to 14 % on single shapes, 0.6 % on the average for MXFP4.) Examples, us before /
-// after: BF16 3001 x 4096 x 4096 90.1 / 74.9 (192 tiles of 256x256 against 256 of 192x256), 4096 x 2880 x 2880 69.2 / 54.1; FP8
-// 8192 x 2880 x 2880 71.8 / 58.6; MXFP4 4096 x 2880 x 2880 35.2 / 27.8; and not taken: BF16 4096 x 4096 x 4096 96.3 / 130.9
-// (256 tiles of 256x256, one round; 352 of 192x256, two). Equal estimates go to 256x192: with the one that pads less instead, 5
-// more shapes of FP8 and 16 of BF16 are behind.
+// when its small-tile kernels became faster). Over the 414 shapes of the sweep and the about 295 of 450 drawn ones that a tile kernel
+// takes, a shorter tile is more than 3 % behind the square one on 3 / 2 / 3 (FP8 / BF16 / MXFP4; the more of two sweeps), and the
+// geometric mean of the drawn ones falls by 2.7 / 1.9 / 2.8 %, of 3.7 / 2.9 / 3.3 that the best kernel for every shape would give. (A
+// fit to all of them on the former tile order, {6.84, 0.882, 0.882}, {6.75, 0.816, 0.881}, {6.73, 1.07, 0.873}, gained 4 % where FP8 and
+// BF16 choose otherwise with it, but lost up to 14 % on single shapes, 0.6 % on the average for MXFP4.) Examples, us, 256x256 /
+// 256x192: BF16 4096 x 2880 x 2880 68.8 / 54.2 (192 tiles against 240); FP8 8192 x 2880 x 2880 71.8 / 59.6; MXFP4 4096 x 2880 x 2880
+// 34.5 / 27.6; and not taken: BF16 4096 x 4096 x 4096 97.8 / 130.1 (256 tiles of 256x256, one round; 352 of 256x192, two). Equal
+// estimates go to 256x192: with the one that pads less instead, 5 more shapes of FP8 and 16 of BF16 were behind on the former order.
 constexpr int kVariant192x256 = 192256, kVariant256x192 = 256192;   // the GEMM entry points' internal numbers for them
 struct ShorterTileRule { float fixed, per_step, small; };
 constexpr ShorterTileRule kShorterTileRules[3] = {{5.7f, 0.87f, 0.82f}, {5.6f, 0.925f, 0.94f}, {7.37f, 1.057f, 0.974f}};

@@ -282,7 +282,9 @@ __device__ __forceinline__ int xcd_chunk_order(int wg, int num_wg, int chunk) {
     const int full = (num_wg / span) * span;
     const int xcd = wg % kNumXcd;
     const int local = wg / kNumXcd;
-    if (wg >= full) {   // the last, partial span: equal runs, the first `longer` XCDs have one id more
+    // The last, partial span: equal runs, the first `longer` XCDs have one id more. us, that span round robin / in runs: FP8
+    // 500 x 6000 x 4096 23.0 / 21.5, MXFP4 3500 x 3000 x 4096 31.1 / 29.9 (the tiles that share a panel fetch it into one L2).
+    if (wg >= full) {
         const int rest = num_wg - full, run = rest / kNumXcd, longer = rest % kNumXcd;
         return full + xcd * run + min(xcd, longer) + (local - full / kNumXcd);
     }

@@ -409,8 +409,8 @@ __global__ __launch_bounds__(512) void moe_fp8blk_gemm_kernel(const MoeFp8Params
 // Results are bit-identical to the kernel above (same MFMA, K order and scaling FMAs).
 constexpr int kF8sMT = kF8BM / 16;                       // at most 10 row fragments per item
 // Items of nine fragments (144 rows): every K-step then runs nine fragments instead of ten. The host picks them
-// when they do not add a pass over the weights (moe_fp8blk_item_rows): at 256 +- 16 rows per expert (the
-// DeepSeek-V3-like layer at 8192 tokens) two items of up to 144 rows cover all but one expert in fifty.
+// when they do not add a pass over the weights (moe_fp8blk_item_rows): up to a mean of 122 rows per expert (the
+// DeepSeek-V3-like layer up to 3930 tokens) one item of up to 144 rows covers all but one expert in fifty.
 constexpr int kF8BMShort = 144;
 constexpr int kF8sStages = 4;                           // LDS stages = weight register sets = positions per trip of the K loop
 constexpr int kF8sStage = 21504;                         // 160 x 128 B, then 16 x 12 row scales, padded to a multiple of 256 B

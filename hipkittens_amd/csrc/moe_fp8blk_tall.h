@@ -20,7 +20,7 @@
 // thirds of their items (all items through the nine: 4319 us instead of 3895). The epilogue, shared, tests each fragment.
 // No non-temporal hint on the weights, which an expert's second item wants from L2 (3907 / 3831 us with / without it).
 // DeepSeek-V3-like layer, 8192 tokens, rows per expert 256 +- 206: 4118-4201 us with the streaming kernel, 3728-3838 with this one
-// (gate+up 2603 -> 2307, down 1458 -> 1311); 256 +- 16: 3760 / 3269. What bounds it now is power as much as latency: the
+// (gate+up 2595 -> 2342, down 1408 -> 1273, both traced in turn on one box); 256 +- 16: 3760 / 3269. What bounds it now is power as much as latency: the
 // clock is 1.64-1.79 GHz where the streaming kernel's is 1.84-1.93, the matrix cores are busy 51-53 % of the time.
 // Same MFMA, K order and scaling FMAs as the other two kernels: the same bits.
 #pragma once

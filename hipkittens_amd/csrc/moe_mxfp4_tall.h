@@ -11,7 +11,7 @@
 // from LDS as a byte (no shift), a weight's is picked by the MFMA. The K loop exists for items of five to nine pairs of row
 // fragments; the epilogue, shared, tests each fragment.
 // GPT-OSS-like layer, 16384 tokens, biases and clamped SwiGLU: 1239-1274 us with the streaming kernel, 1163-1201 with this one (gate+up
-// 860 -> 793, down 418 -> 401, traced). What bounds it (development builds, layer, us): without epilogues 1015, on empty loads 1022, both
+// 836 -> 785, down 406 -> 394, both traced in turn on one box). What bounds it (development builds, layer, us): without epilogues 1015, on empty loads 1022, both
 // 866, of which 140 are not GEMMs: MFMAs, LDS reads and two barriers a position take 1.7 times the MFMAs' own time, the epilogue of
 // all eight waves at once 150, and what loads cost on top 150; matrix cores busy 41 % at 1.83 GHz.
 // Same MFMA and K order as the other kernels: the same bits.
@@ -28,7 +28,7 @@ constexpr int kTlSa = kTlB + 2 * kMoeBTile;              // two of row scales, t
 constexpr int kTlSaTile = kTlBM * 8;
 constexpr int kTlSb = kTlSa + 2 * kTlSaTile;
 constexpr int kTlBias = kTlSb + 2 * kMoeScaleB;          // each wave's 64 biases of the item
-constexpr int kTlLds = kTlBias + 8 * 256;                // 150.5 KiB
+constexpr int kTlLds = kTlBias + 8 * 256;                // 146.5 KiB
 static_assert(kTlLds <= 160 * 1024 && kTlMT == 9, "LDS plan; the K loops are written out for five to nine fragments");
 
 typedef __attribute__((address_space(3))) const int lds_i32_t;
