@@ -48,17 +48,16 @@ PEAK_HBM = 8000.0     # GB/s
 TRAFFIC_FILE = os.path.join(ROOT, "profiles", "traffic.json")
 # The launches that make up one call of each leg's default workload, as rocprofv3 names the kernels.
 TRAFFIC_LEGS = {
-    "fp8_gemm_8192": ("calibration", ["fp8_gemm_4wave_ring_kernel<false>"]),
+    "fp8_gemm_8192": ("calibration", ["fp8_gemm_4wave_ring_kernel<false, 256, 256>"]),
     "mxfp4_gemm": ("mxfp4", ["mxfp4_gemm_4wave_kernel<false>"]),
-    "bf16_gemm": ("bf16", ["bf16_gemm_4wave_ring_kernel<false, true>"]),
+    "bf16_gemm": ("bf16", ["bf16_gemm_4wave_ring_kernel<false, true, 256, 256>"]),
     "fp8_gemm_decode_m16": ("decode", ["fp8_gemm_skinny_kernel<1, 4, 4, 2, true>"]),
     "moe_mxfp4": ("moe_mxfp4", ["moe_topk_softmax_kernel<16>", "moe_sort_quantize_kernel<false>",
-                                "moe_mxfp4_stream4_kernel<0, false, false, true, true>",
-                                "moe_mxfp4_stream4_kernel<1, false, false, false, true>", "moe_unpermute_kernel<4>"]),
+                                "moe_mxfp4_stream4_kernel<0, 0, false, true, true>",
+                                "moe_mxfp4_stream4_kernel<1, 0, false, false, true>", "moe_unpermute_kernel<4>"]),
     "moe_fp8blk": ("moe_fp8blk", ["moe_topk_grouped_sigmoid16_kernel<16>", "moe_sort_count_kernel",
                                   "moe_sort_scan_offsets_kernel", "moe_sort_scatter_kernel", "moe_build_items_kernel",
-                                  "moe_fp8blk_stream_kernel<0, true, false, 9>",
-                                  "moe_fp8blk_stream_kernel<1, false, false, 9>", "moe_unpermute_kernel<8>"]),
+                                  "moe_fp8blk_tall_kernel<0>", "moe_fp8blk_tall_kernel<1>", "moe_unpermute_kernel<8>"]),
 }
 _traffic_cache = None
 
