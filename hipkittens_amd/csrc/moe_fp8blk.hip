@@ -1003,10 +1003,9 @@ static int launch_fp8blk_stream(const MoeFp8Params& p, int max_items, hipStream_
 
 // Rows per work item of the kernels for pre-shuffled weights, for a layer of T * k slots over E experts, judged at mean +
 // two standard deviations of an expert's rows under uniform routing, rounded down to whole rows (288.9 rows are one pass of
-// 288). 144 unless that costs a pass over the weights that
-// 160 would not (streaming kernel); 288 (tall kernel) where that saves a third of the rounds in which the gate+up GEMM's
-// items go over the CUs: by fewer passes over the weights, unless there are too few items for that to matter. us,
-// streaming / tall kernel, even routing: H = 7168, I = 2048, 256 experts, k = 8 (rows per expert) 128 2377 / 2492,
+// 288). 144 unless that costs a pass over the weights that 160 would not (streaming kernel); 288 (tall kernel) where that
+// saves a third of the rounds in which the gate+up GEMM's items go over the CUs: by fewer passes over the weights, unless
+// there are too few items for that to matter. us, streaming / tall kernel, even routing: H = 7168, I = 2048, 256 experts, k = 8 (rows per expert) 128 2377 / 2492,
 // 140 2777 / 2544, 178 3440 / 2714, 256 3760 / 3269, and with experts asked for unevenly (standard deviation 0.8 of the
 // mean) 256 4078 / 3689; H = 4096, I = 1536, 64 experts, k = 4: 125 285 / 299, 169 404 / 328, 281 479 / 483, 312 590 / 531,
 // 512 798 / 693; one expert, H = 7168, I = 2048: 1400 rows 93 / 123 (one round either way), 3000 197 / 152 (two rounds

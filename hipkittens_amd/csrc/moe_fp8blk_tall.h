@@ -448,7 +448,7 @@ __global__ __launch_bounds__(512) void moe_fp8blk_tall_kernel(const MoeFp8Params
         epilogue(cur);
         it += it_stride;
         if (it >= it_end()) break;
-            cur = nxt;
+        cur = nxt;
         load_item(it + it_stride, nxt);
     }
     wait_vmcnt<0>();   // nothing may still be writing LDS when the workgroup retires

@@ -1800,10 +1800,10 @@ static bool moe_gathers(int weight_layout, bool ext, bool a8, int T, int H) {
 
 // Whether a layer on pre-shuffled weights takes the tall kernel (items of up to 288 rows; MXFP4 activations): from a mean of
 // 400 rows per expert on, where it needs fewer rounds of the gate+up GEMM's items over the CUs (judged at mean + two standard
-// deviations of an expert's rows under uniform routing, in whole rows as in moe_fp8blk_item_rows). Layer, us, streaming / tall kernel, at the mean number of rows, `~`
-// with experts asked for unevenly: 2880 x 2880, 128 experts, biases and clamped SwiGLU ~188 578 / 599, 344 851 / 873, 406
-// 1016 / 966, 512 1181 / 1118, ~512 1226 / 1173; 32 experts, plain ~250 192 / 199, ~500 310 / 306, ~750 447 / 415, ~2048 1100 /
-// 1017; 1792 x 1024, 64 experts, plain ~219 118 / 118, ~500 215 / 190, ~1024 375 / 328.
+// deviations of an expert's rows under uniform routing, in whole rows as in moe_fp8blk_item_rows). Layer, us, streaming / tall
+// kernel, at the mean number of rows, `~` with experts asked for unevenly: 2880 x 2880, 128 experts, biases and clamped SwiGLU
+// ~188 578 / 599, 344 851 / 873, 406 1016 / 966, 512 1181 / 1118, ~512 1226 / 1173; 32 experts, plain ~250 192 / 199, ~500
+// 310 / 306, ~750 447 / 415, ~2048 1100 / 1017; 1792 x 1024, 64 experts, plain ~219 118 / 118, ~500 215 / 190, ~1024 375 / 328.
 constexpr int kTallMinMean = 400;
 static bool moe_tall(int T, int H, int I, int E, int k, int weight_layout, bool a8) {
     if (weight_layout != 1 || a8 || H <= 512 || I <= 512) return false;   // (the kernel needs three K-steps)
